@@ -71,6 +71,62 @@ SGNX_HD inline double div_const(double a, const ConstDiv& d) {
   return div_fast(a, d);
 }
 
+// The same quotient without a branch of its own, for sums that never round to
+// -0 in the reference (they start from +0.0): fma(r, rh, q1) is +0 for a = +0
+// and for a = -0, so the sum may drop its leading 0.0 +. Right wherever
+// div_needs_exact(a) is false and the result is finite: a finite result rules
+// out a dividend or quotient that overflowed (an infinite or NaN dividend and
+// an overflowing product both give a non-finite one).
+SGNX_HD inline double div_unchecked(double a, const ConstDiv& d) {
+  const double t = a * d.rl;
+  const double q1 = fma(a, d.rh, t);
+  const double r = fma(-q1, d.b, a);
+  return fma(r, d.rh, q1);
+}
+
+// Several quotients by one divisor known only at run time: its reciprocal y,
+// refined from an approximation y0 of relative error below 2^-20 by two Newton
+// steps (then within 0.5 + 2^-30 ulp) and one more whose residual 1 - b*y is
+// exact, which leaves RN(1/b) for every b but one whose significand is all ones
+// (its reciprocal is too near a half-way case; div_by_ok excludes it), and yl
+// with y + yl = 1/b to about 2^-104. A quotient is then the four-operation
+// sequence above, with the sign of a zero kept. Range: div_by_ok(b), and the
+// dividends that div_fast takes.
+struct DivBy {
+  double b, y, yl;
+  SGNX_HD double quotient(double a) const {
+    const double t = a * yl;
+    const double q1 = fma(a, y, t);
+    const double r = fma(-q1, b, a);
+    return -fma(-r, y, -q1);
+  }
+};
+
+SGNX_HD inline DivBy make_div_by(double b, double y0) {
+  double y = fma(fma(-b, y0, 1.0), y0, y0);
+  y = fma(fma(-b, y, 1.0), y, y);
+  y = fma(fma(-b, y, 1.0), y, y);
+  return DivBy{b, y, fma(-b, y, 1.0) * y};
+}
+
+// 2^-100 <= b < 2^100, by the high word (a negative or NaN b is outside), and
+// the significand's low word not all ones
+SGNX_HD inline bool div_by_ok(double b) {
+  unsigned long long u;
+  __builtin_memcpy(&u, &b, sizeof u);
+  constexpr unsigned lo = (1023u - 100u) << 20, hi = (1023u + 100u) << 20;
+  return ((unsigned)(u >> 32) - lo < hi - lo) & ((unsigned)u != 0xffffffffu);
+}
+
+// whether |a| is below 2^-900 but not zero: doubling the bits drops the sign,
+// and subtracting one takes a zero to the top of the range
+SGNX_HD inline bool div_needs_exact(double a) {
+  unsigned long long u;
+  __builtin_memcpy(&u, &a, sizeof u);
+  constexpr unsigned long long kLow = (unsigned long long)(1023 - 900) << 53;   // bits of 2^-900, doubled
+  return (u << 1) - 1 < kLow - 1;
+}
+
 }  // namespace sgnx
 
 #endif  // SGNX_FASTDIV_H

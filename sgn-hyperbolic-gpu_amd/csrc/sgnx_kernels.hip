@@ -312,9 +312,10 @@ k_rhs(const double* __restrict__ U, double* __restrict__ dU, Geometry g, Phys ph
 //
 // A workgroup owns a strip of TW element columns and a chunk of `rows`
 // element rows and walks up the chunk one element row r per iteration:
-//   A  the row's nodes (loaded during the previous iteration; the loads of
-//      row r+1 are issued here): stage input, primitives, nodal F and G,
-//      source -> LDS / registers
+//   A  the row's nodes: stage input, primitives, nodal F and G, source -> LDS
+//      / registers. Node operands are loaded two rows ahead: row r + 1 has
+//      landed, and its bottom faces go to LDS too (with the halo nodes of the
+//      strip's outer x lines); row r + 2's loads are issued here.
 //   B  interface items: the TW+1 x-interface lines of row r, and the
 //      y-interface line r+1 on top of the row (the line at its bottom was
 //      done in the previous iteration, or before the loop). A y-interface is
@@ -325,12 +326,19 @@ k_rhs(const double* __restrict__ U, double* __restrict__ dU, Geometry g, Phys ph
 //      F* - F(left/lower state) and F* - F(right/upper state) and the depth
 //      jumps h* - h, which are the jumps the reference forms for each of the
 //      two elements (sgn2d.cpp:251-257, :268-275); y lines are double-buffered.
-//      The operands an interface item takes from global memory (face depth,
-//      halo node, the bottom face of row r+1) are also loaded one row ahead.
 //   C  nodes: the complete RHS of row r (and, in the candidate stage, its
 //      scaled embedded error).
 // Every y-interface is evaluated once; the stage input is read once per chunk,
-// plus the top faces of the row below the chunk and the x-halo nodes.
+// plus the faces of the rows below and above the chunk and the x-halo nodes.
+//
+// What bounds it: the stage launches, their traffic (stage 3 moves 3.1 to 3.2
+// GB at 1024x512, 4.9 TB/s, the rate of a large copy); the plain launch, the
+// instructions and latencies of the row (about 500 vector and 80 LDS
+// instructions per wave and row, three waves per SIMD). Hence no branch around
+// a global access, no face loaded twice, quotients without a branch each, and
+// no vector instruction spent on an address. On 1024x512, per launch, before
+// and after these (one MI355X, both builds in turn): plain 0.409 -> 0.348 ms,
+// stage 2 0.549 -> 0.436, stage 3 0.725 -> 0.640, k4 0.628 -> 0.505.
 template <int TW>
 struct Sweep {
   static constexpr int NT = ((NPP * TW + 63) / 64) * 64;
@@ -353,44 +361,58 @@ struct NodeExtra {
   double x0[(MODE == kCand || MODE == kErr) ? NV : 1], x1[MODE == kErr ? NV : 1];
 };
 
-// A five-variable operand by one base pointer: variable v of node n is
-// base[n + v Nd] with a 32-bit index (the grid has at most 2^28 nodes per
-// variable, so 5 Nd < 2^32). One base per operand instead of five plane
-// pointers keeps the launch's uniform values within the scalar registers.
-struct VarPtrs {
-  const double* base;
-  unsigned nd;
-  __device__ __forceinline__ double at(int v, unsigned node) const {
-    return base[node + (unsigned)v * nd];
-  }
-};
-__device__ __forceinline__ VarPtrs var_ptrs(const double* base, long long Nd) {
-  VarPtrs r;
-  r.base = base;
-  r.nd = (unsigned)Nd;
-  return r;
+// Global operands are addressed as a wave-uniform base (scalar registers and
+// scalar adds) plus a 32-bit byte offset of the lane, so that no vector
+// instruction forms an address. Variable v of an operand lies v planes of
+// `plane` bytes above its base; the planes are stepped to one after another,
+// which needs one scalar pair per operand instead of five.
+typedef __attribute__((address_space(1))) char GlobalByte;
+typedef __attribute__((address_space(1))) double GlobalDouble;
+typedef __attribute__((address_space(3))) double LdsDouble;
+__device__ __forceinline__ GlobalByte* global_at(const double* base, size_t first) {
+  GlobalByte* p = (GlobalByte*)base + first;
+  __asm__ volatile("" : "+s"(p));   // formed by scalar instructions, before the lane's part
+  return p;
 }
-
-struct StagePtrs {
-  VarPtrs u, k, x0, x1;
-};
-
-template <int MODE>
-__device__ __forceinline__ void stage_load(const StagePtrs& P, unsigned node, StageRaw<MODE>& R) {
+__device__ __forceinline__ double load_at(const GlobalByte* base, unsigned off) {
+  return *(const GlobalDouble*)(base + off);
+}
+__device__ __forceinline__ void store_at(GlobalByte* base, unsigned off, double x) {
+  *(GlobalDouble*)(base + off) = x;
+}
+__device__ __forceinline__ void load_vars(const double* base, size_t first, size_t plane,
+                                          unsigned off, double* W) {
+  const GlobalByte* p = global_at(base, first);
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    R.u[v] = P.u.at(v, node);
-    if (StageRaw<MODE>::kHasK) R.k[v] = P.k.at(v, node);
+    W[v] = load_at(p, off);
+    p += plane;
   }
 }
 
+// The launch's arguments in constant memory (kernel arguments, or one entry
+// of a batch's table), read by scalar loads. What a phase needs once per row
+// is read there again, through a pointer made opaque in that row: all of it
+// kept across rows exceeds the scalar registers, and the excess would travel
+// through vector lanes.
+typedef const BatchMember __attribute__((address_space(4))) * SweepArgs;
+__device__ __forceinline__ SweepArgs opaque(SweepArgs A) {
+  __asm__ volatile("" : "+s"(A));
+  return A;
+}
+
 template <int MODE>
-__device__ __forceinline__ void extra_load(const StagePtrs& P, unsigned node, NodeExtra<MODE>& E) {
-#pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    if (MODE == kCand || MODE == kErr) E.x0[v] = P.x0.at(v, node);
-    if (MODE == kErr) E.x1[v] = P.x1.at(v, node);
-  }
+__device__ __forceinline__ void stage_load(SweepArgs A, size_t first, size_t plane, unsigned off,
+                                           StageRaw<MODE>& R) {
+  load_vars(A->sa.u, first, plane, off, R.u);
+  if (StageRaw<MODE>::kHasK) load_vars(A->sa.k1, first, plane, off, R.k);
+}
+
+template <int MODE>
+__device__ __forceinline__ void extra_load(SweepArgs A, size_t first, size_t plane, unsigned off,
+                                           NodeExtra<MODE>& E) {
+  if (MODE == kCand || MODE == kErr) load_vars(MODE == kCand ? A->sa.kc : A->sa.u0, first, plane, off, E.x0);
+  if (MODE == kErr) load_vars(A->sa.z, first, plane, off, E.x1);
 }
 
 // rk.cpp:100, :102: the stage input u + (c dt) k from its operands (a = c dt)
@@ -403,153 +425,216 @@ __device__ __forceinline__ void stage_combine(const StageRaw<MODE>& R, double a,
   }
 }
 
+// a face's state: the stage input + 0.0
 template <int MODE>
-__device__ __forceinline__ void stage_face(const StagePtrs& P, double a, unsigned node,
-                                           double* W) {
-  StageRaw<MODE> R;
-  stage_load<MODE>(P, node, R);
+__device__ __forceinline__ void stage_combine_face(const StageRaw<MODE>& R, double a, double* W) {
   stage_combine<MODE>(R, a, W);
 #pragma unroll
   for (int v = 0; v < NV; ++v) W[v] = W[v] + 0.0;
 }
 
-// S[v] for a v that may not be a compile-time constant (selects, no
-// indexed register access)
-__device__ __forceinline__ double pick(const double* S, int v) {
-  return (v == IH) ? S[IH] : (v == IHU) ? S[IHU] : (v == IHV) ? S[IHV] : (v == IHW) ? S[IHW] : S[IHP];
-}
-
-// Lane permutes within each group of four lanes (DPP quad_perm): the value
-// of the even lane of the pair, of the odd lane, and of the other lane.
-template <int CTRL>
-__device__ __forceinline__ double lane_perm(double x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xF, 0xF, false);
+// The other lane's value within each pair of lanes (DPP quad_perm [1,0,3,2]).
+__device__ __forceinline__ double lane_swap(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0xB1, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0xB1, 0xF, 0xF, true);
   return __hiloint2double(hi, lo);
 }
-__device__ __forceinline__ double lane_even(double x) { return lane_perm<0xA0>(x); }  // [0,0,2,2]
-__device__ __forceinline__ double lane_odd(double x) { return lane_perm<0xF5>(x); }   // [1,1,3,3]
-__device__ __forceinline__ double lane_swap(double x) { return lane_perm<0xB1>(x); }  // [1,0,3,2]
+
+// barrier that instructions of the two phases do not cross in either direction
+// (arithmetic hoisted over it only lengthens registers' lives)
+__device__ __forceinline__ void row_sync() {
+  __builtin_amdgcn_sched_barrier(0);
+  __syncthreads();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// whether the condition holds on some active lane of the wave
+__device__ __forceinline__ bool wave_any(int c) { return __builtin_amdgcn_ballot_w64(c != 0) != 0; }
+
+// The primitives of prims() by one refined reciprocal of h for the four
+// quotients where h and the four dividends are in the range of DivBy; else, on
+// some lane of the wave, by IEEE division for the wave. Same bits.
+__device__ __forceinline__ Prim prims_shared(const double* U) {
+  const DivBy d = make_div_by(U[IH], __builtin_amdgcn_rcp(U[IH]));
+  Prim q;
+  q.u = d.quotient(U[IHU]);
+  q.v = d.quotient(U[IHV]);
+  q.w = d.quotient(U[IHW]);
+  q.p = d.quotient(U[IHP]);
+  const double big = fmax(fmax(fabs(U[IHU]), fabs(U[IHV])), fmax(fabs(U[IHW]), fabs(U[IHP])));
+  const int bad = (int)!div_by_ok(U[IH]) | (int)!(big <= 0x1p+800) |
+                  (int)div_needs_exact(U[IHU]) | (int)div_needs_exact(U[IHV]) |
+                  (int)div_needs_exact(U[IHW]) | (int)div_needs_exact(U[IHP]);
+  if (__builtin_expect(wave_any(bad), 0)) q = prims(U);
+  return q;
+}
+
+// y = x as a move at this place
+__device__ __forceinline__ void move_to(double& y, double x) {
+  __asm__ volatile("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
+}
+
+// x with its sign bit changed where mask = 0x80000000 (0: unchanged)
+__device__ __forceinline__ double flip_sign(double x, int mask) {
+  return __hiloint2double(__double2hiint(x) ^ mask, __double2loint(x));
+}
 
 __device__ __forceinline__ unsigned node_of(int Nx, int ex, int ey, int a, int b) {
   return ((unsigned)ey * (unsigned)Nx + (unsigned)ex) * NPP + a + NP * b;
 }
 
+template <int V>
+struct IntC { static constexpr int value = V; };
+
+// LDS of one workgroup. A node's record holds h, hu, hv, hw, hp, the fluxes
+// F[1..4] and G[1..4] (F[0] is hu and G[0] is hv) and, with HXR, the still
+// depth; every operand of phase C is then an immediate offset from the lane's
+// row, its column or its own record. 13 and 15 doubles are odd multiples of a
+// bank pair, so neither the records' writes nor the row and column reads
+// conflict. Interface jumps: F* - F(side) and, as a sixth entry, h* - h(side)
+// (side 0 = left / lower, 1 = right / upper), for the x lines of the row and
+// the y lines below and above it (by line parity).
+template <int TW, bool HXR>
+struct SweepLds {
+  static constexpr int kRec = HXR ? 15 : 13;
+  static constexpr int kF = 4, kG = 8, kH = 13;      // record offsets: F[v] at kF + v, v >= 1
+  static constexpr int kJ = NP * (TW + 1);           // interface nodes of one jump plane
+  static constexpr int kJSide = (NV + 1) * kJ, kJLine = 2 * kJSide;
+  double node[NPP * TW * kRec];
+  double jump[3 * kJLine];                           // x lines, even y line, odd y line
+  double face[(NP * TW + 2 * NP) * NV];              // bottom faces of the row above, halo nodes
+  double tab[NP][NP + 2];                            // per node index a: D[a][.], gL'[a], gR'[a]
+  static __device__ __forceinline__ constexpr int offF(int v) { return v == IH ? IHU : kF + v; }
+  static __device__ __forceinline__ constexpr int offG(int v) { return v == IH ? IHV : kG + v; }
+};
+
 // One workgroup's strip x chunk `tile` of one grid (the body of the plain and
 // the batched launches).
 template <int TW, int MODE, int WAVES, bool KEEP = false, bool HXR = false>
-__device__ __forceinline__ void sweep_tile(const double* __restrict__ U, double* __restrict__ dU,
-                                           const Geometry& g, const Phys& phIn, const GhostTime& gt,
-                                           const Stage& sa, int nStrips, int tile) {
-  constexpr int NT = Sweep<TW>::NT, NXI = Sweep<TW>::NXI, NYI = Sweep<TW>::NYI;
+__device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
+  using L = SweepLds<TW, HXR>;
+  constexpr int kRec = L::kRec, kJ = L::kJ, kJSide = L::kJSide, kJLine = L::kJLine;
   // the row sweep runs without the Manning friction term (the launchers
   // refuse it; solvers with friction use the element-row tiles), so its
   // branch is compiled out
-  Phys ph = phIn;
-  ph.nManning = 0.0;
-  __shared__ double sU[NV][NT];
-  __shared__ double sF[NV][NT];
-  __shared__ double sG[NV][NT];
-  // interface jumps by side s (0 = left / lower, 1 = right / upper):
-  // F* - F(side s) and h* - h(side s); y lines double-buffered
-  __shared__ double xJ[2][NV][NXI], xhJ[2][NXI];
-  __shared__ double yJ[2][2][NV][NYI], yhJ[2][2][NYI];
-  __shared__ double sD[NPP], sgL[NP], sgR[NP];
-  // HXR: the still depth at the row's nodes, from which phase C forms Hx, Hy
-  // (sgn2d.cpp:54-71) instead of reading them
-  __shared__ double sH[HXR ? NT : 1];
+  Phys ph{A->ph.g, A->ph.c, A->ph.gamma, 0.0, A->ph.halfg, A->ph.c2, A->ph.mc2, A->ph.m2c2};
+  const ConstDiv divX{A->g.dx.b, A->g.dx.rh, A->g.dx.rl, 1}, divY{A->g.dy.b, A->g.dy.rh, A->g.dy.rl, 1};
+  const double stA = A->sa.a, stDt = A->sa.dt, atol = A->sa.atol, rtol = A->sa.rtol;
+  const int bcL = A->g.bc[0], bcR = A->g.bc[1], bcB = A->g.bc[2], bcT = A->g.bc[3];
+  const int nStrips = A->nStrips, rows = A->g.rows, Nx = A->g.Nx, Ny = A->g.Ny;
+  __shared__ L lds;
 
-  if (threadIdx.x < NPP) sD[threadIdx.x] = g.ops->D[threadIdx.x];
   if (threadIdx.x < NP) {
-    sgL[threadIdx.x] = g.ops->gLp[threadIdx.x];
-    sgR[threadIdx.x] = g.ops->gRp[threadIdx.x];
+    const OpTables* const T = A->g.ops;
+    double* const to = lds.tab[threadIdx.x];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) to[k] = T->D[threadIdx.x * NP + k];
+    to[NP] = T->gLp[threadIdx.x];
+    to[NP + 1] = T->gRp[threadIdx.x];
   }
 
-  const int chunk = tile / nStrips;
+  const int chunk = __builtin_amdgcn_readfirstlane(tile / nStrips);
   const int ex0 = (tile - chunk * nStrips) * TW;
-  const int nW = min(TW, g.Nx - ex0);
-  const int ey0 = chunk * g.rows;
-  const int ey1 = min(g.Ny, ey0 + g.rows);
+  const int nW = min(TW, Nx - ex0);
+  const int ey0 = chunk * rows;
+  const int ey1 = min(Ny, ey0 + rows);
   const int nNodes = NPP * nW;
   const int t = threadIdx.x;
-  const long long Nd = g.Nd;
-  const int Nx = g.Nx, Ny = g.Ny;
-  StagePtrs P;
-  P.u = var_ptrs(MODE == kPlain ? U : sa.u, Nd);
-  P.k = var_ptrs(sa.k1, Nd);
-  P.x0 = var_ptrs(MODE == kCand ? sa.kc : sa.u0, Nd);
-  P.x1 = var_ptrs(sa.z, Nd);
+  const size_t plane0 = (size_t)A->g.Nd * sizeof(double);
+  const unsigned rowBytes = (unsigned)Nx * (NPP * 8u);   // a plane has at most 2^31 bytes
 
+  // Every lane has an item in every phase, so that no branch stands around a
+  // global access: the compiler then knows how many accesses are in flight at
+  // each wait and waits for the oldest only. Lanes beyond the strip's items
+  // repeat item 0, with the same values at the same addresses.
+  //
   // node work item: node (a, b) of element j of the strip
-  const int j = t / NPP, loc = t - NPP * j;
-  const int b = loc / NP, a = loc - NP * b;
   const bool isNode = t < nNodes;
+  const int tn = isNode ? t : 0;
+  const int j = tn / NPP, loc = tn - NPP * j;
+  const int b = loc / NP, a = loc - NP * b;
+  unsigned t8 = (unsigned)tn * 8u;                       // the node
+  unsigned f8 = (unsigned)(j * NPP + a) * 8u;            // the bottom face of its column
   // Interface half-items: two lanes per interface node, lane 2k + side
   // taking one side (0 = left / lower, 1 = right / upper) of interface k.
-  // Items 0 .. 2 nX - 1 are the x-interface nodes of the row (k = i NP + bb:
-  // line i on the left edge of strip column i, node bb); the next 2 NP nW items
+  // Items 0 .. nX - 1 are the x-interface nodes of the row (k = i NP + bb:
+  // line i on the left edge of strip column i, node bb); the next NP nW items
   // the y-interface nodes of the line above the row (k = nX + jj NP + aa).
   // Each lane evaluates its own side (primitives, one-sided flux, wave speed)
   // and the pair exchanges them with lane permutes, so the interface work is
   // spread over every wave of the workgroup.
   const int nX = NP * (nW + 1);
-  const int side = t & 1, kk = t >> 1;
-  const bool isX = t < 2 * nX;
-  const bool isY = !isX && t < 2 * nX + 2 * NP * nW;
+  const int side = t & 1, kk = (t >> 1) < nX + NP * nW ? t >> 1 : 0;
+  const bool isX = kk < nX, isY = !isX;
   const int xi = isX ? kk / NP : 0, xb = isX ? kk - NP * xi : 0;
   const int ky = isY ? kk - nX : 0;
   const int jj = ky / NP, aa = ky - NP * jj;
-
-  // The global node this lane's side takes for row r, if any: the halo node
-  // of the strip's outer x-lines, or the bottom face of row r+1 for the upper
-  // side of a y item (false at a wall, where a ghost replaces it, and for
-  // every side that lies in the workgroup's row).
-  auto face_node = [&](int r, unsigned& n) -> bool {
-    if (isX) {
-      if (side == 0 && xi == 0) {
-        if (ex0 > 0) { n = node_of(Nx, ex0 - 1, r, NP - 1, xb); return true; }
-        if (g.bc[0] == 0) { n = node_of(Nx, Nx - 1, r, NP - 1, xb); return true; }
-        return false;
-      }
-      if (side == 1 && xi == nW) {
-        const int ex = ex0 + nW;
-        if (ex < Nx) { n = node_of(Nx, ex, r, 0, xb); return true; }
-        if (g.bc[1] == 0) { n = node_of(Nx, 0, r, 0, xb); return true; }
-        return false;
-      }
-      return false;
-    }
-    if (side == 0) return false;
-    const int y = r + 1;
-    if (y < Ny) { n = node_of(Nx, ex0 + jj, y, aa, 0); return true; }
-    if (g.bc[3] == 0) { n = node_of(Nx, ex0 + jj, 0, aa, 0); return true; }
-    return false;
-  };
+  // The side's state: a node of the row in LDS, the bottom face of the row
+  // above for the upper side of a y line (gY, in LDS too), or the halo node of
+  // the strip's outer x lines (gX, a global node). At a wall it is the other
+  // side's node, mirrored. The inflow side's ghost is data.
+  const bool outer = isX && (side == 0 ? xi == 0 : xi == nW);
+  const bool gX = outer && (side == 0 ? ex0 > 0 || bcL == 0 : ex0 + nW < Nx || bcR == 0);
+  const bool gY = isY && side == 1;
+  const bool inflow = outer && side == 0 && ex0 == 0 && bcL == 2;
+  const bool wallTop = bcT != 0;
+  int src;
+  if (isX) {
+    const int col = outer ? (side == 0 ? 0 : nW - 1) : (side == 0 ? xi - 1 : xi);
+    const bool high = outer ? side == 1 : side == 0;
+    src = col * NPP + (high ? NP - 1 : 0) + NP * xb;
+  } else {
+    src = jj * NPP + aa + NP * (NP - 1);
+  }
+  int mirror = outer && !gX ? (int)0x80000000 : 0;
+  LdsDouble* sSrc = (LdsDouble*)lds.node + src * kRec;
+  LdsDouble* sHalo = (LdsDouble*)lds.face + (NP * TW + NP * side + xb) * NV;
+  LdsDouble* sFrom = gX ? sHalo : gY ? (LdsDouble*)lds.face + ky * NV : sSrc;
+  // the global node of the gX lanes (byte offset), for the row whose
+  // interfaces are next (the others: the strip's first node); it moves up one
+  // element row with r
+  unsigned fOff = node_of(Nx, ex0, ey0, 0, 0) * 8u;
+  if (gX) {
+    const int col = side == 0 ? (ex0 > 0 ? ex0 - 1 : Nx - 1) : (ex0 + nW < Nx ? ex0 + nW : 0);
+    fOff = node_of(Nx, col, ey0, side == 0 ? NP - 1 : 0, xb) * 8u;
+  }
+  // face depth of the lane's line of row r, and its step to the next row
+  const GlobalDouble* pHf =
+      isX ? (const GlobalDouble*)A->g.HfX + ((size_t)ey0 * (Nx + 1) + ex0 + xi) * NP + xb
+          : (const GlobalDouble*)A->g.HfY + ((size_t)(ey0 + 1) * Nx + ex0 + jj) * NP + aa;
+  const unsigned hfStep = (unsigned)(Nx + (isX ? 1 : 0)) * NP;
+  LdsDouble* sJ = (LdsDouble*)lds.jump + (isX ? 0 : kJLine) + side * kJSide + (isX ? kk : ky);
 
   // One interface node evaluated by a lane pair. W is this lane's side's
   // state in the interface frame (a y interface has hu and hv exchanged:
   // fluxY(U) is fluxX of the exchanged state with hu and hv of the result
-  // exchanged back, and |v| is the exchanged |u|). Returns this side's flux
-  // jump F* - F(W) (frame order) and depth jump h* - h(W), with the Rusanov
-  // flux of sgn_flux2d.h:169-179: F* = 0.5 (FL + FR) - 0.5 max(sL, sR) (UR - UL).
-  auto half_iface = [&](const double* W, double Hf, double* jf, double& jh) {
-    const Prim q = prims(W);
+  // exchanged back, and |v| is the exchanged |u|). Stores this side's flux
+  // jump F* - F(W) and depth jump h* - h(W), with the Rusanov flux of
+  // sgn_flux2d.h:169-179: F* = 0.5 (FL + FR) - 0.5 max(sL, sR) (UR - UL).
+  // Both lanes take the other's values by one swap: UR - UL is other - own on
+  // the lower side and its negative on the upper one, which the sign of hl
+  // carries (where the difference is zero, F* - F is the same +0 either way).
+  auto half_iface = [&](const double* W, double Hf, LdsDouble* to) {
+    const Prim q = prims_shared(W);
     double F[NV];
     flux_x(W, q, Hf, ph, F);
     const double so = fabs(q.u) + signal_speed(W[IH], q, ph);
-    const double lam = fmax(lane_even(so), lane_odd(so));
-    const double hl = 0.5 * lam;
-    double hL = 0.0, hR = 0.0;
+    const double lam = fmax(so, lane_swap(so));
+    const double hl = flip_sign(0.5 * lam, side << 31);
+    double jf[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const double ul = lane_even(W[v]), ur = lane_odd(W[v]);
+      const double o = lane_swap(W[v]);
       // FL + FR in either lane order (addition commutes exactly)
-      const double Fs = 0.5 * (F[v] + lane_swap(F[v])) - hl * (ur - ul);
+      const double Fs = 0.5 * (F[v] + lane_swap(F[v])) - hl * (o - W[v]);
       jf[v] = Fs - F[v];
-      if (v == IH) { hL = ul; hR = ur; }
+      if (v == IH) to[NV * kJ] = 0.5 * (W[IH] + o) - W[IH];
     }
-    const double hs = 0.5 * (hL + hR);
-    jh = hs - W[IH];
+    to[IH * kJ] = jf[IH];
+    to[IHU * kJ] = isY ? jf[IHV] : jf[IHU];
+    to[IHV * kJ] = isY ? jf[IHU] : jf[IHV];
+    to[IHW * kJ] = jf[IHW];
+    to[IHP * kJ] = jf[IHP];
   };
   auto to_frame = [&](double* W) {             // exchange hu, hv on y lanes
     const double u_ = W[IHU], v_ = W[IHV];
@@ -557,337 +642,330 @@ __device__ __forceinline__ void sweep_tile(const double* __restrict__ U, double*
     W[IHV] = isY ? u_ : v_;
   };
 
-  // prologue: the y line at the bottom of the chunk, both sides from global
-  // memory (the bottom wall's ghost mirrors the upper side)
-  if (isY) {
-    double W[NV];
-    const int y = ey0;
-    const unsigned nUp = node_of(Nx, ex0 + jj, y, aa, 0);
-    if (side == 1) {
-      stage_face<MODE>(P, sa.a, nUp, W);
-    } else if (y > 0) {
-      stage_face<MODE>(P, sa.a, node_of(Nx, ex0 + jj, y - 1, aa, NP - 1), W);
-    } else if (g.bc[2] == 0) {
-      stage_face<MODE>(P, sa.a, node_of(Nx, ex0 + jj, Ny - 1, aa, NP - 1), W);
-    } else {
-      double Wu[NV];
-      stage_face<MODE>(P, sa.a, nUp, Wu);
-      wall_ghost(Wu, IHV, W);
-    }
-    to_frame(W);
-    const double Hf = g.HfY[((long long)y * Nx + ex0 + jj) * NP + aa];
-    double jf[NV], jh;
-    half_iface(W, Hf, jf, jh);
-    to_frame(jf);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) yJ[y & 1][side][v][ky] = jf[v];
-    yhJ[y & 1][side][ky] = jh;
-  }
-
-  auto face_node_now = [&](int r) -> bool {
-    unsigned n;
-    return face_node(r, n);
-  };
-  // The interface lanes' global operands of row r + 1: the halo nodes and
-  // the bottom face of row r + 2. The two-wave stage launches issue them
-  // after their phase A of row r. The plain launch and the three-wave stage-2
-  // launch issue them at the start of phase C, which leaves phase C and the
-  // next phase A to cover their latency, brings the full loads of row r + 2
-  // (issued after that phase A) close enough behind that fewer bottom-face
-  // lines have left L2, and shortens their register lifetime: the plain
-  // launch measured 4 % faster, and the stage-2 build fits three waves per
-  // SIMD (with Hx, Hy read) with 3 registers spilled instead of 15. The
-  // two-wave stage launches were not faster this way.
-  constexpr bool kLateFace = MODE == kPlain || (MODE == kAxpy && WAVES == 3);
+  // The interface lanes' global operands: the halo nodes and the face depths.
+  // Those of row r + 1 are issued at the start of phase C of row r, so phase C
+  // and the next phase A cover their latency.
   StageRaw<MODE> fR;
-  double fH = 0.0;
-  auto face_prefetch = [&](int r) {
-    if (isX || isY) {
-      unsigned n;
-      if (face_node(r, n)) stage_load<MODE>(P, n, fR);
-      fH = isX ? g.HfX[((long long)r * (Nx + 1) + ex0 + xi) * NP + xb]
-               : g.HfY[((long long)(r + 1) * Nx + ex0 + jj) * NP + aa];
+  double fH;
+  auto face_load = [&](SweepArgs R, size_t plane) {
+    stage_load<MODE>(R, 0, plane, fOff, fR);
+    fH = *pHf;
+  };
+
+  // The nodes' operands, two rows ahead: while row r is worked on, row r + 1
+  // has landed (its bottom faces are the upper side of the y line between the
+  // two, so no lane loads a face a second time) and row r + 2 is in flight.
+  // Above the chunk only the bottom faces are needed (from the first row
+  // across a periodic top side), so every lane takes its column's; with
+  // nothing to load, row r's first nodes stand in.
+  struct Node {
+    StageRaw<MODE> s;
+    double H, Hx, Hy;
+    __device__ __forceinline__ void take(const Node& o) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        move_to(s.u[v], o.s.u[v]);
+        if (StageRaw<MODE>::kHasK) move_to(s.k[v], o.s.k[v]);
+      }
+      move_to(H, o.H);
+      if (!HXR) {
+        move_to(Hx, o.Hx);
+        move_to(Hy, o.Hy);
+      }
     }
   };
-  face_prefetch(ey0);
-
-  // loads of row ey0's node data
-  StageRaw<MODE> pR;
-  NodeExtra<MODE> pE;
-  double pH = 0.0, pHx = 0.0, pHy = 0.0;
-  if (isNode) {
-    const unsigned gn = node_of(Nx, ex0, ey0, 0, 0) + t;
-    stage_load<MODE>(P, gn, pR);
-    extra_load<MODE>(P, gn, pE);
-    pH = g.Hnod[gn];
-    if (!HXR) { pHx = g.Hx[gn]; pHy = g.Hy[gn]; }
+  Node cur, nxt;
+  const unsigned row0 = (unsigned)ex0 * (NPP * 8u);
+  unsigned rowOff = row0 + (unsigned)ey0 * rowBytes;     // row r's first node (bytes)
+  auto node_load = [&](SweepArgs R, int r, int ahead, size_t plane, Node& n) {
+    int to = r + ahead;
+    const bool full = to < ey1;
+    to = to > ey1 ? r : to;
+    to = to == Ny ? (wallTop ? r : 0) : to;
+    const unsigned first =
+        __builtin_amdgcn_readfirstlane((int)(row0 + (unsigned)to * rowBytes));
+    const unsigned off = full ? t8 : f8;
+    stage_load<MODE>(R, first, plane, off, n.s);
+    n.H = load_at(global_at(R->g.Hnod, first), off);
+    if (!HXR) {
+      n.Hx = load_at(global_at(R->g.Hx, first), off);
+      n.Hy = load_at(global_at(R->g.Hy, first), off);
+    }
+  };
+  node_load(A, ey0, 0, plane0, cur);
+  node_load(A, ey0, 1, plane0, nxt);
+  face_load(A, plane0);
+  // the y line at the bottom of the chunk, both sides from global memory (the
+  // bottom wall's ghost mirrors the upper side)
+  if (isY) {
+    const bool below = ey0 > 0 || bcB == 0;
+    const bool lower = side == 0 && below;
+    const unsigned n = lower ? node_of(Nx, ex0 + jj, ey0 > 0 ? ey0 - 1 : Ny - 1, aa, NP - 1)
+                             : node_of(Nx, ex0 + jj, ey0, aa, 0);
+    StageRaw<MODE> R;
+    stage_load<MODE>(A, 0, plane0, n * 8u, R);
+    double W[NV];
+    stage_combine_face<MODE>(R, stA, W);
+    to_frame(W);
+    if (side == 0 && !below) W[IHU] = -W[IHU];
+    half_iface(W, ((const GlobalDouble*)A->g.HfY)[((size_t)ey0 * Nx + ex0 + jj) * NP + aa],
+               sJ + (ey0 & 1) * kJLine);
   }
+  // a Jacobian outside the branch-free quotient's range: always IEEE division
+  const bool never_fast = !A->g.dx.fast || !A->g.dy.fast;
   // scaled embedded error of this work-item's nodes (kErr)
   double eS = 0.0, eC = 0.0, eM = 0.0;
 
-  for (int r = ey0; r < ey1; ++r) {
-    const unsigned rowBase = node_of(Nx, ex0, r, 0, 0);
+  LdsDouble* sOwn = (LdsDouble*)lds.node + tn * kRec;
+  LdsDouble* sRow = (LdsDouble*)lds.node + (j * NPP + NP * b) * kRec;
+  LdsDouble* sCol = (LdsDouble*)lds.node + (j * NPP + a) * kRec;
+  LdsDouble* sBot = (LdsDouble*)lds.face + (j * NP + a) * NV;
+  LdsDouble* sJx = (LdsDouble*)lds.jump + j * NP + b;   // the line on the element's left
+  LdsDouble* sJy = (LdsDouble*)lds.jump + kJLine + j * NP + a;
+  LdsDouble* sTa = (LdsDouble*)lds.tab[a];
+  LdsDouble* sTb = (LdsDouble*)lds.tab[b];
+
+  auto row = [&](int r) {
+    // opaque in every row: the planes of all operands kept across rows would
+    // exceed the scalar registers, and a lane offset folded into them would
+    // make the addresses vectors
+    size_t plane = plane0;
+    __asm__ volatile("" : "+s"(plane));
+    __asm__ volatile("" : "+v"(t8));
+    __asm__ volatile("" : "+v"(f8));
+    // likewise the lane's places in LDS, whose offset forms the rows would
+    // otherwise share through registers of their own
+    for (LdsDouble** q : {&sOwn, &sRow, &sCol, &sBot, &sJx, &sJy, &sTa, &sTb, &sFrom, &sHalo, &sJ})
+      __asm__ volatile("" : "+v"(*q));
     // ---- A ---------------------------------------------------------------------
-    double S[NV], qu = 0.0, qv = 0.0, qw = 0.0;
-    SrcPart sp{0.0, 0.0, 0.0};
-    // per-node operands phase C needs beyond the RHS (rk.cpp:106-108, :119-120,
-    // sums evaluated left to right as there):
-    //   kCand: c0 = u, c1 = 2/9 kc + 1/3 k, c2 = 7/24 kc + 0.25 k
-    //   kErr:  c0 = u0, c2 = z
-    double c0[NV], c1[NV], c2[NV];
-    // the interface lane's global node state and face depth for this row
-    // (the plain launch takes them at the start of phase B instead)
-    double SG[NV];
-    double Hf = 0.0;
-    const bool haveG = (isX || isY) && face_node_now(r);
-    if (!kLateFace && (isX || isY)) {
-      Hf = fH;
-      if (haveG) {
-        stage_combine<MODE>(fR, sa.a, SG);
-#pragma unroll
-        for (int v = 0; v < NV; ++v) SG[v] = SG[v] + 0.0;
-      }
-    }
-    if (isNode) {
+    double S[NV], qu, qv, qw;
+    SrcPart sp;
+    // row r's operands that phase C needs again: the stage operands and those
+    // of the candidate and the error, which nothing needs before phase C
+    NodeExtra<MODE> ext;
+    extra_load<MODE>(opaque(A), rowOff, plane, t8, ext);
+    const StageRaw<MODE> own = cur.s;
+    {
       double Un[NV];
-      stage_combine<MODE>(pR, sa.a, Un);
-      if (KEEP && sa.yOut) {
+      stage_combine<MODE>(own, stA, Un);
+      double* const yOut = KEEP ? opaque(A)->sa.yOut : nullptr;
+      if (KEEP && yOut) {
         // the stage input, kept for a later reverse sweep
+        GlobalByte* p = global_at(yOut, rowOff);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) sa.yOut[rowBase + t + (unsigned)v * (unsigned)Nd] = Un[v];
-      }
-      const double Hn = pH, Hxn = pHx, Hyn = pHy;
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        if (MODE == kCand) {
-          c0[v] = pR.u[v];
-          c1[v] = 2.0 / 9.0 * pE.x0[v] + 1.0 / 3.0 * pR.k[v];
-          c2[v] = 7.0 / 24.0 * pE.x0[v] + 0.25 * pR.k[v];
-        } else if (MODE == kErr) {
-          c0[v] = pE.x0[v];
-          c2[v] = pE.x1[v];
+        for (int v = 0; v < NV; ++v) {
+          store_at(p, t8, Un[v]);
+          p += plane;
         }
       }
-      const Prim q = prims(Un);
+      const double Hn = cur.H;
+      const Prim q = prims_shared(Un);
       qu = q.u;
       qv = q.v;
       if (HXR) {
         // the gradient terms wait for phase C
         sp = source_part(Un, q, Hn, ph);
         qw = q.w;
-        sH[t] = Hn;
+        sOwn[L::kH] = Hn;
       } else {
-        source(Un, q, Hn, Hxn, Hyn, ph, S);
+        source(Un, q, Hn, cur.Hx, cur.Hy, ph, S);
       }
       double F[NV], G[NV];
       flux_x(Un, q, Hn, ph, F);
       flux_y(Un, q, Hn, ph, G);
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        sU[v][t] = Un[v];
-        sF[v][t] = F[v];
-        sG[v][t] = G[v];
+        sOwn[v] = Un[v];
+        if (v > IH) {
+          sOwn[L::offF(v)] = F[v];
+          sOwn[L::offG(v)] = G[v];
+        }
       }
     }
-    // row r+1's node operands, consumed one iteration later. Issued after
-    // the last use of this row's, and fenced against the scheduler hoisting
-    // them above those uses: the loads then land in the registers the loop
-    // carries, so no copy (and no wait for them) is needed at the back-edge.
     __builtin_amdgcn_sched_barrier(0);
-    if (!kLateFace && r + 1 < ey1) face_prefetch(r + 1);
-    if (isNode && r + 1 < ey1) {
-      const unsigned gn = rowBase + (unsigned)Nx * NPP + t;
-      stage_load<MODE>(P, gn, pR);
-      extra_load<MODE>(P, gn, pE);
-      pH = g.Hnod[gn];
-      if (!HXR) { pHx = g.Hx[gn]; pHy = g.Hy[gn]; }
+    if (b == 0) {
+      // the bottom faces of row r + 1
+      double W[NV];
+      stage_combine_face<MODE>(nxt.s, stA, W);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) sBot[v] = W[v];
     }
-    __syncthreads();
+    if (gX) {
+      double W[NV];
+      stage_combine_face<MODE>(fR, stA, W);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) sHalo[v] = W[v];
+    }
+    // Row r + 1's operands into row r's registers, row r + 2's loads into
+    // theirs. The moves are written out: left to itself the compiler moves at
+    // the end of the row, and there waits for the loads in flight.
+    __builtin_amdgcn_sched_barrier(0);
+    cur.take(nxt);
+    node_load(opaque(A), r, 2, plane, nxt);
+    row_sync();
 
     // ---- B ---------------------------------------------------------------------
-    if (isX || isY) {
+    {
+      if (wallTop && r + 1 == Ny && gY) {
+        sFrom = sSrc;                            // the top wall mirrors the row's own nodes
+        mirror = (int)0x80000000;
+      }
       double W[NV];
-      if (kLateFace) {
-        Hf = fH;
-        if (haveG) {
-          stage_combine<MODE>(fR, sa.a, W);
 #pragma unroll
-          for (int v = 0; v < NV; ++v) W[v] = W[v] + 0.0;
-        }
-      } else if (haveG) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) W[v] = SG[v];
-      }
-      if (isX) {
-        // own side: a node of this row, the halo node, or a ghost of the
-        // other side's node (a wall mirrors it; the inflow side is the table)
-        const int li = (side == 0) ? xi - 1 : xi;         // strip column of the node
-        const bool inRow = (side == 0) ? xi > 0 : xi < nW;
-        if (inRow) {
-          const int n = li * NPP + (side == 0 ? NP - 1 : 0) + NP * xb;
-#pragma unroll
-          for (int v = 0; v < NV; ++v) W[v] = sU[v][n] + 0.0;
-        } else if (!haveG) {
-          if (side == 0 && g.bc[0] == 2) {
-            const double* c = g.inflow + ((long long)r * NP + xb) * (NV * 3);
-#pragma unroll
-            for (int v = 0; v < NV; ++v)
-              W[v] = (c[3 * v] + c[3 * v + 1] * gt.s) + c[3 * v + 2] * gt.c;
-          } else {
-            const int n = (side == 0) ? NP * xb : (nW - 1) * NPP + (NP - 1) + NP * xb;
-            double Wo[NV];
-#pragma unroll
-            for (int v = 0; v < NV; ++v) Wo[v] = sU[v][n] + 0.0;
-            wall_ghost(Wo, IHU, W);
-          }
-        }
-      } else {
-        const int n = jj * NPP + aa + NP * (NP - 1);    // top face of row r
-        if (side == 0 || !haveG) {
-          double Wo[NV];
-#pragma unroll
-          for (int v = 0; v < NV; ++v) Wo[v] = sU[v][n] + 0.0;
-          if (side == 0) {
-#pragma unroll
-            for (int v = 0; v < NV; ++v) W[v] = Wo[v];
-          } else {
-            wall_ghost(Wo, IHV, W);                   // the top wall
-          }
-        }
-      }
+      for (int v = 0; v < NV; ++v) W[v] = sFrom[v] + 0.0;
       to_frame(W);
-      double jf[NV], jh;
-      half_iface(W, Hf, jf, jh);
-      to_frame(jf);
-      if (isX) {
+      W[IHU] = flip_sign(W[IHU], mirror);
+      if (inflow) {
+        const SweepArgs R = opaque(A);
+        const GlobalDouble* c = (const GlobalDouble*)R->g.inflow + ((size_t)r * NP + xb) * (NV * 3);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) xJ[side][v][xi * NP + xb] = jf[v];
-        xhJ[side][xi * NP + xb] = jh;
-      } else {
-        const int buf = (r + 1) & 1;
-#pragma unroll
-        for (int v = 0; v < NV; ++v) yJ[buf][side][v][ky] = jf[v];
-        yhJ[buf][side][ky] = jh;
+        for (int v = 0; v < NV; ++v)
+          W[v] = (c[3 * v] + c[3 * v + 1] * R->gt.s) + c[3 * v + 2] * R->gt.c;
       }
+      half_iface(W, fH, isX ? sJ : sJ + ((r + 1) & 1) * kJLine);
     }
-    __syncthreads();
+    row_sync();
 
     // ---- C: dU of row r ---------------------------------------------------------
-    if (kLateFace) {
-      if (r + 1 < ey1) face_prefetch(r + 1);
-      __builtin_amdgcn_sched_barrier(0);
+    if (r + 1 < ey1) {
+      fOff += rowBytes;
+      pHf += hfStep;
     }
-    if (isNode) {
+    face_load(opaque(A), plane);
+    __builtin_amdgcn_sched_barrier(0);
+    {
       double Da[NP], Db[NP];
 #pragma unroll
-      for (int k = 0; k < NP; ++k) { Da[k] = sD[a * NP + k]; Db[k] = sD[b * NP + k]; }
-      const double gLa = sgL[a], gRa = sgR[a], gLb = sgL[b], gRb = sgR[b];
-      const int ixL = j * NP + b, ixR = (j + 1) * NP + b, iy = j * NP + a;
-      const int bot = r & 1, top = (r + 1) & 1;
-      const int rowx = j * NPP + NP * b, coly = j * NPP + a;
-      double dhx = 0.0, dhy = 0.0, dHx = 0.0, dHy = 0.0;
-      // the three-wave stage-2 build keeps this loop rolled: unrolled, its
-      // hoisted LDS operands cost the 3 registers it otherwise spills (1 %
-      // faster without the spill; rolled, the other builds ran 3-8 % slower)
-      constexpr int kDepthUnroll = (WAVES == 3 && MODE == kAxpy) ? 1 : NP;
-#pragma unroll kDepthUnroll
-      for (int k = 0; k < NP; ++k) {
-        dhx = dhx + Da[k] * sU[IH][rowx + k];
-        dhy = dhy + Db[k] * sU[IH][coly + NP * k];
-        if (HXR) {
-          // sgn2d.cpp:54-71: (D H) / J along the node's x and y lines
-          dHx = dHx + Da[k] * sH[rowx + k];
-          dHy = dHy + Db[k] * sH[coly + NP * k];
-        }
-      }
-      if (HXR) source_rest(sp, qu, qv, qw, div_const(dHx, g.dx), div_const(dHy, g.dy), ph, S);
-      dhx = dhx + (xhJ[1][ixL] * gLa + xhJ[0][ixR] * gRa);
-      dhy = dhy + (yhJ[bot][1][iy] * gLb + yhJ[top][0][iy] * gRb);
-      const double hx = div_const(dhx, g.dx), hy = div_const(dhy, g.dy);
-      // the hp entries of the non-conservative products (the others are zero,
-      // and subtracting zero changes no sum)
-      const double Bx = ph.mc2 * qu * hx;
-      const double By = ph.mc2 * qv * hy;
-      const unsigned gn = rowBase + t;
-      auto variable = [&](int v) {
-        double dfx = 0.0, dgy = 0.0;
+      for (int k = 0; k < NP; ++k) { Da[k] = sTa[k]; Db[k] = sTb[k]; }
+      const double gLa = sTa[NP], gRa = sTa[NP + 1], gLb = sTb[NP], gRb = sTb[NP + 1];
+      LdsDouble* const jB = sJy + (r & 1) * kJLine;         // the line below the row
+      LdsDouble* const jT = sJy + ((r + 1) & 1) * kJLine;   // and the one above it
+      // The dividends of one pair of quotients, along x and along y: D . f of
+      // the records' entry `fx` / `fy` plus the lift of the jump plane v. The
+      // reference's sums start from 0.0; here they start from the first
+      // product, which differs only in a zero's sign, and div_unchecked takes
+      // both zeros to +0.
+      auto sums = [&](int fx, int fy, int v, double& ax, double& ay) {
+        double dx = Da[0] * sRow[fx], dy = Db[0] * sCol[fy];
 #pragma unroll
-        for (int k = 0; k < NP; ++k) {
-          dfx = dfx + Da[k] * sF[v][rowx + k];
-          dgy = dgy + Db[k] * sG[v][coly + NP * k];
+        for (int k = 1; k < NP; ++k) {
+          dx = dx + Da[k] * sRow[k * kRec + fx];
+          dy = dy + Db[k] * sCol[NP * k * kRec + fy];
         }
-        const double cx = xJ[1][v][ixL] * gLa + xJ[0][v][ixR] * gRa;
-        const double cy = yJ[bot][1][v][iy] * gLb + yJ[top][0][v][iy] * gRb;
-        double o = -div_const(dfx + cx, g.dx) - div_const(dgy + cy, g.dy);
-        if (v == IHP) o = o - Bx - By;
-        const double k4 = o + pick(S, v);
-        const unsigned vi = gn + (unsigned)v * (unsigned)Nd;
+        if (v < 0) { ax = dx; ay = dy; return; }
+        ax = dx + (sJx[kJSide + v * kJ] * gLa + sJx[v * kJ + NP] * gRa);
+        ay = dy + (jB[kJSide + v * kJ] * gLb + jT[v * kJ] * gRb);
+      };
+      double hx, hy;
+      const SweepArgs R = opaque(A);
+      auto finish = [&](int v, double k4, size_t pl) {
+        auto put = [&](double* base, double x) { store_at(global_at(base, pl), t8, x); };
         if (MODE == kCand) {
           // rk.cpp:106-108 and the first three terms of :119-120 (k4 is k3 here)
-          sa.uNew[vi] = pick(c0, v) + sa.dt * (pick(c1, v) + 4.0 / 9.0 * k4);
-          sa.zOut[vi] = pick(c2, v) + 1.0 / 3.0 * k4;
+          const double k1 = ext.x0[v], k2 = own.k[v];
+          put(R->sa.uNew, own.u[v] + stDt * (2.0 / 9.0 * k1 + 1.0 / 3.0 * k2 + 4.0 / 9.0 * k4));
+          put(R->sa.zOut, 7.0 / 24.0 * k1 + 0.25 * k2 + 1.0 / 3.0 * k4);
         } else {
-          dU[vi] = k4;
+          put(R->dU, k4);
         }
-        if (MODE == kAxpy && KEEP && sa.y3Out) {
+        if (MODE == kAxpy && KEEP && R->sa.y3Out) {
           // the stage-3 input u + (3/4 dt) k2 of a recomputed step
           // (rk.cpp:104), formed as the elementwise combination forms it
-          sa.y3Out[vi] = P.u.at(v, gn) + sa.a3 * k4;
+          put(R->sa.y3Out, own.u[v] + R->sa.a3 * k4);
         }
         if (MODE == kErr) {
           // rk.cpp:119-129 for this entry
-          const double u0 = pick(c0, v), un = sU[v][t];
-          const double uEmb = u0 + sa.dt * (pick(c2, v) + 0.125 * k4);
+          const double u0 = ext.x0[v], un = sOwn[v];
+          const double uEmb = u0 + stDt * (ext.x1[v] + 0.125 * k4);
           const double e = un - uEmb;
           const double au = fabs(u0), an = fabs(un);
-          const double r_ = e / (sa.atol + sa.rtol * ((au < an) ? an : au));
+          const double r_ = e / (atol + rtol * ((au < an) ? an : au));
           acc_add(eS, eC, r_ * r_);
           const double ar = fabs(r_);
           eM = (eM < ar) ? ar : eM;
         }
       };
-      if (WAVES == 3 && MODE == kAxpy) {
-        // one variable per trip keeps the LDS operands of a single variable
-        // live (the register budget of three waves per SIMD)
-#pragma unroll 1
-        for (int v = 0; v < NV; ++v) variable(v);
-      } else {
-        // unrolled, so that the per-node operands stay in registers without
-        // selects. Scheduling fences bound how far the LDS operands of later
-        // variables are hoisted: the stage builds take two groups, (the depth
-        // gradient, h, hu) and (hv, hw, hp), which lets one variable's LDS
-        // reads overlap another's arithmetic within their two-wave register
-        // budget (k4 2.5 %, stage 3 1.5 %, the two-wave stage 2 2.4 % faster,
-        // same bits); the plain build keeps the depth gradient and each
-        // variable in a group of its own (grouped, it ran slower)
-        constexpr bool kGrouped = MODE != kPlain;
+      // A scheduling group: the quotients of the entries [e0, e1), -2 the
+      // still-depth gradient (HXR), -1 the depth gradient, v >= 0 variable v,
+      // by the branch-free sequence; then, where a lane of the wave has one
+      // outside its range or not finite, by IEEE division (+ 0.0: the
+      // reference's sums are never -0); then the variables' results.
+      auto group = [&](auto e0_, auto e1_) {
+        constexpr int e0 = decltype(e0_)::value, e1 = decltype(e1_)::value, n = e1 - e0;
+        double ax[n], ay[n], qx[n], qy[n];
+        int bad = never_fast;
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-          if (kGrouped ? v == 2 : true) __builtin_amdgcn_sched_barrier(0);
-          variable(v);
+        for (int i = 0; i < n; ++i) {
+          const int v = e0 + i;
+          if (v == -2) sums(L::kH, L::kH, -1, ax[i], ay[i]);
+          else if (v == -1) sums(IH, IH, NV, ax[i], ay[i]);
+          else sums(L::offF(v), L::offG(v), v, ax[i], ay[i]);
+          qx[i] = div_unchecked(ax[i], divX);
+          qy[i] = div_unchecked(ay[i], divY);
+          bad |= (int)div_needs_exact(ax[i]) | (int)div_needs_exact(ay[i]) |
+                 (int)!(fabs(qx[i] + qy[i]) < HUGE_VAL);
         }
-      }
+        if (__builtin_expect(wave_any(bad), 0)) {
+#pragma unroll
+          for (int i = 0; i < n; ++i) {
+            qx[i] = (ax[i] + 0.0) / divX.b;
+            qy[i] = (ay[i] + 0.0) / divY.b;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+          const int v = e0 + i;
+          if (v == -2) {
+            // sgn2d.cpp:54-71: Hx, Hy = (D H) / J along the node's x and y lines
+            source_rest(sp, qu, qv, qw, qx[i], qy[i], ph, S);
+          } else if (v == -1) {
+            hx = qx[i];
+            hy = qy[i];
+          } else {
+            // the non-conservative products enter hp only (the others' are
+            // zero, and subtracting zero changes no sum)
+            double o = -qx[i] - qy[i];
+            if (v == IHP) o = o - ph.mc2 * qu * hx - ph.mc2 * qv * hy;
+            finish(v, o + S[v], rowOff + (size_t)v * plane);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      // One entry per group: with two or more, the compiler hoists the LDS
+      // operands of the later ones over the first and needs 30 to 70 registers
+      // more, which costs a wave per SIMD.
+      if (HXR) group(IntC<-2>{}, IntC<-1>{});
+      group(IntC<-1>{}, IntC<0>{});
+      group(IntC<0>{}, IntC<1>{});
+      group(IntC<1>{}, IntC<2>{});
+      group(IntC<2>{}, IntC<3>{});
+      group(IntC<3>{}, IntC<4>{});
+      group(IntC<4>{}, IntC<5>{});
     }
-    __syncthreads();
-  }
+    row_sync();
+    rowOff += rowBytes;
+  };
+  for (int r = ey0; r < ey1; ++r) row(r);
 
   if (MODE == kErr) {
+    if (!isNode) eS = eC = eM = 0.0;                     // node 0 counts once
     // fixed-order reduction over the workgroup (LDS of the last row reused)
-    block_reduce(eS, eC, eM, &sF[0][0]);
+    block_reduce(eS, eC, eM, lds.node);
     if (t == 0) {
-      sa.part[3 * tile] = eS;
-      sa.part[3 * tile + 1] = eC;
-      sa.part[3 * tile + 2] = eM;
+      double* const part = A->sa.part + 3 * (size_t)tile;
+      part[0] = eS;
+      part[1] = eC;
+      part[2] = eM;
     }
   }
 }
 
+// The arguments are the kernel's only parameter, read where they lie.
 template <int TW, int MODE, int WAVES, bool KEEP = false, bool HXR = false>
-__global__ void __launch_bounds__(Sweep<TW>::NT, WAVES)
-k_rhs_sweep(const double* __restrict__ U, double* __restrict__ dU, Geometry g, Phys ph,
-            GhostTime gt, Stage sa, int nStrips) {
-  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(U, dU, g, ph, gt, sa, nStrips,
-                                         xcd_tile(blockIdx.x, gridDim.x));
+__global__ void __launch_bounds__(Sweep<TW>::NT, WAVES) k_rhs_sweep(BatchMember) {
+  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(
+      (SweepArgs)__builtin_amdgcn_kernarg_segment_ptr(),
+      xcd_tile(blockIdx.x, gridDim.x));
 }
 
 // Many grids in one launch: the workgroups of every member's tiles, packed
@@ -904,11 +982,15 @@ k_rhs_sweep_batch(const BatchMember* __restrict__ mem, const long long* __restri
     const int mid = (lo + hi + 1) >> 1;
     if (tileStart[mid] <= w) lo = mid; else hi = mid - 1;
   }
-  const BatchMember& M = mem[lo];
-  const long long tile = w - tileStart[lo];
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  const size_t at = reinterpret_cast<size_t>(mem + lo);
+  const SweepArgs M = reinterpret_cast<SweepArgs>(
+      (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)at) |
+      (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32);
+  const int tile = __builtin_amdgcn_readfirstlane((int)(w - tileStart[lo]));
   // a grid larger than the members' tiles (never launched so) does nothing
-  if (tile >= M.nTiles) return;
-  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(M.U, M.dU, M.g, M.ph, M.gt, M.sa, M.nStrips, (int)tile);
+  if (tile >= M->nTiles) return;
+  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(M, tile);
 }
 
 // Hx, Hy at every node (sgn2d.cpp:54-71).
@@ -1205,14 +1287,9 @@ namespace {
 // one row-sweep launch of a (mode, waves, keep) build, with the still-depth
 // gradients read (hxr false) or formed from Hnod (hxr true)
 template <int M, int W, bool K>
-void sweep_launch(bool hxr, dim3 grid, dim3 block, hipStream_t st, const double* U, double* dU,
-                  const Geometry& g, const Phys& ph, GhostTime gt, const Stage& sa, int strips) {
-  if (hxr)
-    hipLaunchKernelGGL((k_rhs_sweep<kTileW, M, W, K, true>), grid, block, 0, st, U, dU, g, ph, gt,
-                       sa, strips);
-  else
-    hipLaunchKernelGGL((k_rhs_sweep<kTileW, M, W, K, false>), grid, block, 0, st, U, dU, g, ph, gt,
-                       sa, strips);
+void sweep_launch(bool hxr, dim3 grid, dim3 block, hipStream_t st, const BatchMember& a) {
+  if (hxr) hipLaunchKernelGGL((k_rhs_sweep<kTileW, M, W, K, true>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((k_rhs_sweep<kTileW, M, W, K, false>), grid, block, 0, st, a);
 }
 
 template <int M, int W, bool K>
@@ -1241,8 +1318,9 @@ hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const S
   // Hx, Hy formed from Hnod (when the device check allowed it) in the
   // two-wave stage builds; the plain build and the three-wave stage-2 build
   // have no registers for it and read them
-  const bool hxr = g.hxr != 0 && mode != kPlain && !(mode == kAxpy && w3);
-#define SGNX_SWEEP(M, W, K) sweep_launch<M, W, K>(hxr, grid, block, st, sa.u, dU, g, ph, gt, sa, strips)
+  const bool hxr = g.hxr != 0;
+  const BatchMember args{sa.u, dU, g, ph, gt, sa, strips, (int)tiles};
+#define SGNX_SWEEP(M, W, K) sweep_launch<M, W, K>(hxr, grid, block, st, args)
   const bool keep = sa.yOut != nullptr;
   if (mode == kPlain) { if (w3) SGNX_SWEEP(kPlain, 3, false); else SGNX_SWEEP(kPlain, 2, false); }
   else if (mode == kAxpy) {
@@ -1264,7 +1342,6 @@ hipError_t launch_rhs_stage_batch(const BatchMember* mem, const long long* tileS
   if (nMem < 1 || totalTiles < 1 || totalTiles > 0x7fffffffLL) return hipErrorInvalidValue;
   if (mode < kPlain || mode > kErr) return hipErrorInvalidValue;
   const dim3 grid((unsigned)totalTiles), block(Sweep<kTileW>::NT);
-  hxr = hxr && mode != kPlain && !(mode == kAxpy && waves3);
 #define SGNX_SWEEPB(M, W, K) sweep_launch_batch<M, W, K>(hxr, grid, block, st, mem, tileStart, nMem)
   if (mode == kPlain) { if (waves3) SGNX_SWEEPB(kPlain, 3, false); else SGNX_SWEEPB(kPlain, 2, false); }
   else if (mode == kAxpy && keep) { if (waves3) SGNX_SWEEPB(kAxpy, 3, true); else SGNX_SWEEPB(kAxpy, 2, true); }
