@@ -12,44 +12,32 @@
 
 namespace sgnx {
 
-// out = acc0 + acc1 + acc2 + (dR/dU (U))^T W,  W = ca*A + cb*B,
-// thetaBar += (dR/dtheta)^T W  (when not null).
-// A, B, acc* and out are 5*Nd arrays; any acc* or B may be null; out may be
-// the same array as A or an acc* (every node is read before it is written,
-// by the thread that writes it). coef: 120*Nx*Ny doubles of scratch.
+// W = ca*A (+ cb*B when B is given); out = (dR/dU (U))^T W, or, when acc is
+// given (with B), ((A + acc) + B) + that; thetaBar += (dR/dtheta)^T W (when not
+// null). 5*Nd arrays; out is none of the inputs (a workgroup reads its
+// neighbours' A and B).
 struct VjpArgs {
   const double* U;
   const double* A;
   double ca;
   const double* B;
   double cb;
-  const double* acc0;
-  const double* acc1;
-  const double* acc2;
+  const double* acc;
   double* out;
   double* thetaBar;
-  double* coef;
-  // Optional (coefNext not null): the launch also writes the face
-  // coefficients of the step's next product, whose cotangent is
-  // can*An + cbn*out (out: this product's result) at the state Un, into
-  // coefNext -- what the coefficient kernel would write for it.
-  const double* Un;
-  const double* An;
-  double can, cbn;
-  double* coefNext;
-  bool coefReady;   // coef already holds this product's coefficients
 };
 
-inline long long vjp_coef_doubles(const Geometry& g) { return 120LL * g.Nx * g.Ny; }
-
-// Batched forms (one launch over every member, tiles packed behind a
-// per-member offset table as in the batched RHS): a product per member ...
+// One product with its geometry and decomposition: a launch's arguments, or
+// one member of a batched launch (tiles packed behind a per-member offset
+// table as in the batched RHS)
 struct VjpMember {
   VjpArgs va;
   Geometry g;
   Phys ph;
   GhostTime gt;
+  int nStrips, nTiles;
 };
+VjpMember vjp_member(const Geometry& g, const Phys& ph, const VjpArgs& va, GhostTime gt);
 // ... and one gauge log row's cotangents per member (Gb null: none)
 struct GaugeMember {
   const double* Gb;
@@ -59,8 +47,12 @@ struct GaugeMember {
   double* thetaBar;
 };
 long long vjp_tiles(const Geometry& g);       // workgroups of one product launch
+long long vjp_row_tiles(const Geometry& g);   // strips times element rows
+// element rows per workgroup for the grids of one launch (Geometry::vrows)
+int vjp_rows(const Geometry* const* g, int n, int cus);
+// nop: 1 = A only, 2 = A and B, 3 = with acc too, for all members
 hipError_t launch_rhs_vjp_batch(const VjpMember* mem, const long long* tileStart, int nMem,
-                                long long totalTiles, bool coefReady, hipStream_t st);
+                                long long totalTiles, int nop, hipStream_t st);
 hipError_t launch_gauge_bar_batch(const GaugeMember* gm, int nMem, hipStream_t st);
 
 hipError_t launch_rhs_vjp(const Geometry& g, const Phys& ph, const VjpArgs& va, GhostTime gt,

@@ -14,18 +14,13 @@
 //               face depth of an interface line node the mean of the two edge
 //               values meeting there (the one interior value on a non-periodic
 //               side); sgnx_set_depth builds that still depth.
-// Two launches:
-//   k_vjp_coef  per element line: the cotangents of the FR lift's face jumps
-//               (the transposed lift, Lambda = -(g' . W)/J) and of the
-//               central face depths of the non-conservative products
-//               (lambda = (g' . W_hp c^2 u)/J), 6 numbers per face node;
-//   k_vjp_elem  per element: the volume adjoint (source, non-conservative
-//               products, nodal fluxes through D^T), and for each face node the
-//               Rusanov adjoint of every interface line its edge state feeds,
-//               kept for the own side only (each interior line is thus
-//               evaluated by both of its elements), the derivative of
-//               max(sL, sR) taken on the side that attains it, walls mirrored
-//               back onto the interior state, the inflow ghost constant.
+// One launch (vjp_tile): the transposed lift gives each face node the cotangents
+// of its line's face jumps, Lambda = -(g' . W)/J, and of the central face depths
+// of the non-conservative products, lambda = (g' . W_hp c^2 u)/J; each interface
+// line's Rusanov adjoint takes them, the derivative of max(sL, sR) on the side
+// that attains it, walls mirrored back onto the interior state, the inflow ghost
+// constant; the volume adjoint (source, non-conservative products, nodal fluxes
+// through D^T) adds each node's parts of the lines around its element.
 // Every sum has one writer and a fixed order, so the results are
 // deterministic. The products are the derivatives of R away from its
 // non-smooth points (a zero normal velocity, sL = sR off a wall, a clamped
@@ -35,15 +30,15 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "sgnx_adjoint.h"
+#include "sgnx_device.h"
 
 namespace sgnx {
 namespace {
 
 constexpr int kT = 256;    // threads per block of the elementwise kernels
-constexpr int kEW = 5;     // elements per tile of k_vjp_coef / k_vjp_elem (one element row)
-constexpr int kVT = ((kEW * NPP + 63) / 64) * 64;   // their threads per block (whole waves)
-static_assert(20 * kEW <= kVT, "one thread per element face node");
 
 // --- pointwise adjoints of sgnx_phys.h (nManning = 0) --------------------------
 // Every term is differentiated with the primitives u = hu/h, v, w, p as
@@ -136,454 +131,492 @@ __device__ __forceinline__ void node_terms_acc(const St& s, double Hl, double Hx
   q.p += ph.gamma * W[IHW] + ph.gamma * bathb;
 }
 
-// One interface line node: Fs = 0.5 (FL + FR) - 0.5 lam (UR - UL) with its
-// cotangent LamL + LamR, the two sides' own face fluxes FL, FR (same state,
-// same face depth) with cotangents -LamL, -LamR, and the central depth
-// 0.5 (hL + hR) with cotangent lh. UbL, UbR = the state cotangents; returns the
-// face-depth cotangent.
-template <int DIR>
-__device__ __forceinline__ double line_bar(const double* UL, const double* UR, double Hf,
-                                           const double* LamL, const double* LamR, double lh,
-                                           const Phys& ph, double* UbL, double* UbR) {
-  const St L = make_st(UL), R = make_st(UR);
-  const double aL = ph.g * L.h + L.p + ph.c2, aR = ph.g * R.h + R.p + ph.c2;
-  const double gL = sqrt(aL > 0.0 ? aL : 0.0), gR = sqrt(aR > 0.0 ? aR : 0.0);
-  const double sL = fabs(DIR == 0 ? L.u : L.v) + gL;
-  const double sR = fabs(DIR == 0 ? R.u : R.v) + gR;
-  const double hl = 0.5 * fmax(sL, sR);
-  PrimBar qL{0.0, 0.0, 0.0, 0.0}, qR{0.0, 0.0, 0.0, 0.0};
-  double FbL[NV], FbR[NV], hlb = 0.0;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const double Fsb = LamL[k] + LamR[k];
-    FbL[k] = 0.5 * Fsb - LamL[k];
-    FbR[k] = 0.5 * Fsb - LamR[k];
-    UbL[k] = hl * Fsb;
-    UbR[k] = -hl * Fsb;
-    hlb -= Fsb * (UR[k] - UL[k]);
-  }
-  UbL[IH] += 0.5 * lh;
-  UbR[IH] += 0.5 * lh;
-  if (sL > sR) speed_acc<DIR>(L, gL, ph, 0.5 * hlb, UbL, qL);
-  else speed_acc<DIR>(R, gR, ph, 0.5 * hlb, UbR, qR);
-  const double hfb = flux_acc<DIR>(L, Hf, ph, FbL, UbL, qL) + flux_acc<DIR>(R, Hf, ph, FbR, UbR, qR);
-  prims_fin(L, qL, UbL);
-  prims_fin(R, qR, UbR);
-  return hfb;
+// a value that is the same on every lane, in scalar registers
+__device__ __forceinline__ double uniform_value(double x) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(x)));
 }
 
-__device__ __forceinline__ double cot_at(const VjpArgs& va, long long j) {
-  double w = va.ca * va.A[j];
-  if (va.B) w = w + va.cb * va.B[j];
-  return w;
-}
+// ---- the product, row sweep ---------------------------------------------------
+//
+// A workgroup owns a strip of kEW element columns and a chunk of g.vrows
+// element rows and walks up the chunk. Per row r:
+//   stage  row r's nodes (one per lane; the elements left and right of the
+//          strip too, whose lines' Lambda the strip's outer lines need): state,
+//          cotangent W and the integrands of the depth-gradient cotangents,
+//          c^2 W_hp u / Jx and c^2 W_hp v / Jy, to LDS; row r + 1's loads are
+//          issued
+//   faces  two lanes per interface line node, one per side: the x lines of
+//          row r and the y line between rows r - 1 and r. Each lane forms its
+//          own side's lift cotangents from its element's line,
+//            Lambda = -(g' . W)/J (of the FR lift's face jump) and
+//            lambda = g' . (c^2 W_hp vel / J) (of the central face depth),
+//          the pair exchanges states and Lambda by lane permutes, and each
+//          lane keeps the Rusanov adjoint of its own side. The lower row's
+//          side of a y line (Lambda, lambda, edge state) was kept in LDS when
+//          that row was staged. A y line is handled in the x frame: with P the
+//          exchange of hu and hv, flux_y(U) = P flux_x(P U), so its adjoint is
+//          P applied to the x adjoint of the exchanged states and cotangents.
+//   lines  meanwhile on the wave without interface lines, a lane per element
+//          line: D^T along it of W and of the depth gradients' integrand, of row
+//          r - 1's Hx, Hy cotangents, and D of h, all five nodes at once, with
+//          D in scalar registers
+//   nodes  row r - 1 is finished (the upper y line's part of its top nodes, the
+//          Hx, Hy cotangents' sums, the stores) and row r's node adjoint formed
+//          from the line sums: source, non-conservative products, nodal fluxes,
+//          depth gradients, its other faces' parts.
+// One row below the chunk is staged for the lower side of its first y line and
+// one above for the upper side of its last.
+//
+// The face depths drop out: an interface's flux and the two elements' own face
+// fluxes take the same depth, and its cotangents, with FbL + FbR = Fsb - LamL -
+// LamR = 0 in the momentum row, cancel. A periodic axis has two lines on its
+// wrap, each feeding one element; the adjoint is linear in Lambda and, but for
+// the face depth, the same on both, so one evaluation with both Lambda serves.
+//
+// What bounds it: a step's products move 160, 200 and 240 B a node, 434, 543 and
+// 651 us at 1024x512 at a copy's rate; they take 560, 668 and 850 us (2.1 to 2.2
+// ms for the three; per-element coefficients written to and read from memory by
+// a launch of their own, each line evaluated by both of its elements: 3.8 ms).
+// The rest is LDS traffic and the row's barriers, met by the four workgroups
+// that 160 KB and 168 registers let a compute unit hold (three of the third
+// product, whose sum of the other cotangents waits in LDS for a row). The line
+// sums taken by the line lanes instead of by every node for itself, each
+// reading 80 values: 615 -> 560 and 700 -> 668 us. A third product that keeps
+// that sum in global memory between the rows, for four workgroups: 1028 us.
+constexpr int kEW = 5;                       // element columns of a strip
+constexpr int kVT = 192;                     // threads: 125 nodes, 50 halo nodes
+static_assert(NPP * (kEW + 2) <= kVT && kVT % 64 == 0, "one lane per staged node");
 
-// local node of face f (0 left, 1 right, 2 bottom, 3 top), line node n
-__device__ __forceinline__ int face_loc(int f, int n) {
-  return f == 0 ? NP * n : f == 1 ? NP - 1 + NP * n : f == 2 ? n : n + NP * (NP - 1);
-}
-
-// ---- element tiles --------------------------------------------------------------
-// Both launches work on tiles of kEW elements of one element row, one node per
-// thread; the tile's cotangents W and the integrands of the depth-gradient
-// cotangents, c^2 W_hp u / Jx and c^2 W_hp v / Jy, are staged in LDS.
-struct TileLds {
-  double D[NPP], gL[NP], gR[NP];
-  double W[NV][kEW * NPP];
-  double DX[kEW * NPP], DY[kEW * NPP];
+struct VjpLds {
+  static constexpr int kRec = 13;            // odd: no bank conflicts
+  static constexpr int kW = 0, kU = 5, kDX = 10, kDY = 11, kDhx = 12;
+  static constexpr int kF = NP * (kEW + 1), kNY = NP * kEW, kN = NPP * kEW;
+  static constexpr int kCen = 2 * NV * kF;   // from an own-side cotangent to its central depth
+  static constexpr int kTop = NV + 1 + NV;   // Lambda, lambda, edge state
+  double rec[NPP * (kEW + 2) * kRec];        // strip nodes, left halo, right halo
+  double xU[2][NV][kF], xh[kF];              // own side's cotangents, central depth
+  double yU[2][NV][kF], yh[kF], yhT[kNY];    // the line below row r; central depth above
+  double top[kNY][kTop];                     // the top faces of row r - 1
+  // per node: D^T along x and along y of W and of the depth-gradient
+  // cotangents' integrand, D h along y (along x: kDhx of its record)
+  double sx[NV + 1][kN], sy[NV + 1][kN], dhy[kN];
+  // per node: cotangent of Hx over Jx, of Hy over Jy; then D^T of them
+  double tx[kN], ty[kN];
+  double gw[2][NP];                          // gL', gR'
 };
 
-// Lambda_c = -(g' . W_c)/J along the face's element line (the cotangent of
-// the FR lift's face jump) and lambda = g' . (c^2 W_hp vel / J) (that of the
-// central face depth of the non-conservative products), g' = gL' on a low
-// face, gR' on a high one; f = 0 left, 1 right, 2 bottom, 3 top, line node n
-__device__ __forceinline__ void face_coef(const TileLds& L, int jb, int f, int n, double iJx,
-                                          double iJy, double* Lam, double& lam) {
-  const int dir = f >> 1;
-  const bool hi = (f & 1) != 0;
-  double sum[NV] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  double q = 0.0;
-  // rolled: fewer registers live in the product kernel's face phase (its
-  // four-wave build spills 3 registers instead of 5)
-#pragma unroll 1
-  for (int k = 0; k < NP; ++k) {
-    const int node = jb + (dir == 0 ? k + NP * n : n + NP * k);
-    const double gk = hi ? L.gR[k] : L.gL[k];
-#pragma unroll
-    for (int c = 0; c < NV; ++c) sum[c] = sum[c] + gk * L.W[c][node];
-    q = q + gk * (dir == 0 ? L.DX[node] : L.DY[node]);
-  }
-  const double iJ = dir == 0 ? iJx : iJy;
-#pragma unroll
-  for (int c = 0; c < NV; ++c) Lam[c] = -sum[c] * iJ;
-  lam = q;
-}
-
-// the tile's operator tables and node data; returns the thread's node index
-__device__ __forceinline__ void tile_stage(const VjpArgs& va, const Geometry& g, const Phys& ph,
-                                           TileLds& L, int t, bool isNode, long long i,
-                                           double* sH) {
-  const OpTables* T = g.ops;
-  if (t < NPP) L.D[t] = T->D[t];
-  if (t < NP) {
-    L.gL[t] = T->gLp[t];
-    L.gR[t] = T->gRp[t];
-  }
-  if (!isNode) return;
-  const long long Nd = g.Nd;
-  double W[NV];
+// W = ca A (+ cb B) as the host forms it: products and sum rounded apart
+template <int NOP>
+__device__ __forceinline__ void cotangent(const double* A, const double* B, double ca, double cb,
+                                          double* W) {
 #pragma unroll
   for (int c = 0; c < NV; ++c) {
-    W[c] = cot_at(va, (long long)c * Nd + i);
-    L.W[c][t] = W[c];
+    W[c] = ca * A[c];
+    if (NOP > 1) W[c] = W[c] + cb * B[c];
   }
-  const double h = va.U[i];
-  if (sH) sH[t] = h;
-  const double q = W[IHP] * ph.c2 / h;
-  L.DX[t] = q * va.U[(long long)IHU * Nd + i] * (1.0 / g.Jx);
-  L.DY[t] = q * va.U[(long long)IHV * Nd + i] * (1.0 / g.Jy);
 }
 
-// ---- launch 1: face-line cotangents -----------------------------------------------
-// coef[((e * 4 + f) * NP + n) * 6 + c]: c < 5 Lambda_c, c = 5 lambda
-__device__ __forceinline__ void vjp_coef_tile(const VjpArgs& va, const Geometry& g,
-                                              const Phys& ph, int tile) {
-  __shared__ TileLds L;
+// NOP: 1: W = ca A; 2: W = ca A + cb B; 3: that, and out = ((A + acc) + B) +
+// the product.
+template <int NOP>
+struct VjpLdsOf : VjpLds {};
+template <>
+struct VjpLdsOf<3> : VjpLds {
+  double base[2][NV][kN];                    // (A + acc) + B by row parity
+};
+
+template <int NOP>
+__device__ __forceinline__ void vjp_tile(ConstArgs<VjpMember> M, int tile) {
+  using L = VjpLds;
+  constexpr int kRec = L::kRec;
+  __shared__ VjpLdsOf<NOP> lds;
   const int t = threadIdx.x;
-  const int Nx = g.Nx;
-  const int strips = (Nx + kEW - 1) / kEW;
-  const int ey = tile / strips;
-  const int ex0 = (tile - ey * strips) * kEW;
-  const int nW = min(kEW, Nx - ex0);
-  const int j = t / NPP;
-  const long long i = ((long long)ey * Nx + ex0) * NPP + t;
-  tile_stage(va, g, ph, L, t, j < nW, i, nullptr);
-  __syncthreads();
-  if (t < 20 * nW) {
-    const int jf = t / 20, r = t - 20 * jf;
-    const int f = r / NP, n = r - NP * f;
-    double Lam[NV], lam;
-    face_coef(L, NPP * jf, f, n, 1.0 / g.Jx, 1.0 / g.Jy, Lam, lam);
-    double* cp = va.coef + (((long long)ey * Nx + ex0) * 20 + t) * 6;
+  if (t < NP) {
+    lds.gw[0][t] = M->g.ops->gLp[t];
+    lds.gw[1][t] = M->g.ops->gRp[t];
+  }
+  const double iJx = uniform_value(1.0 / M->g.Jx), iJy = uniform_value(1.0 / M->g.Jy);
+  // read where it is used: kept, it would take scalar registers of the other phases
+  auto phys = [&] {
+    const ConstArgs<VjpMember> P = opaque(M);
+    return Phys{P->ph.g, P->ph.c, P->ph.gamma, 0.0, P->ph.halfg, P->ph.c2, P->ph.mc2, P->ph.m2c2};
+  };
+  const int Nx = M->g.Nx, Ny = M->g.Ny, nStrips = M->nStrips, rows = M->g.vrows;
+  const int bcL = M->g.bc[0], bcR = M->g.bc[1];
+  const bool wallB = M->g.bc[2] != SGNX_BC_PERIODIC, wallT = M->g.bc[3] != SGNX_BC_PERIODIC;
+  const int chunk = __builtin_amdgcn_readfirstlane(tile / nStrips);
+  const int ex0 = (tile - chunk * nStrips) * kEW, nW = min(kEW, Nx - ex0);
+  const int ey0 = chunk * rows, ey1 = min(Ny, ey0 + rows);
+  const size_t plane0 = (size_t)M->g.Nd * sizeof(double);
+  const unsigned rowBytes = (unsigned)Nx * (NPP * 8u);
+  const double ca = M->va.ca, cb = NOP > 1 ? M->va.cb : 0.0;
+
+  // Staged node: a strip node, a halo node (its own record also where there is
+  // no such element), or node 0 again.
+  const bool hasL = ex0 > 0 || bcL == SGNX_BC_PERIODIC;
+  const bool hasR = ex0 + nW < Nx || bcR == SGNX_BC_PERIODIC;
+  const bool isNode = t < NPP * nW;
+  constexpr int kHaloL = NPP * kEW, kHaloR = NPP * (kEW + 1);
+  const bool inL = t >= kHaloL && t < kHaloR, inR = t >= kHaloR && t < NPP * (kEW + 2);
+  const int tn = isNode ? t : 0;
+  const int j = tn / NPP, loc = tn - NPP * j, b = loc / NP, a = loc - NP * b;
+  const int sRecIdx = inL || inR ? t : tn;
+  unsigned n8;                               // its byte offset within a row of a plane
+  if (inL) n8 = (unsigned)((hasL ? (ex0 > 0 ? ex0 - 1 : Nx - 1) : ex0) * NPP + t - kHaloL) * 8u;
+  else if (inR) n8 = (unsigned)((hasR ? (ex0 + nW < Nx ? ex0 + nW : 0) : ex0) * NPP + t - kHaloR) * 8u;
+  else n8 = (unsigned)(ex0 * NPP + tn) * 8u;
+
+  // Interface half-items, from the third wave (which has no node) on: two
+  // lanes per line node, lane 2k + side taking side 0 (left / lower) or 1.
+  const int nX = NP * (nW + 1);
+  const int it = t < 128 ? t + 64 : t - 128, side = it & 1, kk = it >> 1;
+  const bool isItem = kk < nX + NP * nW;
+  const bool isX = kk < nX;
+  const int xi = isX ? kk / NP : 0, xn = isX ? kk - NP * xi : 0;
+  const int ky = !isX && isItem ? kk - nX : 0, jj = ky / NP, aa = ky - NP * jj;
+  const bool outL = isX && side == 0 && xi == 0, outR = isX && side == 1 && xi == nW;
+  const bool ghostX = (outL && !hasL) || (outR && !hasR);
+  const bool inflow = ghostX && outL && bcL == SGNX_BC_INFLOW;
+  // the other side of this lane's line is a wall's ghost
+  const bool wallX = isX && ((side == 1 && xi == 0 && !hasL && bcL == SGNX_BC_WALL) ||
+                             (side == 0 && xi == nW && !hasR));
+  const bool lowerY = !isX && side == 0, upperY = !isX && side == 1;
+  // the element line whose Lambda the lane forms (y, lower side: that of row
+  // r's top, kept for the next row), its weights, and its edge node
+  int rec0;
+  if (isX) rec0 = outL ? kHaloL : outR ? kHaloR : NPP * (xi - 1 + side);
+  else rec0 = NPP * jj;
+  LdsDouble* sLine = (LdsDouble*)lds.rec + (rec0 + (isX ? NP * xn : aa)) * kRec;
+  const int step = (isX ? 1 : NP) * kRec;
+  LdsDouble* sEdge = sLine + (side == 0 ? NP - 1 : 0) * step;
+  LdsDouble* sGw = (LdsDouble*)lds.gw[side == 0 ? 1 : 0];
+  const int dOff = isX ? L::kDX : L::kDY;
+  const double miJ = isX ? -iJx : -iJy;
+  LdsDouble* sTop = (LdsDouble*)lds.top[ky];
+  LdsDouble* sOut = isX ? (LdsDouble*)lds.xU[side][0] + kk : (LdsDouble*)lds.yU[side][0] + ky;
+  unsigned h8 = (unsigned)((ex0 + jj) * NPP + aa) * 8u;   // the column's bottom face node
+
+  // Element lines, on the second wave (which has no half-item): lanes 0-24 the
+  // x lines, 25-49 the y lines, each all five nodes of its line.
+  const int ln = t - 64, ll = ln < NP * kEW ? ln : ln - NP * kEW;
+  const bool lineX = ln < NP * kEW, isLine = ln >= 0 && ln < 2 * NP * kEW && ll < NP * nW;
+  const int le = isLine ? ll / NP : 0, lq = isLine ? ll - NP * le : 0;
+  const int lNode = NPP * le + (lineX ? NP * lq : lq), lStep = lineX ? 1 : NP;
+
+  struct Raw {
+    double U[NV], A[NV], B[NOP > 1 ? NV : 1], acc[NOP > 2 ? NV : 1];
+  };
+  // row `to`, clamped to the grid (where it is beyond a wall nothing of it is
+  // used) and wrapped on a periodic axis
+  auto row_of = [&](int to) {
+    to = to < 0 ? (wallB ? 0 : Ny - 1) : to;
+    to = to >= Ny ? (wallT ? Ny - 1 : min(to - Ny, Ny - 1)) : to;
+    return __builtin_amdgcn_readfirstlane((int)((unsigned)to * rowBytes));
+  };
+  auto load_row = [&](ConstArgs<VjpMember> R, int to, size_t plane, unsigned off, Raw& x) {
+    const unsigned first = (unsigned)row_of(to);
+    load_vars(R->va.U, first, plane, off, x.U);
+    load_vars(R->va.A, first, plane, off, x.A);
+    if (NOP > 1) load_vars(R->va.B, first, plane, off, x.B);
+    if (NOP > 2) load_vars(R->va.acc, first, plane, off, x.acc);
+  };
+  auto load_h = [&](ConstArgs<VjpMember> R, int to, unsigned off) {
+    return load_at(global_at(R->va.U, (unsigned)row_of(to)), off);
+  };
+
+  LdsDouble* sRec = (LdsDouble*)lds.rec + sRecIdx * kRec;
+  LdsDouble* sXU = (LdsDouble*)lds.xU[0][0] + NP * j + b;
+  LdsDouble* sYU = (LdsDouble*)lds.yU[0][0] + NP * j + a;
+  LdsDouble* sNode = (LdsDouble*)lds.sx[0] + (t < L::kN ? t : 0);
+  constexpr int kSy = (NV + 1) * L::kN, kDhy = 2 * kSy, kTx = kDhy + L::kN, kTy = kTx + L::kN;
+  LdsDouble* sL = (LdsDouble*)lds.rec + lNode * kRec;
+  LdsDouble* sSum = (LdsDouble*)(lineX ? lds.sx[0] : lds.sy[0]) + lNode;
+
+  Raw raw;
+  load_row(M, ey0 - 1, plane0, n8, raw);
+  double hAbove = load_h(M, ey0, h8);          // of the row after the one staged next
+  // row r - 1's node results: the product without its top faces' part, what it
+  // is added to, its still-depth cotangent
+  double pend[NV], th = 0.0;
+
+  for (int r = ey0 - 1; r <= ey1; ++r) {
+    size_t plane = plane0;
+    __asm__ volatile("" : "+s"(plane));
+    __asm__ volatile("" : "+v"(n8));
+    __asm__ volatile("" : "+v"(h8));
+    for (LdsDouble** q : {&sRec, &sXU, &sYU, &sNode, &sLine, &sEdge, &sOut, &sTop, &sL, &sSum})
+      __asm__ volatile("" : "+v"(*q));
+    // ---- stage ---------------------------------------------------------------
+    const ConstArgs<VjpMember> R0 = opaque(M);
+    double* const tbar = R0->va.thetaBar;
+    const double thOld = load_at(global_at(tbar ? tbar : R0->va.U, (unsigned)row_of(r - 1)), n8);
+    const double hNext = load_h(R0, r + 2, h8);
+    const unsigned rowAt = (unsigned)row_of(r);
+    const double Hl = load_at(global_at(R0->g.Hnod, rowAt), n8);
+    const double Hx = load_at(global_at(R0->g.Hx, rowAt), n8);
+    const double Hy = load_at(global_at(R0->g.Hy, rowAt), n8);
+    {
+      double W[NV];
+      cotangent<NOP>(raw.A, raw.B, ca, cb, W);
+      const double q = W[IHP] * R0->ph.c2 / raw.U[IH];
 #pragma unroll
-    for (int c = 0; c < NV; ++c) cp[c] = Lam[c];
-    cp[NV] = lam;
+      for (int c = 0; c < NV; ++c) {
+        sRec[L::kW + c] = W[c];
+        sRec[L::kU + c] = raw.U[c];
+        if constexpr (NOP > 2)
+          if (t < NPP * kEW) lds.base[r & 1][c][t] = (raw.A[c] + raw.acc[c]) + raw.B[c];
+      }
+      sRec[L::kDX] = q * raw.U[IHU] * iJx;
+      sRec[L::kDY] = q * raw.U[IHV] * iJy;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load_row(opaque(M), r + 1, plane, n8, raw);
+    row_sync();
+
+    // ---- faces -----------------------------------------------------------------
+    if (isItem && (!isX || (r >= ey0 && r < ey1))) {
+      double La[NV], la, E[NV];
+      {
+        double w = sGw[0];
+#pragma unroll
+        for (int c = 0; c < NV; ++c) La[c] = w * sLine[L::kW + c];
+        la = w * sLine[dOff];
+#pragma unroll
+        for (int k = 1; k < NP; ++k) {
+          w = sGw[k];
+#pragma unroll
+          for (int c = 0; c < NV; ++c) La[c] = fma(w, sLine[k * step + L::kW + c], La[c]);
+          la = fma(w, sLine[k * step + dOff], la);
+        }
+#pragma unroll
+        for (int c = 0; c < NV; ++c) {
+          La[c] = La[c] * miJ;
+          E[c] = sEdge[L::kU + c];
+        }
+      }
+      if (lowerY) {
+        // row r's top faces for the next row; row r - 1's for this line
+        const bool atWall = wallT && r + 1 == Ny;
+        lds.yhT[ky] = 0.5 * (E[IH] + (atWall ? E[IH] : hAbove));
+        double o[L::kTop];
+#pragma unroll
+        for (int c = 0; c < L::kTop; ++c) o[c] = sTop[c];
+#pragma unroll
+        for (int c = 0; c < NV; ++c) {
+          sTop[c] = La[c];
+          sTop[NV + 1 + c] = E[c];
+          La[c] = o[c];
+          E[c] = o[NV + 1 + c];
+        }
+        sTop[NV] = la;
+        la = o[NV];
+      }
+      auto to_frame = [&](double* x) {
+        const double u_ = x[IHU], v_ = x[IHV];
+        x[IHU] = isX ? u_ : v_;
+        x[IHV] = isX ? v_ : u_;
+      };
+      to_frame(E);
+      to_frame(La);
+      const bool lowWall = wallB && r == 0, topWall = wallT && r == Ny;
+      const bool ghost = ghostX || (lowerY && lowWall) || (upperY && topWall);
+      const bool wallOther = wallX || (upperY && lowWall) || (lowerY && topWall);
+      if (wave_any(ghost)) {
+        double o[NV];
+#pragma unroll
+        for (int c = 0; c < NV; ++c) o[c] = lane_swap(E[c]);
+        if (ghost) {
+#pragma unroll
+          for (int c = 0; c < NV; ++c) {
+            E[c] = c == IHU ? -o[c] : o[c];
+            La[c] = 0.0;
+          }
+          la = 0.0;
+          if (inflow) {
+            const int rr = min(max(r, 0), Ny - 1);   // (rows outside the grid are not used)
+            const GlobalDouble* cf =
+                (const GlobalDouble*)R0->g.inflow + ((size_t)rr * NP + xn) * (NV * 3);
+#pragma unroll
+            for (int c = 0; c < NV; ++c)
+              E[c] = (cf[3 * c] + cf[3 * c + 1] * R0->gt.s) + cf[3 * c + 2] * R0->gt.c;
+          }
+        }
+      }
+      // Fs = 0.5 (FL + FR) - 0.5 lam (UR - UL) with its cotangent LamL + LamR,
+      // the sides' own face fluxes with cotangents -LamL, -LamR, the central
+      // depth 0.5 (hL + hR) with cotangent lamL + lamR and the own edge depth
+      // with -lam
+      const Phys ph = phys();
+      const St s = make_st(E);
+      const double arg = ph.g * s.h + s.p + ph.c2;
+      const double sig = sqrt(arg > 0.0 ? arg : 0.0);
+      const double sp = fabs(s.u) + sig, so = lane_swap(sp);
+      const double hl = flip_sign(0.5 * fmax(sp, so), side << 31);
+      double Ub[NV], Fb[NV], dot = 0.0;
+#pragma unroll
+      for (int c = 0; c < NV; ++c) {
+        const double Fsb = La[c] + lane_swap(La[c]);
+        const double Eo = lane_swap(E[c]);
+        if (c == IH && side == 0) sOut[L::kCen] = 0.5 * (E[c] + Eo);
+        Ub[c] = hl * Fsb;
+        Fb[c] = fma(0.5, Fsb, -La[c]);
+        dot = fma(Fsb, Eo - E[c], dot);
+      }
+      Ub[IH] = fma(0.5, la + lane_swap(la), Ub[IH]) - la;
+      PrimBar q{0.0, 0.0, 0.0, 0.0};
+      const double hlb = side == 0 ? -dot : dot;
+      if (side == 0 ? sp > so : !(so > sp)) speed_acc<0>(s, sig, ph, 0.5 * hlb, Ub, q);
+      flux_acc<0>(s, 0.0, ph, Fb, Ub, q);
+      prims_fin(s, q, Ub);
+      if (wave_any(wallOther)) {
+        // a wall's ghost is the own state with the normal momentum negated
+#pragma unroll
+        for (int c = 0; c < NV; ++c) {
+          const double o = lane_swap(Ub[c]);
+          if (wallOther) Ub[c] = c == IHU ? Ub[c] - o : Ub[c] + o;
+        }
+      }
+      to_frame(Ub);
+#pragma unroll
+      for (int c = 0; c < NV; ++c) sOut[c * L::kF] = Ub[c];
+    }
+    // ---- lines -----------------------------------------------------------------
+    if (isLine) {
+      const auto* const T = (ConstArgs<OpTables>)opaque(M)->g.ops;
+      // out[a] = sum over k of D[k][a] in[k]
+      auto transposed = [&](const LdsDouble* in, int inStep, LdsDouble* out) {
+        double x[NP];
+#pragma unroll
+        for (int k = 0; k < NP; ++k) x[k] = in[k * inStep];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          double v = T->D[q] * x[0];
+#pragma unroll
+          for (int k = 1; k < NP; ++k) v = fma(T->D[k * NP + q], x[k], v);
+          out[q * lStep] = v;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      const int in = lStep * kRec;
+#pragma unroll
+      for (int c = 0; c < NV; ++c) transposed(sL + L::kW + c, in, sSum + c * L::kN);
+      transposed(sL + (lineX ? L::kDX : L::kDY), in, sSum + NV * L::kN);
+      LdsDouble* const sT = sSum + (lineX ? kTx : kTy - kSy);
+      transposed(sT, lStep, sT);
+      double h[NP];
+#pragma unroll
+      for (int k = 0; k < NP; ++k) h[k] = sL[k * in + L::kU];
+      LdsDouble* const to = lineX ? sL + L::kDhx : sSum + (kDhy - kSy);
+      const int toStep = lineX ? kRec : NP;
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        double v = T->D[q * NP] * h[0];
+#pragma unroll
+        for (int k = 1; k < NP; ++k) v = fma(T->D[q * NP + k], h[k], v);
+        to[q * toStep] = v;
+      }
+    }
+    row_sync();
+
+    // ---- nodes -----------------------------------------------------------------
+    if (t < NPP * kEW) {
+      if (r > ey0) {
+        // row r - 1
+        const unsigned first = (unsigned)row_of(r - 1);
+        if (b == NP - 1) {
+#pragma unroll
+          for (int c = 0; c < NV; ++c) pend[c] += sYU[c * L::kF];
+        }
+        GlobalByte* p = global_at(R0->va.out, first);
+#pragma unroll
+        for (int c = 0; c < NV; ++c) {
+          double o = pend[c];
+          if constexpr (NOP > 2) o = lds.base[(r - 1) & 1][c][t] + o;
+          if (isNode) store_at(p, n8, o);
+          p += plane;
+        }
+        if (tbar) {
+          // still depth: Hnod = theta, Hx = (D theta)/Jx, Hy = (D theta)/Jy per line
+          th = (th + sNode[kTx]) + sNode[kTy];
+          if (isNode) store_at(global_at(tbar, first), n8, thOld + th);
+        }
+      }
+      if (r >= ey0 && r < ey1) {
+        double U[NV], W[NV];
+#pragma unroll
+        for (int c = 0; c < NV; ++c) {
+          U[c] = sRec[L::kU + c];
+          W[c] = sRec[L::kW + c];
+        }
+        const Phys ph = phys();
+        const St s = make_st(U);
+        // the depth gradient: the line sums and the jumps to the central depths
+        double dhx = sRec[L::kDhx], dhy = sNode[kDhy];
+        {
+          LdsDouble* const x0 = (LdsDouble*)lds.rec + (NPP * j + NP * b) * kRec + L::kU;
+          LdsDouble* const y0 = (LdsDouble*)lds.rec + (NPP * j + a) * kRec + L::kU;
+          LdsDouble* const cx = sXU + L::kCen;
+          LdsDouble* const cy = sYU + L::kCen;
+          dhx += (cx[0] - x0[0]) * lds.gw[0][a] + (cx[NP] - x0[(NP - 1) * kRec]) * lds.gw[1][a];
+          dhy += (cy[0] - y0[0]) * lds.gw[0][b] +
+                 (cy[L::kF] - y0[(NP - 1) * NP * kRec]) * lds.gw[1][b];
+        }
+        double Fb[NV], Gb[NV];
+        double Hlb, Hxb, Hyb;
+        PrimBar q{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int c = 0; c < NV; ++c) {
+          pend[c] = 0.0;
+          Fb[c] = -sNode[c * L::kN] * iJx;
+          Gb[c] = -sNode[kSy + c * L::kN] * iJy;
+        }
+        node_terms_acc(s, Hl, Hx, Hy, dhx * iJx, dhy * iJy, ph, W, pend, q, Hlb, Hxb, Hyb);
+        Hlb += flux_acc<0>(s, Hl, ph, Fb, pend, q);
+        Hlb += flux_acc<1>(s, Hl, ph, Gb, pend, q);
+        prims_fin(s, q, pend);
+        pend[IH] += sNode[NV * L::kN] + sNode[kSy + NV * L::kN];
+        auto face_add = [&](LdsDouble* f) {
+#pragma unroll
+          for (int c = 0; c < NV; ++c) pend[c] += f[c * L::kF];
+        };
+        if (a == 0) face_add(sXU + NV * L::kF);        // upper side of the line on the left
+        if (a == NP - 1) face_add(sXU + NP);            // lower side of the one on the right
+        if (b == 0) face_add(sYU + NV * L::kF);        // upper side of the line below
+        th = Hlb;
+        sNode[kTx] = Hxb * iJx;
+        sNode[kTy] = Hyb * iJy;
+      }
+    }
+    hAbove = hNext;
+    row_sync();
   }
 }
 
-// ---- launch 2: one element row strip per block ---------------------------------
-__device__ __forceinline__ void vjp_elem_tile(const VjpArgs& va, const Geometry& g,
-                                              const Phys& ph, const GhostTime& gt, int tile) {
-  __shared__ TileLds L;
-  __shared__ double sH[kEW * NPP];
-  __shared__ double sHS[kEW * 20], sLam[kEW * 20], sTF[kEW * 20];
-  __shared__ double sUF[NV][kEW * 20];
-  const int t = threadIdx.x;
-  const int Nx = g.Nx, Ny = g.Ny;
-  const long long Nd = g.Nd;
-  const int strips = (Nx + kEW - 1) / kEW;
-  const int ey = tile / strips;
-  const int ex0 = (tile - ey * strips) * kEW;
-  const int nW = min(kEW, Nx - ex0);
-  const double* U = va.U;
-  const double* sD = L.D;
-  const double* sgL = L.gL;
-  const double* sgR = L.gR;
-  const double iJx = 1.0 / g.Jx, iJy = 1.0 / g.Jy;
-
-  // phase 1: the cotangent loads, the cotangents of the two D-sums and of the
-  // depth gradients of the non-conservative products; the face threads (20
-  // per element, see phase 2) issue their global loads before the barrier too
-  const int j = t / NPP, loc = t - NPP * (t / NPP);
-  const int b = loc / NP, a = loc - NP * b;
-  const bool isNode = j < nW;
-  const long long i = ((long long)ey * Nx + ex0 + j) * NPP + loc;
-  const bool isFace = t < 20 * nW;
-  const int jf = t / 20, r = t - 20 * (t / 20);
-  const int f = r / NP, n = r - NP * f;
-  const int ex = ex0 + jf;
-  const long long e = (long long)ey * Nx + ex;
-  const int dir = f >> 1;
-  const bool ownHigh = (f & 1) == 0;               // own element on the line's high side
-  const int pos = dir == 0 ? ex : ey, nL = dir == 0 ? Nx : Ny;
-  const int sideLo = dir == 0 ? 0 : 2;              // bc index of the low side
-  const bool periodic = g.bc[sideLo] == SGNX_BC_PERIODIC;
-  const int posO = ownHigh ? pos - 1 : pos + 1;
-  const bool inLine = posO >= 0 && posO < nL;
-  const int wrapO = posO < 0 ? nL - 1 : (posO >= nL ? 0 : posO);
-  const int bcSide = ownHigh ? sideLo : sideLo + 1;
-  const bool ghost = !inLine && !periodic;
-  const bool wall = ghost && g.bc[bcSide] == SGNX_BC_WALL;
-  // pass 0: the own line; pass 1 (an edge on the wrap of a periodic axis):
-  // the line at the far end, where only the far element's face is in line
-  const int passes = (!inLine && periodic) ? 2 : 1;
-  double Uo[NV], Uw[NV], Lw[NV], lw = 0.0, hfp[2] = {0.0, 0.0};
-  if (isFace) {
-    const long long io = e * NPP + face_loc(f, n);
-#pragma unroll
-    for (int c = 0; c < NV; ++c) {
-      Uo[c] = U[(long long)c * Nd + io];
-      Lw[c] = 0.0;
-    }
-    if (!ghost) {
-      // the element across the line (across the wrap on a periodic axis)
-      const long long eo = dir == 0 ? (long long)ey * Nx + wrapO : (long long)wrapO * Nx + ex;
-      const long long ioth = eo * NPP + face_loc(f ^ 1, n);
-      const double* cw = va.coef + ((eo * 4 + (f ^ 1)) * NP + n) * 6;
-#pragma unroll
-      for (int c = 0; c < NV; ++c) {
-        Uw[c] = U[(long long)c * Nd + ioth];
-        Lw[c] = cw[c];
-      }
-      lw = cw[NV];
-    } else if (!wall) {
-      const double* cf = g.inflow + ((long long)ey * NP + n) * (NV * 3);
-#pragma unroll
-      for (int c = 0; c < NV; ++c) Uw[c] = (cf[3 * c] + cf[3 * c + 1] * gt.s) + cf[3 * c + 2] * gt.c;
-    }
-#pragma unroll
-    for (int ps = 0; ps < 2; ++ps) {
-      if (ps < passes) {
-        const int line = ps == 0 ? pos + (ownHigh ? 0 : 1) : (ownHigh ? nL : 0);
-        hfp[ps] = dir == 0 ? g.HfX[((long long)ey * (Nx + 1) + line) * NP + n]
-                           : g.HfY[((long long)line * Nx + ex) * NP + n];
-      }
-    }
-  }
-  tile_stage(va, g, ph, L, t, isNode, i, sH);
-  __syncthreads();
-
-  // phase 2: face nodes (20 per element): the interface lines each edge
-  // state feeds, their adjoint kept for the own side. A y line is handled in
-  // the x frame: with P the exchange of hu and hv, flux_y(U) = P flux_x(P U)
-  // and the y wave speed is the x one of P U, so its adjoint is P applied to
-  // the x adjoint of the exchanged states and cotangents.
-  if (isFace) {
-    double Lo[NV], lo;
-    face_coef(L, NPP * jf, f, n, iJx, iJy, Lo, lo);
-    if (wall) {
-#pragma unroll
-      for (int c = 0; c < NV; ++c) Uw[c] = Uo[c];
-      Uw[dir == 0 ? IHU : IHV] = -Uo[dir == 0 ? IHU : IHV];
-    }
-    auto to_x = [&](double* x) {
-      if (dir == 1) {
-        const double tmp = x[IHU];
-        x[IHU] = x[IHV];
-        x[IHV] = tmp;
-      }
-    };
-    to_x(Uo);
-    to_x(Lo);
-    to_x(Uw);
-    to_x(Lw);
-    double Ub[NV] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    double tf = 0.0;
-    for (int ps = 0; ps < passes; ++ps) {
-      const double hf = ps == 0 ? hfp[0] : hfp[1];
-      const bool ownIn = ps == 0, othIn = ps == 1 || inLine;
-      double UL[NV], UR[NV], LL[NV], LR[NV], UbL[NV], UbR[NV];
-#pragma unroll
-      for (int c = 0; c < NV; ++c) {
-        const double lo_c = ownIn ? Lo[c] : 0.0, lw_c = othIn ? Lw[c] : 0.0;
-        UL[c] = ownHigh ? Uw[c] : Uo[c];
-        UR[c] = ownHigh ? Uo[c] : Uw[c];
-        LL[c] = ownHigh ? lw_c : lo_c;
-        LR[c] = ownHigh ? lo_c : lw_c;
-      }
-      const double lh = (ownIn ? lo : 0.0) + (othIn ? lw : 0.0);
-      const double hfb = line_bar<0>(UL, UR, hf, LL, LR, lh, ph, UbL, UbR);
-#pragma unroll
-      for (int c = 0; c < NV; ++c) {
-        const double own = ownHigh ? UbR[c] : UbL[c], oth = ownHigh ? UbL[c] : UbR[c];
-        // a wall ghost is the own state with the normal momentum negated
-        Ub[c] += wall ? (c == IHU ? own - oth : own + oth) : own;
-      }
-      // face depth: the mean of two edge values, or the one interior value
-      // on a non-periodic side
-      tf += ghost ? hfb : 0.5 * hfb;
-      if (ps == 0) sHS[t] = 0.5 * (UL[IH] + UR[IH]);
-    }
-    to_x(Ub);
-#pragma unroll
-    for (int c = 0; c < NV; ++c) sUF[c][t] = Ub[c];
-    sLam[t] = lo;
-    sTF[t] = tf;
-  }
-  __syncthreads();
-
-  // the node's own operands of phase 3, loaded after the face phase (h, hu,
-  // hv are lines tile_stage has just read), which keeps them out of the
-  // registers live across it: 0.7 % faster than loading them in phase 1
-  double Un[NV], Hl = 0.0, Hxl = 0.0, Hyl = 0.0;
-  if (isNode) {
-#pragma unroll
-    for (int c = 0; c < NV; ++c) Un[c] = U[(long long)c * Nd + i];
-    Hl = g.Hnod[i];
-    Hxl = g.Hx[i];
-    Hyl = g.Hy[i];
-  }
-  // phase 3: node adjoint
-  const int jb = NPP * j, fb = 20 * j;
-  double Hxb = 0.0, Hyb = 0.0, th = 0.0;
-  double outv[NV] = {0.0, 0.0, 0.0, 0.0, 0.0};   // the node's result, for the next product
-  if (isNode) {
-    double dhx = 0.0, dhy = 0.0;
-    // rolled, like the D^T loop below: unrolled, the compiler hoists its LDS
-    // operands into 20 more VGPRs, which keeps the kernel off four waves
-#pragma unroll 1
-    for (int k = 0; k < NP; ++k) {
-      dhx = dhx + sD[a * NP + k] * sH[jb + k + NP * b];
-      dhy = dhy + sD[b * NP + k] * sH[jb + a + NP * k];
-    }
-    dhx = dhx + ((sHS[fb + b] - sH[jb + NP * b]) * sgL[a] +
-                 (sHS[fb + NP + b] - sH[jb + NP - 1 + NP * b]) * sgR[a]);
-    dhy = dhy + ((sHS[fb + 2 * NP + a] - sH[jb + a]) * sgL[b] +
-                 (sHS[fb + 3 * NP + a] - sH[jb + a + NP * (NP - 1)]) * sgR[b]);
-    const double hx = dhx * iJx, hy = dhy * iJy;
-    double Ub[NV] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    double Hlb, Wn[NV];
-#pragma unroll
-    for (int c = 0; c < NV; ++c) Wn[c] = L.W[c][t];
-    const St sn = make_st(Un);
-    PrimBar qn{0.0, 0.0, 0.0, 0.0};
-    node_terms_acc(sn, Hl, Hxl, Hyl, hx, hy, ph, Wn, Ub, qn, Hlb, Hxb, Hyb);
-    // the nodal flux cotangents: D^T applied along the row (x) and the column
-    // (y) to the cotangents -W/Jx, -W/Jy of the two D-sums. The k loop stays
-    // rolled so that only one k's ten LDS operands are live at a time.
-    double Fb[NV] = {0.0, 0.0, 0.0, 0.0, 0.0}, Gb[NV] = {0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma unroll 1
-    for (int k = 0; k < NP; ++k) {
-      const double dxk = sD[k * NP + a], dyk = sD[k * NP + b];
-      const int nx = jb + k + NP * b, ny = jb + a + NP * k;
-#pragma unroll
-      for (int c = 0; c < NV; ++c) {
-        Fb[c] = Fb[c] + dxk * L.W[c][nx];
-        Gb[c] = Gb[c] + dyk * L.W[c][ny];
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < NV; ++c) {
-      Fb[c] = -Fb[c] * iJx;
-      Gb[c] = -Gb[c] * iJy;
-    }
-    Hlb += flux_acc<0>(sn, Hl, ph, Fb, Ub, qn);
-    Hlb += flux_acc<1>(sn, Hl, ph, Gb, Ub, qn);
-    prims_fin(sn, qn, Ub);
-    double hb = 0.0;
-#pragma unroll
-    for (int k = 0; k < NP; ++k)
-      hb = hb + (sD[k * NP + a] * L.DX[jb + k + NP * b] + sD[k * NP + b] * L.DY[jb + a + NP * k]);
-    if (a == 0) hb -= sLam[fb + b];
-    if (a == NP - 1) hb -= sLam[fb + NP + b];
-    if (b == 0) hb -= sLam[fb + 2 * NP + a];
-    if (b == NP - 1) hb -= sLam[fb + 3 * NP + a];
-    Ub[IH] += hb;
-    double tb = 0.0;
-    auto face_add = [&](int slot) {
-#pragma unroll
-      for (int c = 0; c < NV; ++c) Ub[c] += sUF[c][slot];
-      tb += sTF[slot];
-    };
-    if (a == 0) face_add(fb + b);
-    if (a == NP - 1) face_add(fb + NP + b);
-    if (b == 0) face_add(fb + 2 * NP + a);
-    if (b == NP - 1) face_add(fb + 3 * NP + a);
-#pragma unroll
-    for (int c = 0; c < NV; ++c) {
-      const long long o = (long long)c * Nd + i;
-      double base = 0.0;
-      if (va.acc0) base = va.acc0[o];
-      if (va.acc1) base = base + va.acc1[o];
-      if (va.acc2) base = base + va.acc2[o];
-      outv[c] = base + Ub[c];
-      va.out[o] = outv[c];
-    }
-    th = Hlb + tb;
-  }
-  if (va.thetaBar) {   // uniform over the block
-    // still depth: Hnod = theta, Hx = (D theta)/Jx, Hy = (D theta)/Jy per line
-    __syncthreads();
-    if (isNode) {
-      L.DX[t] = Hxb * iJx;
-      L.DY[t] = Hyb * iJy;
-    }
-    __syncthreads();
-    if (isNode) {
-#pragma unroll
-      for (int k = 0; k < NP; ++k)
-        th = th + (sD[k * NP + a] * L.DX[jb + k + NP * b] + sD[k * NP + b] * L.DY[jb + a + NP * k]);
-      va.thetaBar[i] += th;
-    }
-  }
-  if (va.coefNext) {   // uniform over the block
-    // the next product's cotangent can*An + cbn*out on this tile, staged as
-    // tile_stage stages a product's own, then its face coefficients as
-    // vjp_coef_tile forms them
-    __syncthreads();
-    if (isNode) {
-      double Wn[NV];
-#pragma unroll
-      for (int c = 0; c < NV; ++c) {
-        Wn[c] = va.can * va.An[(long long)c * Nd + i];
-        Wn[c] = Wn[c] + va.cbn * outv[c];
-        L.W[c][t] = Wn[c];
-      }
-      const double q = Wn[IHP] * ph.c2 / va.Un[i];
-      L.DX[t] = q * va.Un[(long long)IHU * Nd + i] * (1.0 / g.Jx);
-      L.DY[t] = q * va.Un[(long long)IHV * Nd + i] * (1.0 / g.Jy);
-    }
-    __syncthreads();
-    if (isFace) {
-      double Ln[NV], ln;
-      face_coef(L, NPP * jf, f, n, iJx, iJy, Ln, ln);
-      double* cp = va.coefNext + (((long long)ey * Nx + ex0) * 20 + t) * 6;
-#pragma unroll
-      for (int c = 0; c < NV; ++c) cp[c] = Ln[c];
-      cp[NV] = ln;
-    }
-  }
+// The arguments are the kernel's only parameter, read where they lie.
+template <int NOP>
+__global__ void __launch_bounds__(kVT, 3) k_vjp_sweep(VjpMember) {
+  vjp_tile<NOP>((ConstArgs<VjpMember>)__builtin_amdgcn_kernarg_segment_ptr(),
+                     xcd_tile(blockIdx.x, gridDim.x));
 }
 
-__global__ void __launch_bounds__(kVT)
-k_vjp_coef(VjpArgs va, Geometry g, Phys ph) {
-  vjp_coef_tile(va, g, ph, blockIdx.x);
-}
-
-// four waves per SIMD (at most 128 VGPRs; 3 spilled, 12 B of scratch per
-// lane): 5.6 % faster per product and 8.7 % per reversed step than three
-// waves (134 VGPRs), same bits
-__global__ void __launch_bounds__(kVT, 4)
-k_vjp_elem(VjpArgs va, Geometry g, Phys ph, GhostTime gt) {
-  vjp_elem_tile(va, g, ph, gt, blockIdx.x);
-}
-
-// ---- batches: every member's tiles packed into one launch -------------------------
-// the member owning packed tile w: tileStart[m] <= w < tileStart[m + 1]
-__device__ __forceinline__ int member_of(const long long* tileStart, int nMem, long long w) {
+// every member's tiles packed into one launch: the member owning packed tile
+// w has tileStart[m] <= w < tileStart[m + 1]
+template <int NOP>
+__global__ void __launch_bounds__(kVT, 3)
+k_vjp_sweep_batch(const VjpMember* __restrict__ mem, const long long* __restrict__ tileStart,
+                  int nMem) {
+  const long long w = xcd_tile(blockIdx.x, gridDim.x);
   int lo = 0, hi = nMem - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (tileStart[mid] <= w) lo = mid;
     else hi = mid - 1;
   }
-  return lo;
-}
-
-__global__ void __launch_bounds__(kVT)
-k_vjp_coef_batch(const VjpMember* __restrict__ mem, const long long* __restrict__ tileStart,
-                 int nMem) {
-  const long long w = blockIdx.x;
-  const int m = member_of(tileStart, nMem, w);
-  vjp_coef_tile(mem[m].va, mem[m].g, mem[m].ph, (int)(w - tileStart[m]));
-}
-
-__global__ void __launch_bounds__(kVT, 4)
-k_vjp_elem_batch(const VjpMember* __restrict__ mem, const long long* __restrict__ tileStart,
-                 int nMem) {
-  const long long w = blockIdx.x;
-  const int m = member_of(tileStart, nMem, w);
-  vjp_elem_tile(mem[m].va, mem[m].g, mem[m].ph, mem[m].gt, (int)(w - tileStart[m]));
+  const int tile = __builtin_amdgcn_readfirstlane((int)(w - tileStart[lo]));
+  const ConstArgs<VjpMember> M = const_entry(mem, lo);
+  if (tile >= M->nTiles) return;   // (a grid larger than the members' tiles is never launched)
+  vjp_tile<NOP>(M, tile);
 }
 
 // lam[node] += Gb[k], thetaBar[node] -= Gb[k] for the n gauges of one log row,
@@ -660,31 +693,78 @@ __global__ void k_gauge_bar(const double* __restrict__ Gb, const long long* __re
 
 }  // namespace
 
+namespace {
+int vjp_strips(const Geometry& g) { return (g.Nx + kEW - 1) / kEW; }
+// which build a product takes: its operands
+int vjp_nop(const VjpArgs& va) { return va.acc ? 3 : va.B ? 2 : 1; }
+}  // namespace
+
+long long vjp_tiles(const Geometry& g) {
+  return (long long)vjp_strips(g) * ((g.Ny + g.vrows - 1) / g.vrows);
+}
+
+long long vjp_row_tiles(const Geometry& g) { return (long long)vjp_strips(g) * g.Ny; }
+
+// A workgroup's time is that of its rows and the two staged beside them, the
+// launch's that of its fullest compute units. Per row a lone workgroup on a
+// unit takes 2.8 us, two, three and four together 3.6, 4.5 and 5.3 (a unit
+// holds four): in the ratio of 5 + 2 x for x workgroups, which is what the
+// heights are compared by, over the sets of four that the launch runs through.
+//   products of a step, us      rows: 2    4    7   10   16   32
+//    128 x   64                     74   71   85  105
+//    256 x  128                    207  183  167  169  203
+//   1024 x  512                   3070 2464 2254 2176 2085 2053
+int vjp_rows(const Geometry* const* g, int n, int cus) {
+  const long long units = std::max(cus, 1);
+  long long best = 0;
+  int rows = 1;
+  for (int r = 1; r <= 32; ++r) {
+    long long tiles = 0;
+    for (int i = 0; i < n; ++i) tiles += (long long)vjp_strips(*g[i]) * ((g[i]->Ny + r - 1) / r);
+    const long long sets = tiles / (4 * units), rest = tiles % (4 * units);
+    const long long cost = (r + 2) * (13 * sets + (rest ? 5 + 2 * ((rest + units - 1) / units) : 0));
+    if (r == 1 || cost < best) {
+      best = cost;
+      rows = r;
+    }
+  }
+  return rows;
+}
+
+VjpMember vjp_member(const Geometry& g, const Phys& ph, const VjpArgs& va, GhostTime gt) {
+  return VjpMember{va, g, ph, gt, vjp_strips(g), (int)vjp_tiles(g)};
+}
+
 hipError_t launch_rhs_vjp(const Geometry& g, const Phys& ph, const VjpArgs& va, GhostTime gt,
                           hipStream_t st) {
-  const long long nb = (long long)g.Ny * ((g.Nx + kEW - 1) / kEW);
-  if (!va.coefReady) {
-    hipLaunchKernelGGL(k_vjp_coef, dim3((unsigned)nb), dim3(kVT), 0, st, va, g, ph);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+  const long long nb = vjp_tiles(g);
+  if (nb > 0x7fffffffLL || va.out == va.A || va.out == va.B || (va.acc && !va.B))
+    return hipErrorInvalidValue;
+  const VjpMember m = vjp_member(g, ph, va, gt);
+  const dim3 grid((unsigned)nb), block(kVT);
+#define SGNX_VJP(N) hipLaunchKernelGGL(k_vjp_sweep<N>, grid, block, 0, st, m)
+  switch (vjp_nop(va)) {
+    case 1: SGNX_VJP(1); break;
+    case 2: SGNX_VJP(2); break;
+    default: SGNX_VJP(3);
   }
-  hipLaunchKernelGGL(k_vjp_elem, dim3((unsigned)nb), dim3(kVT), 0, st, va, g, ph, gt);
+#undef SGNX_VJP
   return hipGetLastError();
 }
 
-long long vjp_tiles(const Geometry& g) { return (long long)g.Ny * ((g.Nx + kEW - 1) / kEW); }
-
 hipError_t launch_rhs_vjp_batch(const VjpMember* mem, const long long* tileStart, int nMem,
-                                long long totalTiles, bool coefReady, hipStream_t st) {
+                                long long totalTiles, int nop, hipStream_t st) {
   if (totalTiles <= 0) return hipSuccess;
-  if (!coefReady) {
-    hipLaunchKernelGGL(k_vjp_coef_batch, dim3((unsigned)totalTiles), dim3(kVT), 0, st, mem,
-                       tileStart, nMem);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+  if (totalTiles > 0x7fffffffLL || nop < 1 || nop > 3) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)totalTiles), block(kVT);
+#define SGNX_VJP(N) \
+  hipLaunchKernelGGL(k_vjp_sweep_batch<N>, grid, block, 0, st, mem, tileStart, nMem)
+  switch (nop) {
+    case 1: SGNX_VJP(1); break;
+    case 2: SGNX_VJP(2); break;
+    default: SGNX_VJP(3);
   }
-  hipLaunchKernelGGL(k_vjp_elem_batch, dim3((unsigned)totalTiles), dim3(kVT), 0, st, mem,
-                     tileStart, nMem);
+#undef SGNX_VJP
   return hipGetLastError();
 }
 

@@ -36,14 +36,11 @@
 
 #include "sgnx_tape.h"
 
-void chain_coef(VjpArgs& a, VjpArgs& b, double* buf) {
-  a.coefNext = buf;
-  a.Un = b.U;
-  a.An = b.A;
-  a.can = b.ca;
-  a.cbn = b.cb;
-  b.coef = buf;
-  b.coefReady = true;
+void step_products(AdjTape* tp, const double* u, const double* y2, const double* y3, double dt,
+                   double* thetaBar, VjpArgs p[3]) {
+  p[0] = VjpArgs{y3, tp->lam, dt * (4.0 / 9.0), nullptr, 0.0, nullptr, tp->y3b, thetaBar};
+  p[1] = VjpArgs{y2, tp->lam, dt * (1.0 / 3.0), tp->y3b, 0.75 * dt, nullptr, tp->y2b, thetaBar};
+  p[2] = VjpArgs{u, tp->lam, dt * (2.0 / 9.0), tp->y2b, 0.5 * dt, tp->y3b, tp->lamNew, thetaBar};
 }
 
 namespace {
@@ -77,20 +74,6 @@ int check_adjoint_support(sgnx_solver* s) {
 int vjp(sgnx_solver* s, const VjpArgs& va, double t) {
   HIPCHK(s, launch_rhs_vjp(s->g, s->ph, va, ghost_time(s, t), s->stream));
   return SGNX_OK;
-}
-
-VjpArgs vjp_args(AdjTape* tp, const double* U, const double* A, double ca, const double* B,
-                 double cb, double* out, double* thetaBar) {
-  VjpArgs va{};
-  va.U = U;
-  va.A = A;
-  va.ca = ca;
-  va.B = B;
-  va.cb = cb;
-  va.out = out;
-  va.thetaBar = thetaBar;
-  va.coef = tp->coef;
-  return va;
 }
 
 // u -> uNew by one BS3 step of size dt with the forward's kernels (fused stage
@@ -127,24 +110,18 @@ int bs3_fixed(sgnx_solver* s, const double* u, double* uNew, double t, double dt
 }
 
 // lam <- (d u_{n+1} / d u_n)^T lam for the step u -> u_{n+1} of size dt at t,
-// whose stage inputs are y2, y3; thetaBar += the still-depth part. The three
-// products are chained: each of the first two also writes the next one's face
-// coefficients (tp->coef2, then tp->coef).
+// whose stage inputs are y2, y3; thetaBar += the still-depth part.
 //   uNew = u + dt ((2/9 k1 + 1/3 k2) + 4/9 k3)   (rk.cpp:106-108)
 int step_adjoint_stored(sgnx_solver* s, AdjTape* tp, const double* u, const double* y2,
                         const double* y3, double t, double dt, double* thetaBar) {
   int rc;
-  VjpArgs a3 = vjp_args(tp, y3, tp->lam, dt * (4.0 / 9.0), nullptr, 0.0, tp->y3b, thetaBar);
-  VjpArgs a2 = vjp_args(tp, y2, tp->lam, dt * (1.0 / 3.0), tp->y3b, 0.75 * dt, tp->y2b, thetaBar);
-  VjpArgs a1 = vjp_args(tp, u, tp->lam, dt * (2.0 / 9.0), tp->y2b, 0.5 * dt, tp->lam, thetaBar);
-  a1.acc0 = tp->lam;
-  a1.acc1 = tp->y3b;
-  a1.acc2 = tp->y2b;
-  chain_coef(a3, a2, tp->coef2);
-  chain_coef(a2, a1, tp->coef);
-  if ((rc = vjp(s, a3, t + 0.75 * dt))) return rc;
-  if ((rc = vjp(s, a2, t + 0.5 * dt))) return rc;
-  return vjp(s, a1, t);
+  VjpArgs p[3];
+  step_products(tp, u, y2, y3, dt, thetaBar, p);
+  if ((rc = vjp(s, p[0], t + 0.75 * dt))) return rc;
+  if ((rc = vjp(s, p[1], t + 0.5 * dt))) return rc;
+  if ((rc = vjp(s, p[2], t))) return rc;
+  std::swap(tp->lam, tp->lamNew);
+  return SGNX_OK;
 }
 
 // step_adjoint_stored with the stage inputs recomputed from u.
@@ -177,8 +154,6 @@ int step_adjoint(sgnx_solver* s, AdjTape* tp, const double* u, double t, double 
 
 int ensure_vjp_buffers(sgnx_solver* s, AdjTape* tp) {
   int rc;
-  if ((rc = alloc_state(s, &tp->coef, (size_t)vjp_coef_doubles(s->g)))) return rc;
-  if ((rc = alloc_state(s, &tp->coef2, (size_t)vjp_coef_doubles(s->g)))) return rc;
   if ((rc = alloc_state(s, &tp->thb, (size_t)s->g.Nd))) return rc;
   return SGNX_OK;
 }
@@ -379,7 +354,7 @@ int adjoint_begin(sgnx_solver* s, bool storeAll, AdjTape** out) {
     return fail(s, SGNX_EINVAL,
                 "adjoint: a batched sweep needs every step's snapshot (max_snapshots >= steps)");
   if ((rc = ensure_vjp_buffers(s, tp))) return rc;
-  for (double** p : {&tp->lam, &tp->y3b, &tp->y2b})
+  for (double** p : {&tp->lam, &tp->lamNew, &tp->y3b, &tp->y2b})
     if ((rc = alloc_state(s, p, s->n()))) return rc;
   *out = tp;
   return SGNX_OK;
@@ -514,7 +489,7 @@ void tape_free(sgnx_solver* s) {
   release_stages(tp);
   for (double* p : tp->spare) (void)hipFree(p);
   for (double* p : tp->seg) (void)hipFree(p);
-  for (double* p : {tp->lam, tp->y3b, tp->y2b, tp->coef, tp->coef2, tp->thb, tp->gb, tp->pp[0],
+  for (double* p : {tp->lam, tp->lamNew, tp->y3b, tp->y2b, tp->thb, tp->gb, tp->pp[0],
                     tp->pp[1]})
     if (p) (void)hipFree(p);
   delete tp;
@@ -566,7 +541,7 @@ int sgnx_rhs_vjp(sgnx_solver* s, const double* U, const double* W, double* Ubar,
     return fail(s, SGNX_EINVAL, "rhs_vjp: Ubar must not overlap U or W");
   }
   if (dTh) HIPCHK(s, hipMemsetAsync(dTh, 0, Nd * sizeof(double), s->stream));
-  VjpArgs va = vjp_args(tp, dU, dW, 1.0, nullptr, 0.0, dOut, dTh);
+  const VjpArgs va{dU, dW, 1.0, nullptr, 0.0, nullptr, dOut, dTh};
   if ((rc = vjp(s, va, t))) return rc;
   if (mem == SGNX_MEM_HOST) {
     HIPCHK(s, hipMemcpyAsync(Ubar, dOut, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));

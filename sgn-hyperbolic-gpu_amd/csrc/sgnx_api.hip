@@ -27,6 +27,7 @@
 #include <string>
 #include <vector>
 
+#include "sgnx_adjoint.h"
 #include "sgnx_handle.h"
 
 // Scratch of sgnx_gauges_noalloc: the node list (SGNX_GAUGES_NOALLOC_MAX
@@ -216,6 +217,7 @@ int sgnx_create(const sgnx_desc* d, sgnx_solver** out) {
 
   CK(hipGetDevice(&s->device));
   CK(scratch_address(s->device, &s->scratch));
+  g.vrows = g.rows;
   if (!std::getenv("SGNX_SWEEP_ROWS")) {
     // default tile height: the tallest that still gives every compute unit
     // about three workgroups (small grids would leave most of the chip idle
@@ -228,6 +230,8 @@ int sgnx_create(const sgnx_desc* d, sgnx_solver** out) {
       g.rows = r;
       if (strips * ((d->Ny + r - 1) / r) >= want) break;
     }
+    const Geometry* const one = &g;
+    g.vrows = vjp_rows(&one, 1, cus);   // (the products do not depend on it)
   }
   const size_t Nd = (size_t)g.Nd, nst = (size_t)NV * Nd;
   const size_t nfx = (size_t)(d->Nx + 1) * d->Ny * NP, nfy = (size_t)d->Nx * (d->Ny + 1) * NP;

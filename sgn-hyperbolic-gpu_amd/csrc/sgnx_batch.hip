@@ -546,7 +546,7 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
   int cus = 0;
   BCHK(b, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
   bool each_fills = n > 0;
-  for (int i = 0; i < n; ++i) each_fills = each_fills && vjp_tiles(b->m[i]->g) >= 6LL * cus;
+  for (int i = 0; i < n; ++i) each_fills = each_fills && vjp_row_tiles(b->m[i]->g) >= 6LL * cus;
   if (each_fills) {
     for (int i = 0; i < n; ++i) {
       sgnx_solver* s = b->m[i];
@@ -561,6 +561,10 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
     }
     return SGNX_OK;
   }
+  // one tile height for all members' products, unless set from outside
+  std::vector<const Geometry*> gs;
+  for (int i = 0; i < n; ++i) gs.push_back(&b->m[i]->g);
+  const int vrows = std::getenv("SGNX_SWEEP_ROWS") ? 0 : vjp_rows(gs.data(), n, cus);
   std::vector<AdjTape*> tp(n, nullptr);
   std::vector<const double*> gb(n, nullptr);
   long Nmax = 0;
@@ -645,36 +649,16 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
         rAcc += sweep_tiles(s->g);
         ++Rn;
       }
-      // uNew = u + dt ((2/9 k1 + 1/3 k2) + 4/9 k3)   (rk.cpp:106-108)
-      VjpArgs a3{};
-      a3.U = y3;
-      a3.A = T->lam;
-      a3.ca = dt * (4.0 / 9.0);
-      a3.out = T->y3b;
-      a3.thetaBar = T->thb;
-      a3.coef = T->coef;
-      VjpArgs a2 = a3;
-      a2.U = y2;
-      a2.ca = dt * (1.0 / 3.0);
-      a2.B = T->y3b;
-      a2.cb = 0.75 * dt;
-      a2.out = T->y2b;
-      VjpArgs a1 = a3;
-      a1.U = u;
-      a1.ca = dt * (2.0 / 9.0);
-      a1.B = T->y2b;
-      a1.cb = 0.5 * dt;
-      a1.out = T->lam;
-      a1.acc0 = T->lam;
-      a1.acc1 = T->y3b;
-      a1.acc2 = T->y2b;
-      chain_coef(a3, a2, T->coef2);
-      chain_coef(a2, a1, T->coef);
-      hV3[A] = VjpMember{a3, s->g, s->ph, ghost_time(s, t + 0.75 * dt)};
-      hV2[A] = VjpMember{a2, s->g, s->ph, ghost_time(s, t + 0.5 * dt)};
-      hV1[A] = VjpMember{a1, s->g, s->ph, ghost_time(s, t)};
+      VjpArgs p[3];
+      step_products(T, u, y2, y3, dt, T->thb, p);
+      Geometry vg = s->g;
+      if (vrows) vg.vrows = vrows;
+      hV3[A] = vjp_member(vg, s->ph, p[0], ghost_time(s, t + 0.75 * dt));
+      hV2[A] = vjp_member(vg, s->ph, p[1], ghost_time(s, t + 0.5 * dt));
+      hV1[A] = vjp_member(vg, s->ph, p[2], ghost_time(s, t));
+      std::swap(T->lam, T->lamNew);   // (the tables hold this step's; the next reads its result)
       hVT[A] = vAcc;
-      vAcc += vjp_tiles(s->g);
+      vAcc += vjp_tiles(vg);
       ++A;
     }
     hRT[Rn] = rAcc;
@@ -691,11 +675,10 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
       BCHK(b, launch_rhs_stage_batch(dR2, dRT, Rn, rAcc, kAxpy, (b->waves3 >> 1) & 1, b->stream,
                                      true, batch_hxr(b)));
     }
-    // the products chained: the first launches the coefficient kernel, each
-    // later one finds its coefficients written by the one before
+    int nop = 0;
     for (size_t o : {oV3, oV2, oV1})
       BCHK(b, launch_rhs_vjp_batch(reinterpret_cast<const VjpMember*>(dptr(o)), dVT, A, vAcc,
-                                   o != oV3, b->stream));
+                                   ++nop, b->stream));
     // the arena is refilled for the next iteration
     BCHK(b, hipStreamSynchronize(b->stream));
   }

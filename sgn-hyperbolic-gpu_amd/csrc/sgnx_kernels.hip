@@ -27,6 +27,7 @@
 // file is compiled with -ffp-contract=off.
 // =============================================================================
 
+#include "sgnx_device.h"
 #include "sgnx_internal.h"
 
 namespace sgnx {
@@ -361,45 +362,8 @@ struct NodeExtra {
   double x0[(MODE == kCand || MODE == kErr) ? NV : 1], x1[MODE == kErr ? NV : 1];
 };
 
-// Global operands are addressed as a wave-uniform base (scalar registers and
-// scalar adds) plus a 32-bit byte offset of the lane, so that no vector
-// instruction forms an address. Variable v of an operand lies v planes of
-// `plane` bytes above its base; the planes are stepped to one after another,
-// which needs one scalar pair per operand instead of five.
-typedef __attribute__((address_space(1))) char GlobalByte;
-typedef __attribute__((address_space(1))) double GlobalDouble;
-typedef __attribute__((address_space(3))) double LdsDouble;
-__device__ __forceinline__ GlobalByte* global_at(const double* base, size_t first) {
-  GlobalByte* p = (GlobalByte*)base + first;
-  __asm__ volatile("" : "+s"(p));   // formed by scalar instructions, before the lane's part
-  return p;
-}
-__device__ __forceinline__ double load_at(const GlobalByte* base, unsigned off) {
-  return *(const GlobalDouble*)(base + off);
-}
-__device__ __forceinline__ void store_at(GlobalByte* base, unsigned off, double x) {
-  *(GlobalDouble*)(base + off) = x;
-}
-__device__ __forceinline__ void load_vars(const double* base, size_t first, size_t plane,
-                                          unsigned off, double* W) {
-  const GlobalByte* p = global_at(base, first);
-#pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    W[v] = load_at(p, off);
-    p += plane;
-  }
-}
-
-// The launch's arguments in constant memory (kernel arguments, or one entry
-// of a batch's table), read by scalar loads. What a phase needs once per row
-// is read there again, through a pointer made opaque in that row: all of it
-// kept across rows exceeds the scalar registers, and the excess would travel
-// through vector lanes.
-typedef const BatchMember __attribute__((address_space(4))) * SweepArgs;
-__device__ __forceinline__ SweepArgs opaque(SweepArgs A) {
-  __asm__ volatile("" : "+s"(A));
-  return A;
-}
+// The launch's arguments: its kernel's own, or one entry of a batch's table.
+typedef ConstArgs<BatchMember> SweepArgs;
 
 template <int MODE>
 __device__ __forceinline__ void stage_load(SweepArgs A, size_t first, size_t plane, unsigned off,
@@ -433,24 +397,6 @@ __device__ __forceinline__ void stage_combine_face(const StageRaw<MODE>& R, doub
   for (int v = 0; v < NV; ++v) W[v] = W[v] + 0.0;
 }
 
-// The other lane's value within each pair of lanes (DPP quad_perm [1,0,3,2]).
-__device__ __forceinline__ double lane_swap(double x) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0xB1, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0xB1, 0xF, 0xF, true);
-  return __hiloint2double(hi, lo);
-}
-
-// barrier that instructions of the two phases do not cross in either direction
-// (arithmetic hoisted over it only lengthens registers' lives)
-__device__ __forceinline__ void row_sync() {
-  __builtin_amdgcn_sched_barrier(0);
-  __syncthreads();
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// whether the condition holds on some active lane of the wave
-__device__ __forceinline__ bool wave_any(int c) { return __builtin_amdgcn_ballot_w64(c != 0) != 0; }
-
 // The primitives of prims() by one refined reciprocal of h for the four
 // quotients where h and the four dividends are in the range of DivBy; else, on
 // some lane of the wave, by IEEE division for the wave. Same bits.
@@ -468,23 +414,6 @@ __device__ __forceinline__ Prim prims_shared(const double* U) {
   if (__builtin_expect(wave_any(bad), 0)) q = prims(U);
   return q;
 }
-
-// y = x as a move at this place
-__device__ __forceinline__ void move_to(double& y, double x) {
-  __asm__ volatile("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
-}
-
-// x with its sign bit changed where mask = 0x80000000 (0: unchanged)
-__device__ __forceinline__ double flip_sign(double x, int mask) {
-  return __hiloint2double(__double2hiint(x) ^ mask, __double2loint(x));
-}
-
-__device__ __forceinline__ unsigned node_of(int Nx, int ex, int ey, int a, int b) {
-  return ((unsigned)ey * (unsigned)Nx + (unsigned)ex) * NPP + a + NP * b;
-}
-
-template <int V>
-struct IntC { static constexpr int value = V; };
 
 // LDS of one workgroup. A node's record holds h, hu, hv, hw, hp, the fluxes
 // F[1..4] and G[1..4] (F[0] is hu and G[0] is hv) and, with HXR, the still
@@ -982,11 +911,7 @@ k_rhs_sweep_batch(const BatchMember* __restrict__ mem, const long long* __restri
     const int mid = (lo + hi + 1) >> 1;
     if (tileStart[mid] <= w) lo = mid; else hi = mid - 1;
   }
-  lo = __builtin_amdgcn_readfirstlane(lo);
-  const size_t at = reinterpret_cast<size_t>(mem + lo);
-  const SweepArgs M = reinterpret_cast<SweepArgs>(
-      (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)at) |
-      (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32);
+  const SweepArgs M = const_entry(mem, lo);
   const int tile = __builtin_amdgcn_readfirstlane((int)(w - tileStart[lo]));
   // a grid larger than the members' tiles (never launched so) does nothing
   if (tile >= M->nTiles) return;
