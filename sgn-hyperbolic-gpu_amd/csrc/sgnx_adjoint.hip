@@ -600,23 +600,23 @@ __global__ void __launch_bounds__(kVT, 3) k_vjp_sweep(VjpMember) {
                      xcd_tile(blockIdx.x, gridDim.x));
 }
 
-// every member's tiles packed into one launch: the member owning packed tile
-// w has tileStart[m] <= w < tileStart[m + 1]
+// every member's tiles in one launch: the member of workgroup w has
+// tileStart[m] <= w < tileStart[m + 1], multiples of the XCDs' number
 template <int NOP>
 __global__ void __launch_bounds__(kVT, 3)
 k_vjp_sweep_batch(const VjpMember* __restrict__ mem, const long long* __restrict__ tileStart,
                   int nMem) {
-  const long long w = xcd_tile(blockIdx.x, gridDim.x);
+  const long long w = blockIdx.x;
   int lo = 0, hi = nMem - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (tileStart[mid] <= w) lo = mid;
     else hi = mid - 1;
   }
-  const int tile = __builtin_amdgcn_readfirstlane((int)(w - tileStart[lo]));
+  const int own = __builtin_amdgcn_readfirstlane((int)(w - tileStart[lo]));
   const ConstArgs<VjpMember> M = const_entry(mem, lo);
-  if (tile >= M->nTiles) return;   // (a grid larger than the members' tiles is never launched)
-  vjp_tile<NOP>(M, tile);
+  if (own >= M->nTiles) return;   // (filling up)
+  vjp_tile<NOP>(M, xcd_tile(own, M->nTiles));
 }
 
 // lam[node] += Gb[k], thetaBar[node] -= Gb[k] for the n gauges of one log row,

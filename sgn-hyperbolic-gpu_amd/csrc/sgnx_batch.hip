@@ -108,7 +108,7 @@ long long fill_offsets(sgnx_batch* b, const std::vector<int>& set) {
   long long acc = 0;
   for (size_t i = 0; i < set.size(); ++i) {
     b->h_ts[i] = acc;
-    acc += sweep_tiles(b->m[set[i]]->g);
+    acc += packed_tiles(sweep_tiles(b->m[set[i]]->g));
   }
   b->h_ts[set.size()] = acc;
   return acc;
@@ -646,7 +646,7 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
         s2.a3 = 0.75 * dt;
         hR2[Rn] = member_args(s, u, s->d_k2, s2, t + 0.5 * dt);
         hRT[Rn] = rAcc;
-        rAcc += sweep_tiles(s->g);
+        rAcc += packed_tiles(sweep_tiles(s->g));
         ++Rn;
       }
       VjpArgs p[3];
@@ -658,7 +658,7 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
       hV1[A] = vjp_member(vg, s->ph, p[2], ghost_time(s, t));
       std::swap(T->lam, T->lamNew);   // (the tables hold this step's; the next reads its result)
       hVT[A] = vAcc;
-      vAcc += vjp_tiles(vg);
+      vAcc += packed_tiles(vjp_tiles(vg));
       ++A;
     }
     hRT[Rn] = rAcc;

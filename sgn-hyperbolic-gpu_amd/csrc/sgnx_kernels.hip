@@ -897,25 +897,24 @@ __global__ void __launch_bounds__(Sweep<TW>::NT, WAVES) k_rhs_sweep(BatchMember)
       xcd_tile(blockIdx.x, gridDim.x));
 }
 
-// Many grids in one launch: the workgroups of every member's tiles, packed
-// back to back (tileStart[m] = first packed index of member m, ascending);
-// each member keeps its own tile decomposition, so its error partials, and
+// Many grids in one launch: the workgroups of every member's tiles, one member
+// after the other (tileStart[m] = first workgroup of member m, ascending, a
+// multiple of the XCDs' number); each member keeps its own tile decomposition, so its error partials, and
 // everything else, equal its own launch's.
 template <int TW, int MODE, int WAVES, bool KEEP = false, bool HXR = false>
 __global__ void __launch_bounds__(Sweep<TW>::NT, WAVES)
 k_rhs_sweep_batch(const BatchMember* __restrict__ mem, const long long* __restrict__ tileStart,
                   int nMem) {
-  const long long w = xcd_tile(blockIdx.x, gridDim.x);
+  const long long w = blockIdx.x;
   int lo = 0, hi = nMem - 1;                  // last member with tileStart <= w
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (tileStart[mid] <= w) lo = mid; else hi = mid - 1;
   }
   const SweepArgs M = const_entry(mem, lo);
-  const int tile = __builtin_amdgcn_readfirstlane((int)(w - tileStart[lo]));
-  // a grid larger than the members' tiles (never launched so) does nothing
-  if (tile >= M->nTiles) return;
-  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(M, tile);
+  const int own = __builtin_amdgcn_readfirstlane((int)(w - tileStart[lo]));
+  if (own >= M->nTiles) return;               // (filling up)
+  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(M, xcd_tile(own, M->nTiles));
 }
 
 // Hx, Hy at every node (sgn2d.cpp:54-71).
