@@ -705,30 +705,21 @@ long long vjp_tiles(const Geometry& g) {
 
 long long vjp_row_tiles(const Geometry& g) { return (long long)vjp_strips(g) * g.Ny; }
 
-// A workgroup's time is that of its rows and the two staged beside them, the
-// launch's that of its fullest compute units. Per row a lone workgroup on a
-// unit takes 2.8 us, two, three and four together 3.6, 4.5 and 5.3 (a unit
-// holds four): in the ratio of 5 + 2 x for x workgroups, which is what the
-// heights are compared by, over the sets of four that the launch runs through.
+// The lowest time by sweep_cost: per row a lone workgroup on a unit takes 2.8 us,
+// two, three and four together 3.6, 4.5 and 5.3 (a unit holds four); the rows
+// staged beside a chunk cost as much as its own.
 //   products of a step, us      rows: 2    4    7   10   16   32
 //    128 x   64                     74   71   85  105
 //    256 x  128                    207  183  167  169  203
 //   1024 x  512                   3070 2464 2254 2176 2085 2053
 int vjp_rows(const Geometry* const* g, int n, int cus) {
-  const long long units = std::max(cus, 1);
-  long long best = 0;
-  int rows = 1;
-  for (int r = 1; r <= 32; ++r) {
+  constexpr SweepPace pace{4, 2.0, 0.8, 2.0, 2.0};
+  cus = std::max(cus, 1);
+  return choose_rows(32, [&](int r) {
     long long tiles = 0;
     for (int i = 0; i < n; ++i) tiles += (long long)vjp_strips(*g[i]) * ((g[i]->Ny + r - 1) / r);
-    const long long sets = tiles / (4 * units), rest = tiles % (4 * units);
-    const long long cost = (r + 2) * (13 * sets + (rest ? 5 + 2 * ((rest + units - 1) / units) : 0));
-    if (r == 1 || cost < best) {
-      best = cost;
-      rows = r;
-    }
-  }
-  return rows;
+    return sweep_cost(tiles, r, cus, pace);
+  });
 }
 
 VjpMember vjp_member(const Geometry& g, const Phys& ph, const VjpArgs& va, GhostTime gt) {

@@ -218,20 +218,15 @@ int sgnx_create(const sgnx_desc* d, sgnx_solver** out) {
   CK(hipGetDevice(&s->device));
   CK(scratch_address(s->device, &s->scratch));
   g.vrows = g.rows;
-  if (!std::getenv("SGNX_SWEEP_ROWS")) {
-    // default tile height: the tallest that still gives every compute unit
-    // about three workgroups (small grids would leave most of the chip idle
-    // at 16 rows). The RHS does not depend on it; the adaptive step's error
-    // norm is summed per workgroup, so its last bits can.
+  s->rowsSet = std::getenv("SGNX_SWEEP_ROWS") != nullptr;
+  if (!s->rowsSet) {
+    // The RHS and the products do not depend on the heights; the adaptive
+    // step's error norm is summed per g.rows rows, so its last bits can.
     int cus = 0;
     CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device));
-    const long long strips = (d->Nx + kStripW - 1) / kStripW, want = 3LL * std::max(cus, 1);
-    for (int r : {16, 12, 8, 6, 4, 3, 2}) {
-      g.rows = r;
-      if (strips * ((d->Ny + r - 1) / r) >= want) break;
-    }
     const Geometry* const one = &g;
-    g.vrows = vjp_rows(&one, 1, cus);   // (the products do not depend on it)
+    g.rows = sweep_rows(&one, 1, cus);
+    g.vrows = vjp_rows(&one, 1, cus);
   }
   const size_t Nd = (size_t)g.Nd, nst = (size_t)NV * Nd;
   const size_t nfx = (size_t)(d->Nx + 1) * d->Ny * NP, nfy = (size_t)d->Nx * (d->Ny + 1) * NP;
@@ -668,6 +663,7 @@ int sgnx_set_rhs_kernel(sgnx_solver* s, int variant, int rows) {
     return fail(s, SGNX_EUNSUPPORTED, "the row sweep has no Manning friction term (variant 0 has)");
   s->g.variant = variant;
   s->g.rows = rows;
+  s->rowsSet = true;
   return SGNX_OK;
 }
 

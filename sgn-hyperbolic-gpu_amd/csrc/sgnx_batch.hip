@@ -34,7 +34,7 @@
 struct sgnx_batch {
   std::vector<sgnx_solver*> m;
   int n = 0;
-  int device = 0;
+  int device = 0, cus = 1;
   int waves3 = 0x2;                    // bit k: launch kind k built for 3 waves/SIMD
   hipStream_t stream = nullptr;
   // argument tables, [4 launch kinds][n slots], and the tile offsets
@@ -90,25 +90,36 @@ void drop_graph(sgnx_batch* b) {
 }
 
 BatchMember member_args(const sgnx_solver* s, const double* U, double* dU, const Stage& sa,
-                        double t) {
-  BatchMember bm{};
-  bm.U = U;
-  bm.dU = dU;
-  bm.g = s->g;
-  bm.ph = s->ph;
-  bm.gt = ghost_time(s, t);
-  bm.sa = sa;
-  bm.nStrips = sweep_strips(s->g);
-  bm.nTiles = (int)sweep_tiles(s->g);
-  return bm;
+                        double t, int times = 1) {
+  return sweep_member(s->g, s->ph, U, dU, ghost_time(s, t), sa, times);
 }
 
-// tile offsets of the members in `set` (slot order) into h_ts; returns the total
-long long fill_offsets(sgnx_batch* b, const std::vector<int>& set) {
+// A member's own tile height suits a launch of its own; packed with others it
+// would make more and shorter workgroups than the device needs (24 grids of
+// 34x17 to 126x63, heights 1 and 2, or 4 for all: stages 2, 3 and 4 103, 142 and
+// 106 us, or 96, 128 and 109; ten accepted steps 5.25 ms, or 5.03).
+// So the members in `set` take the multiple of their own that is nearest to the
+// height for all their tiles together; a height set from outside or by an
+// autotuner is taken as it is.
+std::vector<int> row_multiples(const sgnx_batch* b, const std::vector<int>& set) {
+  std::vector<const Geometry*> gs;
+  for (int i : set) gs.push_back(&b->m[i]->g);
+  const int rows = sweep_rows(gs.data(), (int)gs.size(), b->cus);
+  std::vector<int> times;
+  for (int i : set) {
+    const sgnx_solver* s = b->m[i];
+    times.push_back(s->rowsSet ? 1 : std::max(1, (2 * rows + s->g.rows) / (2 * s->g.rows)));
+  }
+  return times;
+}
+
+// tile offsets of the members in `set` (slot order; their entries of h_mem from
+// `mem` on filled) into h_ts; returns the total
+long long fill_offsets(sgnx_batch* b, const std::vector<int>& set, const BatchMember* mem) {
   long long acc = 0;
   for (size_t i = 0; i < set.size(); ++i) {
     b->h_ts[i] = acc;
-    acc += packed_tiles(sweep_tiles(b->m[set[i]]->g));
+    acc += packed_tiles(mem[i].nTiles);
   }
   b->h_ts[set.size()] = acc;
   return acc;
@@ -195,6 +206,8 @@ int sgnx_batch_create(sgnx_solver* const* members, int n, sgnx_batch** out) {
     }
   };
   chk(hipSetDevice(dev), "hipSetDevice");
+  chk(hipDeviceGetAttribute(&b->cus, hipDeviceAttributeMultiprocessorCount, dev),
+      "hipDeviceGetAttribute");
   chk(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking), "hipStreamCreate");
   chk(hipHostMalloc((void**)&b->h_mem, 4 * (size_t)n * sizeof(BatchMember)), "hipHostMalloc");
   chk(hipMalloc((void**)&b->d_mem, 4 * (size_t)n * sizeof(BatchMember)), "hipMalloc");
@@ -243,13 +256,14 @@ int sgnx_batch_rhs(sgnx_batch* b, const double* const* U, double* const* dU, con
     BCHK(b, hipStreamSynchronize(b->m[i]->stream));
   }
   std::vector<int> all(n);
+  for (int i = 0; i < n; ++i) all[i] = i;
+  const std::vector<int> times = row_multiples(b, all);
   for (int i = 0; i < n; ++i) {
-    all[i] = i;
     Stage sa{};
     sa.u = U[i];
-    b->h_mem[i] = member_args(b->m[i], U[i], dU[i], sa, t[i]);
+    b->h_mem[i] = member_args(b->m[i], U[i], dU[i], sa, t[i], times[i]);
   }
-  const long long total = fill_offsets(b, all);
+  const long long total = fill_offsets(b, all, b->h_mem);
   BCHK(b, hipMemcpyAsync(b->d_mem, b->h_mem, (size_t)n * sizeof(BatchMember),
                          hipMemcpyHostToDevice, b->stream));
   BCHK(b, hipMemcpyAsync(b->d_ts, b->h_ts, ((size_t)n + 1) * sizeof(long long),
@@ -274,15 +288,16 @@ int sgnx_batch_integrate(sgnx_batch* b, const double* t0, const double* tEnd, co
   // FSAL heads: k1 = R(U) of every member, one launch
   {
     std::vector<int> all(n);
+    for (int i = 0; i < n; ++i) all[i] = i;
+    const std::vector<int> times = row_multiples(b, all);
     for (int i = 0; i < n; ++i) {
-      all[i] = i;
       sgnx_solver* s = b->m[i];
       Stage sa{};
       sa.u = s->d_U;
-      b->h_mem[i] = member_args(s, s->d_U, s->d_k1, sa, ctl[i].t);
+      b->h_mem[i] = member_args(s, s->d_U, s->d_k1, sa, ctl[i].t, times[i]);
       ++ctl[i].S.rhsEvals;
     }
-    const long long total = fill_offsets(b, all);
+    const long long total = fill_offsets(b, all, b->h_mem);
     BCHK(b, hipMemcpyAsync(b->d_mem, b->h_mem, (size_t)n * sizeof(BatchMember),
                            hipMemcpyHostToDevice, b->stream));
     BCHK(b, hipMemcpyAsync(b->d_ts, b->h_ts, ((size_t)n + 1) * sizeof(long long),
@@ -293,13 +308,17 @@ int sgnx_batch_integrate(sgnx_batch* b, const double* t0, const double* tEnd, co
     // refill them
     BCHK(b, hipStreamSynchronize(b->stream));
   }
-  std::vector<int> set;
+  std::vector<int> set, lastSet, times;
   int rc = SGNX_OK;
   for (;;) {
     set.clear();
     for (int i = 0; i < n; ++i)
       if (ctl[i].next()) set.push_back(i);
     if (set.empty()) break;
+    if (set != lastSet) {
+      times = row_multiples(b, set);
+      lastSet = set;
+    }
     const int A = (int)set.size();
     // members recording a tape: whether the step's input state is due as a
     // snapshot, and the buffers its stage launches keep their inputs in
@@ -316,12 +335,13 @@ int sgnx_batch_integrate(sgnx_batch* b, const double* t0, const double* tEnd, co
       bs3_launches(s, ctl[i].t, ctl[i].dt, opts[i].atol, opts[i].rtol, L);
       keep = keep || L[0].sa.yOut != nullptr;
       for (int k = 0; k < 3; ++k)
-        b->h_mem[(size_t)(k + 1) * n + slot] = member_args(s, L[k].sa.u, L[k].dU, L[k].sa, L[k].t);
+        b->h_mem[(size_t)(k + 1) * n + slot] =
+            member_args(s, L[k].sa.u, L[k].dU, L[k].sa, L[k].t, times[slot]);
     }
-    const long long total = fill_offsets(b, set);
+    const long long total = fill_offsets(b, set, b->h_mem + n);
     if (useGraph) {
       std::vector<int> rowsNow(A);
-      for (int slot = 0; slot < A; ++slot) rowsNow[slot] = b->m[set[slot]]->g.rows;
+      for (int slot = 0; slot < A; ++slot) rowsNow[slot] = times[slot] * b->m[set[slot]]->g.rows;
       if (!b->exec || b->graphSet != set || b->graphKeep != keep || b->graphTotal != total ||
           b->graphRows != rowsNow) {
         drop_graph(b);
@@ -425,6 +445,7 @@ int sgnx_autotune(sgnx_solver* s, int reps, int* rows_out, int* waves3_out) {
     }
   }
   s->g.rows = bestRows;
+  s->rowsSet = true;
   float p2 = 0.0f, p3 = 0.0f;
   if (timed(0, false, &p2) != hipSuccess || timed(0, true, &p3) != hipSuccess) {
     s->g = keep;
@@ -463,7 +484,7 @@ int sgnx_batch_autotune(sgnx_batch* b, int reps, int* rows_out, int* waves3_out)
       for (int k = 0; k < 3; ++k)
         b->h_mem[(size_t)(k + 1) * nn + i] = member_args(s, L[k].sa.u, L[k].dU, L[k].sa, L[k].t);
     }
-    return fill_offsets(b, all);
+    return fill_offsets(b, all, b->h_mem);
   };
   auto timed = [&](int k, bool three, long long total, float* ms) -> hipError_t {
     hipError_t e = launch_rhs_stage_batch(b->d_mem + k * nn, b->d_ts, n, total, k, three,
@@ -506,7 +527,10 @@ int sgnx_batch_autotune(sgnx_batch* b, int reps, int* rows_out, int* waves3_out)
       bestMask = mask;
     }
   }
-  for (sgnx_solver* s : b->m) s->g.rows = bestRows;
+  for (sgnx_solver* s : b->m) {
+    s->g.rows = bestRows;
+    s->rowsSet = true;
+  }
   const long long total = fill();
   BCHK(b, hipMemcpyAsync(b->d_mem, b->h_mem, 4 * nn * sizeof(BatchMember),
                          hipMemcpyHostToDevice, b->stream));
@@ -543,10 +567,8 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
     return bfail(b, SGNX_EINVAL, "batch adjoint: bad memory kind");
   const int n = b->n;
   BCHK(b, hipSetDevice(b->device));
-  int cus = 0;
-  BCHK(b, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
   bool each_fills = n > 0;
-  for (int i = 0; i < n; ++i) each_fills = each_fills && vjp_row_tiles(b->m[i]->g) >= 6LL * cus;
+  for (int i = 0; i < n; ++i) each_fills = each_fills && vjp_row_tiles(b->m[i]->g) >= 6LL * b->cus;
   if (each_fills) {
     for (int i = 0; i < n; ++i) {
       sgnx_solver* s = b->m[i];
@@ -564,7 +586,7 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
   // one tile height for all members' products, unless set from outside
   std::vector<const Geometry*> gs;
   for (int i = 0; i < n; ++i) gs.push_back(&b->m[i]->g);
-  const int vrows = std::getenv("SGNX_SWEEP_ROWS") ? 0 : vjp_rows(gs.data(), n, cus);
+  const int vrows = std::getenv("SGNX_SWEEP_ROWS") ? 0 : vjp_rows(gs.data(), n, b->cus);
   std::vector<AdjTape*> tp(n, nullptr);
   std::vector<const double*> gb(n, nullptr);
   long Nmax = 0;
@@ -608,6 +630,9 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
   auto* hV1 = reinterpret_cast<VjpMember*>(b->h_adj + oV1);
   auto* hVT = reinterpret_cast<long long*>(b->h_adj + oVT);
   auto dptr = [&](size_t off) { return b->d_adj + off; };
+  std::vector<int> all(n);
+  for (int i = 0; i < n; ++i) all[i] = i;
+  const std::vector<int> times = row_multiples(b, all);
   for (long k = 0; k < Nmax; ++k) {
     int A = 0, Rn = 0;   // members in this step; of those, the ones that recompute stages
     long long rAcc = 0, vAcc = 0;
@@ -634,7 +659,7 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
       if (!kept) {
         Stage s1{};
         s1.u = u;
-        hR1[Rn] = member_args(s, u, s->d_k1, s1, t);
+        hR1[Rn] = member_args(s, u, s->d_k1, s1, t, times[i]);
         // the forward's stage-2 launch, keeping its input and forming the
         // next one: y2, k2 = R(y2) and y3 = u + 3dt/4 k2
         Stage s2{};
@@ -644,9 +669,9 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
         s2.yOut = s->d_tmp;
         s2.y3Out = s->d_k3;
         s2.a3 = 0.75 * dt;
-        hR2[Rn] = member_args(s, u, s->d_k2, s2, t + 0.5 * dt);
+        hR2[Rn] = member_args(s, u, s->d_k2, s2, t + 0.5 * dt, times[i]);
         hRT[Rn] = rAcc;
-        rAcc += packed_tiles(sweep_tiles(s->g));
+        rAcc += packed_tiles(hR1[Rn].nTiles);
         ++Rn;
       }
       VjpArgs p[3];

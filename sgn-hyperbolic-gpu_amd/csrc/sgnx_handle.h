@@ -21,6 +21,7 @@ struct sgnx_solver {
   int P = 4, Nx = 0, Ny = 0;
   double Lx = 0.0, Ly = 0.0, hx = 0.0, hy = 0.0;
   Geometry g{};
+  bool rowsSet = false;      // g.rows set from outside or by an autotuner, not by the rule
   Phys ph{};
   hipStream_t stream = nullptr;
   int device = 0;

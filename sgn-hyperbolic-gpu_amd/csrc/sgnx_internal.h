@@ -57,6 +57,29 @@ __device__ __forceinline__ int xcd_tile(int bid, int nb) {
 // and 538 us instead of 403, 571 and 462.)
 inline long long packed_tiles(long long tiles) { return (tiles + kXcd - 1) / kXcd * kXcd; }
 
+// Time of a sweep launch whose `tiles` workgroups take `rows` rows each, by what
+// one row takes with x workgroups on the same compute unit, alone + each * x
+// (at most `hold` fit): sets of hold * cus workgroups follow each other, the
+// last one spread over the units. `full`, `last`: what starting a workgroup
+// costs in rows, where others fill its wait and where they don't.
+struct SweepPace { int hold; double alone, each, full, last; };
+inline double sweep_cost(long long tiles, int rows, int cus, const SweepPace& p) {
+  const long long set = (long long)p.hold * cus, rest = tiles % set;
+  return (rows + p.full) * (double)(tiles / set) * (p.alone + p.each * p.hold) +
+         (rest ? (rows + p.last) * (p.alone + p.each * (double)((rest + cus - 1) / cus)) : 0.0);
+}
+
+// The lowest height within a hundredth of the best cost: lower tiles even out
+// the end of a launch, which sweep_cost leaves out.
+template <class Cost>
+inline int choose_rows(int most, Cost cost) {
+  double best = cost(1);
+  for (int r = 2; r <= most; ++r) best = cost(r) < best ? cost(r) : best;
+  int r = 1;
+  while (cost(r) > 1.01 * best) ++r;
+  return r;
+}
+
 // What one RHS launch needs besides the stage input and output.
 struct Geometry {
   int Nx, Ny;
@@ -72,7 +95,7 @@ struct Geometry {
   const double* inflow;      // device, Ny*5*15 or null
   ConstDiv dx, dy;           // division by Jx, Jy
   int variant;               // RHS kernel: 0 element-row tiles, 1 row sweep
-  int rows;                  // row sweep: element rows per workgroup
+  int rows;                  // row sweep: element rows per workgroup (in a batch a multiple)
   int vrows;                 // the adjoint's product: element rows per workgroup
   int waves3;                // row sweep: bit m set = stage mode m built for 3 waves/SIMD
   int hxr;                   // Hx, Hy equal (D Hnod) / J bit for bit: the row sweep forms
@@ -117,8 +140,10 @@ struct Stage {
 };
 
 // One grid of a batched launch: its operands, geometry, constants, inflow
-// time factors and stage, and its row-sweep decomposition (strips per chunk
-// row, tiles in all).
+// time factors and stage, and its row-sweep decomposition (element rows per
+// workgroup, a multiple of g.rows; strips per chunk row; tiles in all). kErr
+// writes a partial triple for every g.rows rows of a strip, `parts` in all, so
+// that the norm does not depend on `rows`.
 struct BatchMember {
   const double* U;
   double* dU;
@@ -126,8 +151,10 @@ struct BatchMember {
   Phys ph;
   GhostTime gt;
   Stage sa;
+  int rows;
   int nStrips;
   int nTiles;
+  int parts;
 };
 
 // ---- launchers (sgnx_kernels.hip); all asynchronous on `st` ----------------
@@ -154,12 +181,16 @@ hipError_t launch_rhs_stage_batch(const BatchMember* mem, const long long* tileS
                                   long long totalTiles, int mode, bool waves3, hipStream_t st,
                                   bool keep = false, bool hxr = false);
 // launch_finish for every member: member m's partials (mem[m].sa.part, its
-// nTiles) into out[2m], out[2m + 1]
+// parts) into out[2m], out[2m + 1]
 hipError_t launch_finish_batch(const BatchMember* mem, int nMem, double* out, hipStream_t st);
-// row-sweep strips per chunk row of a grid
-int sweep_strips(const Geometry& g);
-// workgroups of one row-sweep launch (sizes the partial buffer)
+// workgroups of one row-sweep launch of g.rows rows each (the partial triples
+// of kErr, also where a workgroup takes several times g.rows)
 long long sweep_tiles(const Geometry& g);
+// operands and decomposition of a launch whose workgroups take times * g.rows rows
+BatchMember sweep_member(const Geometry& g, const Phys& ph, const double* U, double* dU,
+                         GhostTime gt, const Stage& sa, int times = 1);
+// element rows per workgroup for the grids of one launch
+int sweep_rows(const Geometry* const* g, int n, int cus);
 // Hx, Hy = (D . Hnod) / J per element line (sgn2d.cpp:54-71)
 hipError_t launch_bathy_grad(const Geometry& g, const double* Hnod, double* Hx, double* Hy,
                              hipStream_t st);

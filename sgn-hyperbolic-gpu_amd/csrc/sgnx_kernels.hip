@@ -27,6 +27,8 @@
 // file is compiled with -ffp-contract=off.
 // =============================================================================
 
+#include <algorithm>
+
 #include "sgnx_device.h"
 #include "sgnx_internal.h"
 
@@ -450,7 +452,7 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
   const ConstDiv divX{A->g.dx.b, A->g.dx.rh, A->g.dx.rl, 1}, divY{A->g.dy.b, A->g.dy.rh, A->g.dy.rl, 1};
   const double stA = A->sa.a, stDt = A->sa.dt, atol = A->sa.atol, rtol = A->sa.rtol;
   const int bcL = A->g.bc[0], bcR = A->g.bc[1], bcB = A->g.bc[2], bcT = A->g.bc[3];
-  const int nStrips = A->nStrips, rows = A->g.rows, Nx = A->g.Nx, Ny = A->g.Ny;
+  const int nStrips = A->nStrips, rows = A->rows, Nx = A->g.Nx, Ny = A->g.Ny;
   __shared__ L lds;
 
   if (threadIdx.x < NP) {
@@ -463,7 +465,7 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
   }
 
   const int chunk = __builtin_amdgcn_readfirstlane(tile / nStrips);
-  const int ex0 = (tile - chunk * nStrips) * TW;
+  const int strip = tile - chunk * nStrips, ex0 = strip * TW;
   const int nW = min(TW, Nx - ex0);
   const int ey0 = chunk * rows;
   const int ey1 = min(Ny, ey0 + rows);
@@ -874,18 +876,26 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
     row_sync();
     rowOff += rowBytes;
   };
-  for (int r = ey0; r < ey1; ++r) row(r);
-
-  if (MODE == kErr) {
+  if (MODE != kErr) {
+    for (int r = ey0; r < ey1; ++r) row(r);
+    return;
+  }
+  // the norm's partials: one for every g.rows rows
+  int done = ey0;
+  for (long long at = (long long)(ey0 / A->g.rows) * nStrips + strip; done < ey1; at += nStrips) {
+    const int to = min(ey1, done + A->g.rows);
+    for (; done < to; ++done) row(done);
     if (!isNode) eS = eC = eM = 0.0;                     // node 0 counts once
     // fixed-order reduction over the workgroup (LDS of the last row reused)
     block_reduce(eS, eC, eM, lds.node);
     if (t == 0) {
-      double* const part = A->sa.part + 3 * (size_t)tile;
+      double* const part = A->sa.part + 3 * at;
       part[0] = eS;
       part[1] = eC;
       part[2] = eM;
     }
+    eS = eC = eM = 0.0;
+    row_sync();
   }
 }
 
@@ -1060,7 +1070,7 @@ k_finish_post(const double* __restrict__ part, int nb, double* __restrict__ host
 __global__ void __launch_bounds__(kThreads)
 k_finish_batch(const BatchMember* __restrict__ mem, int nMem, double* __restrict__ out) {
   const BatchMember& M = mem[blockIdx.x];
-  finish_block(M.sa.part, M.nTiles, out + 2 * blockIdx.x);
+  finish_block(M.sa.part, M.parts, out + 2 * blockIdx.x);
 }
 
 // Max of eta = h - H over the nodes inside the open window (x0, x1) x (y0, y1)
@@ -1231,7 +1241,6 @@ void sweep_launch_batch(bool hxr, dim3 grid, dim3 block, hipStream_t st, const B
 
 hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const Stage& sa,
                             double* dU, GhostTime gt, hipStream_t st) {
-  const int strips = (g.Nx + kTileW - 1) / kTileW;
   const long long tiles = sweep_tiles(g);
   if (tiles > 0x7fffffffLL || g.rows < 1) return hipErrorInvalidValue;
   const dim3 grid((unsigned)tiles), block(Sweep<kTileW>::NT);
@@ -1239,11 +1248,8 @@ hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const S
   // g.waves3 set: 3 waves, else 2)
   const bool w3 = (g.waves3 >> mode) & 1;
   if (mode < kPlain || mode > kErr || ph.nManning != 0.0) return hipErrorInvalidValue;
-  // Hx, Hy formed from Hnod (when the device check allowed it) in the
-  // two-wave stage builds; the plain build and the three-wave stage-2 build
-  // have no registers for it and read them
-  const bool hxr = g.hxr != 0;
-  const BatchMember args{sa.u, dU, g, ph, gt, sa, strips, (int)tiles};
+  const bool hxr = g.hxr != 0;   // Hx, Hy formed from Hnod
+  const BatchMember args = sweep_member(g, ph, sa.u, dU, gt, sa);
 #define SGNX_SWEEP(M, W, K) sweep_launch<M, W, K>(hxr, grid, block, st, args)
   const bool keep = sa.yOut != nullptr;
   if (mode == kPlain) { if (w3) SGNX_SWEEP(kPlain, 3, false); else SGNX_SWEEP(kPlain, 2, false); }
@@ -1258,7 +1264,33 @@ hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const S
   return hipGetLastError();
 }
 
-int sweep_strips(const Geometry& g) { return (g.Nx + kTileW - 1) / kTileW; }
+BatchMember sweep_member(const Geometry& g, const Phys& ph, const double* U, double* dU,
+                         GhostTime gt, const Stage& sa, int times) {
+  BatchMember m{U, dU, g, ph, gt, sa, times * g.rows, (g.Nx + kTileW - 1) / kTileW, 0, 0};
+  m.nTiles = (int)(m.nStrips * (((long long)g.Ny + m.rows - 1) / m.rows));
+  m.parts = (int)sweep_tiles(g);
+  return m;
+}
+
+// The lowest time of a step by sweep_cost, in us: six workgroups of the plain
+// launch and of stage 2 fit on a compute unit, four of stage 3 and of the last
+// stage. Measured (plain, stage 2, stage 3, last):
+//   rows            1            2            5            7            8           12           16
+//   128 x  64  16 20 22 20  15 18 19 19  24 28 28 30  31 34 36 37  29 31 33 34  40 43 46 47  51 54 58 60
+//   256 x 128  38 47 58 49  34 41 50 43  33 40 55 42  35 40 43 43  38 43 46 47  50 55 58 61  63 68 72 76
+//   387 x 191 73 104 145 109 63 87 118 92 60 77 105 88 66 82 108 89 72 86 100 96 65 78 109 88 71 85 100 96
+//   603 x 301 (all four) 1033  833  734  728  735  786  770;  1024 x 512  -  -  -  -  1932 1943 1951
+// It takes 2, 7, 5, 8 and 8 rows there.
+int sweep_rows(const Geometry* const* g, int n, int cus) {
+  constexpr SweepPace six{6, 2.5, 0.5, 0.5, 1.8}, four{4, 2.6, 0.65, 0.5, 1.6};
+  cus = std::max(cus, 1);
+  return choose_rows(24, [&](int r) {
+    long long tiles = 0;
+    for (int i = 0; i < n; ++i)
+      tiles += (long long)((g[i]->Nx + kTileW - 1) / kTileW) * ((g[i]->Ny + r - 1) / r);
+    return sweep_cost(tiles, r, cus, six) + sweep_cost(tiles, r, cus, four);
+  });
+}
 
 hipError_t launch_rhs_stage_batch(const BatchMember* mem, const long long* tileStart, int nMem,
                                   long long totalTiles, int mode, bool waves3, hipStream_t st,
