@@ -656,6 +656,21 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
   LdsDouble* sTa = (LdsDouble*)lds.tab[a];
   LdsDouble* sTb = (LdsDouble*)lds.tab[b];
 
+  // The lane's rows of D and weights: kept in registers by the plain launch,
+  // which LDS reads bound (2000x1000 1302 -> 1256 us, 1024x512 350 -> 343); the
+  // stage launches wait for memory and gain nothing.
+  constexpr bool kTabRegs = MODE == kPlain;
+  double Da[NP], Db[NP], gLa, gRa, gLb, gRb;
+  auto load_tab = [&](auto* ta, auto* tb) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) { Da[k] = ta[k]; Db[k] = tb[k]; }
+    gLa = ta[NP], gRa = ta[NP + 1], gLb = tb[NP], gRb = tb[NP + 1];
+  };
+  if (kTabRegs) {
+    __syncthreads();
+    load_tab(sTa, sTb);
+  }
+
   auto row = [&](int r) {
     // opaque in every row: the planes of all operands kept across rows would
     // exceed the scalar registers, and a lane offset folded into them would
@@ -765,10 +780,7 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
     face_load(opaque(A), plane);
     __builtin_amdgcn_sched_barrier(0);
     {
-      double Da[NP], Db[NP];
-#pragma unroll
-      for (int k = 0; k < NP; ++k) { Da[k] = sTa[k]; Db[k] = sTb[k]; }
-      const double gLa = sTa[NP], gRa = sTa[NP + 1], gLb = sTb[NP], gRb = sTb[NP + 1];
+      if (!kTabRegs) load_tab(sTa, sTb);
       LdsDouble* const jB = sJy + (r & 1) * kJLine;         // the line below the row
       LdsDouble* const jT = sJy + ((r + 1) & 1) * kJLine;   // and the one above it
       // The dividends of one pair of quotients, along x and along y: D . f of
