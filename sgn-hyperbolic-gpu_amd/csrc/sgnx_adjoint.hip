@@ -700,7 +700,7 @@ int vjp_nop(const VjpArgs& va) { return va.acc ? 3 : va.B ? 2 : 1; }
 }  // namespace
 
 long long vjp_tiles(const Geometry& g) {
-  return (long long)vjp_strips(g) * ((g.Ny + g.vrows - 1) / g.vrows);
+  return (long long)vjp_strips(g) * (((long long)g.Ny + g.vrows - 1) / g.vrows);
 }
 
 long long vjp_row_tiles(const Geometry& g) { return (long long)vjp_strips(g) * g.Ny; }

@@ -100,9 +100,8 @@ __device__ __forceinline__ double lane32(double x) {
   return __hiloint2double(hi, lo);
 }
 
-// Every thread of the block calls it (no divergence); the result is in
-// thread 0's s, c, m. ws: 3 doubles of LDS per wave.
-__device__ __forceinline__ void block_reduce(double& s, double& c, double& m, double* ws) {
+// a wavefront's triples into its lane 0
+__device__ __forceinline__ void wave_reduce(double& s, double& c, double& m) {
   wave_level<1>(s, c, m);
   wave_level<2>(s, c, m);
   wave_level<4>(s, c, m);
@@ -110,6 +109,12 @@ __device__ __forceinline__ void block_reduce(double& s, double& c, double& m, do
   wave_level<16>(s, c, m);
   const double s2 = lane32(s), c2 = lane32(c), m2 = lane32(m);
   merge3(s, c, m, s2, c2, m2);
+}
+
+// Every thread of the block calls it (no divergence); the result is in
+// thread 0's s, c, m. ws: 3 doubles of LDS per wave.
+__device__ __forceinline__ void block_reduce(double& s, double& c, double& m, double* ws) {
+  wave_reduce(s, c, m);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (lane == 0) {
     ws[3 * w] = s;
@@ -1040,24 +1045,58 @@ k_err_norm(const double* __restrict__ u, const double* __restrict__ uNew,
 }
 
 // Second level: one block folds the nb partial triples in a fixed order.
-// out[0] = sum, out[1] = max.
+// out[0] = sum, out[1] = max. Its time is that of its loads, one after the
+// other where each waits for the last: eight triples a thread are on their way
+// at once (13120 triples, of 1024x512: 25.3 -> 9.5 us; 832: 3.8 either way; twice
+// the threads: 9.4, but 2 % of a 128x64 step).
+constexpr int kFinish = 512;
 __device__ __forceinline__ void finish_block(const double* __restrict__ part, int nb,
                                              double* __restrict__ out) {
-  __shared__ double ws[3 * kThreads / 64];
+  static_assert(kFinish == 8 * 64, "a tree of 8 waves");
+  __shared__ double ws[kFinish / 64][3];
+  constexpr int kAhead = 8;
   double s = 0.0, c = 0.0, m = 0.0;
-  for (int i = threadIdx.x; i < nb; i += kThreads) {
-    acc_add(s, c, part[3 * i]);
-    c = c + part[3 * i + 1];
-    m = fmax(m, part[3 * i + 2]);
+  for (int i0 = threadIdx.x; i0 < nb; i0 += kAhead * kFinish) {
+    double x[kAhead][3];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      const size_t i = (size_t)min(i0 + q * kFinish, nb - 1);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[q][k] = part[3 * i + k];
+    }
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      if (i0 + q * kFinish < nb) {
+        acc_add(s, c, x[q][0]);
+        c = c + x[q][1];
+        m = fmax(m, x[q][2]);
+      }
+    }
   }
-  block_reduce(s, c, m, ws);
-  if (threadIdx.x == 0) {
-    out[0] = s + c;
-    out[1] = m;
+  wave_reduce(s, c, m);
+  if ((threadIdx.x & 63) == 0) {
+    ws[threadIdx.x >> 6][0] = s;
+    ws[threadIdx.x >> 6][1] = c;
+    ws[threadIdx.x >> 6][2] = m;
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    // the waves' triples by a tree of their own (each half of the wave alike)
+    const int w = threadIdx.x & (kFinish / 64 - 1);
+    s = ws[w][0];
+    c = ws[w][1];
+    m = ws[w][2];
+    wave_level<1>(s, c, m);
+    wave_level<2>(s, c, m);
+    wave_level<4>(s, c, m);
+    if (threadIdx.x == 0) {
+      out[0] = s + c;
+      out[1] = m;
+    }
   }
 }
 
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kFinish)
 k_finish(const double* __restrict__ part, int nb, double* __restrict__ out) {
   finish_block(part, nb, out);
 }
@@ -1065,7 +1104,7 @@ k_finish(const double* __restrict__ part, int nb, double* __restrict__ out) {
 // k_finish writing straight into host memory mapped for the device: the
 // (sum, max) pair, then, after a system-scope fence, the attempt's sequence
 // number, for which the host polls.
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kFinish)
 k_finish_post(const double* __restrict__ part, int nb, double* __restrict__ host,
               unsigned long long seq) {
   __shared__ double pair[2];
@@ -1079,7 +1118,7 @@ k_finish_post(const double* __restrict__ part, int nb, double* __restrict__ host
 }
 
 // one block per member: member m's partials into out[2m], out[2m+1]
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kFinish)
 k_finish_batch(const BatchMember* __restrict__ mem, int nMem, double* __restrict__ out) {
   const BatchMember& M = mem[blockIdx.x];
   finish_block(M.sa.part, M.parts, out + 2 * blockIdx.x);
@@ -1323,18 +1362,18 @@ hipError_t launch_rhs_stage_batch(const BatchMember* mem, const long long* tileS
 
 hipError_t launch_finish_batch(const BatchMember* mem, int nMem, double* out, hipStream_t st) {
   if (nMem < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_finish_batch, dim3((unsigned)nMem), dim3(kThreads), 0, st, mem, nMem, out);
+  hipLaunchKernelGGL(k_finish_batch, dim3((unsigned)nMem), dim3(kFinish), 0, st, mem, nMem, out);
   return hipGetLastError();
 }
 
 hipError_t launch_finish_post(const double* part, long long nb, double* host,
                               unsigned long long seq, hipStream_t st) {
-  hipLaunchKernelGGL(k_finish_post, dim3(1), dim3(kThreads), 0, st, part, (int)nb, host, seq);
+  hipLaunchKernelGGL(k_finish_post, dim3(1), dim3(kFinish), 0, st, part, (int)nb, host, seq);
   return hipGetLastError();
 }
 
 hipError_t launch_finish(const double* part, long long nb, double* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, (int)nb, out);
+  hipLaunchKernelGGL(k_finish, dim3(1), dim3(kFinish), 0, st, part, (int)nb, out);
   return hipGetLastError();
 }
 
@@ -1398,7 +1437,7 @@ hipError_t launch_err_norm(const double* u, const double* uNew, const double* k1
                      k4, dt, atol, rtol, n, part);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, kReduceBlocks, out);
+  hipLaunchKernelGGL(k_finish, dim3(1), dim3(kFinish), 0, st, part, kReduceBlocks, out);
   return hipGetLastError();
 }
 
@@ -1429,7 +1468,7 @@ hipError_t launch_diag(const Geometry& g, const Phys& ph, const double* U, int w
   hipLaunchKernelGGL(k_diag, dim3(kReduceBlocks), dim3(kThreads), 0, st, U, g, ph, which, part);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_finish, dim3(1), dim3(kThreads), 0, st, part, kReduceBlocks, out);
+  hipLaunchKernelGGL(k_finish, dim3(1), dim3(kFinish), 0, st, part, kReduceBlocks, out);
   return hipGetLastError();
 }
 
