@@ -14,7 +14,7 @@ namespace sgnx {
 
 // W = ca*A (+ cb*B when B is given); out = (dR/dU (U))^T W, or, when acc is
 // given (with B), ((A + acc) + B) + that; thetaBar += (dR/dtheta)^T W (when not
-// null). 5*Nd arrays; out is none of the inputs (a workgroup reads its
+// null; set to 0 + that where `fresh`, which takes A only). 5*Nd arrays; out is none of the inputs (a workgroup reads its
 // neighbours' A and B).
 struct VjpArgs {
   const double* U;
@@ -25,6 +25,7 @@ struct VjpArgs {
   const double* acc;
   double* out;
   double* thetaBar;
+  bool fresh = false;
 };
 
 // One product with its geometry and decomposition: a launch's arguments, or

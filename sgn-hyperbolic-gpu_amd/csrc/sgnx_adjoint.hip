@@ -218,15 +218,10 @@ __device__ __forceinline__ void cotangent(const double* A, const double* B, doub
 }
 
 // NOP: 1: W = ca A; 2: W = ca A + cb B; 3: that, and out = ((A + acc) + B) +
-// the product.
-template <int NOP>
-struct VjpLdsOf : VjpLds {};
-template <>
-struct VjpLdsOf<3> : VjpLds {
-  double base[2][NV][kN];                    // (A + acc) + B by row parity
-};
-
-template <int NOP>
+// the product. FRESH: thetaBar is set to 0 + the product and not read (a product
+// by itself: 597 -> 566 us at 1024x512 against clearing it and adding; as a
+// run-time switch 583, and 0.6 % of a reverse sweep for the registers it takes).
+template <int NOP, bool FRESH>
 __device__ __forceinline__ void vjp_tile(ConstArgs<VjpMember> M, int tile) {
   using L = VjpLds;
   constexpr int kRec = L::kRec;
@@ -350,7 +345,9 @@ __device__ __forceinline__ void vjp_tile(ConstArgs<VjpMember> M, int tile) {
     // ---- stage ---------------------------------------------------------------
     const ConstArgs<VjpMember> R0 = opaque(M);
     double* const tbar = R0->va.thetaBar;
-    const double thOld = load_at(global_at(tbar ? tbar : R0->va.U, (unsigned)row_of(r - 1)), n8);
+    // (a fresh one isn't read: every lane takes the same entry in its place)
+    const double thOld =
+        FRESH ? 0.0 : load_at(global_at(tbar ? tbar : R0->va.U, (unsigned)row_of(r - 1)), n8);
     const double hNext = load_h(R0, r + 2, h8);
     const unsigned rowAt = (unsigned)row_of(r);
     const double Hl = load_at(global_at(R0->g.Hnod, rowAt), n8);
@@ -594,9 +591,9 @@ __device__ __forceinline__ void vjp_tile(ConstArgs<VjpMember> M, int tile) {
 }
 
 // The arguments are the kernel's only parameter, read where they lie.
-template <int NOP>
+template <int NOP, bool FRESH>
 __global__ void __launch_bounds__(kVT, 3) k_vjp_sweep(VjpMember) {
-  vjp_tile<NOP>((ConstArgs<VjpMember>)__builtin_amdgcn_kernarg_segment_ptr(),
+  vjp_tile<NOP, FRESH>((ConstArgs<VjpMember>)__builtin_amdgcn_kernarg_segment_ptr(),
                      xcd_tile(blockIdx.x, gridDim.x));
 }
 
@@ -616,7 +613,7 @@ k_vjp_sweep_batch(const VjpMember* __restrict__ mem, const long long* __restrict
   const int own = __builtin_amdgcn_readfirstlane((int)(w - tileStart[lo]));
   const ConstArgs<VjpMember> M = const_entry(mem, lo);
   if (own >= M->nTiles) return;   // (filling up)
-  vjp_tile<NOP>(M, xcd_tile(own, M->nTiles));
+  vjp_tile<NOP, false>(M, xcd_tile(own, M->nTiles));
 }
 
 // lam[node] += Gb[k], thetaBar[node] -= Gb[k] for the n gauges of one log row,
@@ -729,16 +726,16 @@ VjpMember vjp_member(const Geometry& g, const Phys& ph, const VjpArgs& va, Ghost
 hipError_t launch_rhs_vjp(const Geometry& g, const Phys& ph, const VjpArgs& va, GhostTime gt,
                           hipStream_t st) {
   const long long nb = vjp_tiles(g);
-  if (nb > 0x7fffffffLL || va.out == va.A || va.out == va.B || (va.acc && !va.B))
+  const int nop = vjp_nop(va);
+  if (nb > 0x7fffffffLL || (va.fresh && nop != 1) || va.out == va.A || va.out == va.B || (va.acc && !va.B))
     return hipErrorInvalidValue;
   const VjpMember m = vjp_member(g, ph, va, gt);
   const dim3 grid((unsigned)nb), block(kVT);
-#define SGNX_VJP(N) hipLaunchKernelGGL(k_vjp_sweep<N>, grid, block, 0, st, m)
-  switch (vjp_nop(va)) {
-    case 1: SGNX_VJP(1); break;
-    case 2: SGNX_VJP(2); break;
-    default: SGNX_VJP(3);
-  }
+#define SGNX_VJP(...) hipLaunchKernelGGL((k_vjp_sweep<__VA_ARGS__>), grid, block, 0, st, m)
+  if (va.fresh) SGNX_VJP(1, true);
+  else if (nop == 1) SGNX_VJP(1, false);
+  else if (nop == 2) SGNX_VJP(2, false);
+  else SGNX_VJP(3, false);
 #undef SGNX_VJP
   return hipGetLastError();
 }

@@ -540,8 +540,7 @@ int sgnx_rhs_vjp(sgnx_solver* s, const double* U, const double* W, double* Ubar,
   } else if (Ubar == U || Ubar == W) {
     return fail(s, SGNX_EINVAL, "rhs_vjp: Ubar must not overlap U or W");
   }
-  if (dTh) HIPCHK(s, hipMemsetAsync(dTh, 0, Nd * sizeof(double), s->stream));
-  const VjpArgs va{dU, dW, 1.0, nullptr, 0.0, nullptr, dOut, dTh};
+  const VjpArgs va{dU, dW, 1.0, nullptr, 0.0, nullptr, dOut, dTh, true};
   if ((rc = vjp(s, va, t))) return rc;
   if (mem == SGNX_MEM_HOST) {
     HIPCHK(s, hipMemcpyAsync(Ubar, dOut, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
