@@ -217,6 +217,14 @@ __device__ __forceinline__ void cotangent(const double* A, const double* B, doub
   }
 }
 
+// the third product's workgroup also holds a row's sums of the other cotangents
+template <int NOP>
+struct VjpLdsOf : VjpLds {};
+template <>
+struct VjpLdsOf<3> : VjpLds {
+  double base[2][NV][kN];                    // (A + acc) + B by row parity
+};
+
 // NOP: 1: W = ca A; 2: W = ca A + cb B; 3: that, and out = ((A + acc) + B) +
 // the product. FRESH: thetaBar is set to 0 + the product and not read (a product
 // by itself: 597 -> 566 us at 1024x512 against clearing it and adding; as a
