@@ -180,9 +180,10 @@ hipError_t launch_finish_post(const double* part, long long nb, double* host,
 hipError_t launch_rhs_stage_batch(const BatchMember* mem, const long long* tileStart, int nMem,
                                   long long totalTiles, int mode, bool waves3, hipStream_t st,
                                   bool keep = false, bool hxr = false);
-// launch_finish for every member: member m's partials (mem[m].sa.part, its
-// parts) into out[2m], out[2m + 1]
-hipError_t launch_finish_batch(const BatchMember* mem, int nMem, double* out, hipStream_t st);
+// launch_finish_post for every member: member m's partials (mem[m].sa.part, its
+// parts) into host[3m], host[3m + 1], then *seq (device) into host[3m + 2]
+hipError_t launch_finish_batch(const BatchMember* mem, int nMem, double* host,
+                               const long long* seq, hipStream_t st);
 // workgroups of one row-sweep launch of g.rows rows each (the partial triples
 // of kErr, also where a workgroup takes several times g.rows)
 long long sweep_tiles(const Geometry& g);

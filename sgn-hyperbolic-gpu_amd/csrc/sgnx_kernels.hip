@@ -1117,11 +1117,21 @@ k_finish_post(const double* __restrict__ part, int nb, double* __restrict__ host
   }
 }
 
-// one block per member: member m's partials into out[2m], out[2m+1]
+// k_finish_post for every member, a block each: member m's pair and the
+// attempt's sequence number into host[3m], host[3m + 1], host[3m + 2]
 __global__ void __launch_bounds__(kFinish)
-k_finish_batch(const BatchMember* __restrict__ mem, int nMem, double* __restrict__ out) {
+k_finish_batch(const BatchMember* __restrict__ mem, int nMem, double* __restrict__ host,
+               const unsigned long long* __restrict__ seq) {
   const BatchMember& M = mem[blockIdx.x];
-  finish_block(M.sa.part, M.parts, out + 2 * blockIdx.x);
+  double* const out = host + 3 * (size_t)blockIdx.x;
+  __shared__ double pair[2];
+  finish_block(M.sa.part, M.parts, pair);
+  if (threadIdx.x == 0) {
+    out[0] = pair[0];
+    out[1] = pair[1];
+    __threadfence_system();
+    reinterpret_cast<volatile unsigned long long*>(out)[2] = *seq;
+  }
 }
 
 // Max of eta = h - H over the nodes inside the open window (x0, x1) x (y0, y1)
@@ -1360,9 +1370,11 @@ hipError_t launch_rhs_stage_batch(const BatchMember* mem, const long long* tileS
   return hipGetLastError();
 }
 
-hipError_t launch_finish_batch(const BatchMember* mem, int nMem, double* out, hipStream_t st) {
+hipError_t launch_finish_batch(const BatchMember* mem, int nMem, double* host,
+                               const long long* seq, hipStream_t st) {
   if (nMem < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_finish_batch, dim3((unsigned)nMem), dim3(kFinish), 0, st, mem, nMem, out);
+  hipLaunchKernelGGL(k_finish_batch, dim3((unsigned)nMem), dim3(kFinish), 0, st, mem, nMem, host,
+                     reinterpret_cast<const unsigned long long*>(seq));
   return hipGetLastError();
 }
 
