@@ -47,10 +47,9 @@ struct GaugeMember {
   double* lam;
   double* thetaBar;
 };
-long long vjp_tiles(const Geometry& g);       // workgroups of one product launch
 long long vjp_row_tiles(const Geometry& g);   // strips times element rows
-// element rows per workgroup for the grids of one launch (Geometry::vrows)
-int vjp_rows(const Geometry* const* g, int n, int cus);
+// element rows per workgroup for the grids of one launch (Geometry::vrows[third])
+int vjp_rows(const Geometry* const* g, int n, int cus, bool third);
 // nop: 1 = A only, 2 = A and B, 3 = with acc too, for all members
 hipError_t launch_rhs_vjp_batch(const VjpMember* mem, const long long* tileStart, int nMem,
                                 long long totalTiles, int nop, hipStream_t st);

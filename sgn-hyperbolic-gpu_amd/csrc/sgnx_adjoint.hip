@@ -245,7 +245,7 @@ __device__ __forceinline__ void vjp_tile(ConstArgs<VjpMember> M, int tile) {
     const ConstArgs<VjpMember> P = opaque(M);
     return Phys{P->ph.g, P->ph.c, P->ph.gamma, 0.0, P->ph.halfg, P->ph.c2, P->ph.mc2, P->ph.m2c2};
   };
-  const int Nx = M->g.Nx, Ny = M->g.Ny, nStrips = M->nStrips, rows = M->g.vrows;
+  const int Nx = M->g.Nx, Ny = M->g.Ny, nStrips = M->nStrips, rows = M->g.vrows[NOP > 2];
   const int bcL = M->g.bc[0], bcR = M->g.bc[1];
   const bool wallB = M->g.bc[2] != SGNX_BC_PERIODIC, wallT = M->g.bc[3] != SGNX_BC_PERIODIC;
   const int chunk = __builtin_amdgcn_readfirstlane(tile / nStrips);
@@ -704,41 +704,43 @@ int vjp_strips(const Geometry& g) { return (g.Nx + kEW - 1) / kEW; }
 int vjp_nop(const VjpArgs& va) { return va.acc ? 3 : va.B ? 2 : 1; }
 }  // namespace
 
-long long vjp_tiles(const Geometry& g) {
-  return (long long)vjp_strips(g) * (((long long)g.Ny + g.vrows - 1) / g.vrows);
-}
-
 long long vjp_row_tiles(const Geometry& g) { return (long long)vjp_strips(g) * g.Ny; }
 
 // The lowest time by sweep_cost: per row a lone workgroup on a unit takes 2.8 us,
-// two, three and four together 3.6, 4.5 and 5.3 (a unit holds four); the rows
-// staged beside a chunk cost as much as its own.
-//   products of a step, us      rows: 2    4    7   10   16   32
-//    128 x   64                     74   71   85  105
-//    256 x  128                    207  183  167  169  203
-//   1024 x  512                   3070 2464 2254 2176 2085 2053
-int vjp_rows(const Geometry* const* g, int n, int cus) {
-  constexpr SweepPace pace{4, 2.0, 0.8, 2.0, 2.0};
+// two, three and four together 3.6, 4.4 and 5.2 (a unit holds four), of the third
+// product 3.2, 4.1 and 5.0 (three); the rows staged beside a chunk cost as much
+// as its own.
+//   first two products, us     rows: 2    3    4    7   10   16   32
+//    128 x   64                     44   46   46   65   73
+//    256 x  128                    126  115  112   99  107  130  199
+//   1024 x  512                   1800 1552 1426 1306 1271 1224 1224
+//   third product
+//    128 x   64                     30   27   25   36   40
+//    256 x  128                     81   71   70   68   62   74  111
+//   1024 x  512                   1269 1121 1038  948  906  854  829
+int vjp_rows(const Geometry* const* g, int n, int cus, bool third) {
+  constexpr SweepPace two{4, 2.0, 0.8, 2.0, 2.0}, last{3, 2.3, 0.9, 2.0, 2.0};
   cus = std::max(cus, 1);
   return choose_rows(32, [&](int r) {
     long long tiles = 0;
     for (int i = 0; i < n; ++i) tiles += (long long)vjp_strips(*g[i]) * ((g[i]->Ny + r - 1) / r);
-    return sweep_cost(tiles, r, cus, pace);
+    return sweep_cost(tiles, r, cus, third ? last : two);
   });
 }
 
 VjpMember vjp_member(const Geometry& g, const Phys& ph, const VjpArgs& va, GhostTime gt) {
-  return VjpMember{va, g, ph, gt, vjp_strips(g), (int)vjp_tiles(g)};
+  const long long rows = g.vrows[vjp_nop(va) > 2];
+  const int strips = vjp_strips(g);
+  return VjpMember{va, g, ph, gt, strips, (int)(strips * ((g.Ny + rows - 1) / rows))};
 }
 
 hipError_t launch_rhs_vjp(const Geometry& g, const Phys& ph, const VjpArgs& va, GhostTime gt,
                           hipStream_t st) {
-  const long long nb = vjp_tiles(g);
-  const int nop = vjp_nop(va);
-  if (nb > 0x7fffffffLL || (va.fresh && nop != 1) || va.out == va.A || va.out == va.B || (va.acc && !va.B))
-    return hipErrorInvalidValue;
   const VjpMember m = vjp_member(g, ph, va, gt);
-  const dim3 grid((unsigned)nb), block(kVT);
+  const int nop = vjp_nop(va);
+  if ((va.fresh && nop != 1) || va.out == va.A || va.out == va.B || (va.acc && !va.B))
+    return hipErrorInvalidValue;
+  const dim3 grid((unsigned)m.nTiles), block(kVT);
 #define SGNX_VJP(...) hipLaunchKernelGGL((k_vjp_sweep<__VA_ARGS__>), grid, block, 0, st, m)
   if (va.fresh) SGNX_VJP(1, true);
   else if (nop == 1) SGNX_VJP(1, false);

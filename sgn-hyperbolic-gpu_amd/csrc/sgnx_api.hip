@@ -217,7 +217,7 @@ int sgnx_create(const sgnx_desc* d, sgnx_solver** out) {
 
   CK(hipGetDevice(&s->device));
   CK(scratch_address(s->device, &s->scratch));
-  g.vrows = g.rows;
+  g.vrows[0] = g.vrows[1] = g.rows;
   s->rowsSet = std::getenv("SGNX_SWEEP_ROWS") != nullptr;
   if (!s->rowsSet) {
     // The RHS and the products do not depend on the heights; the adaptive
@@ -226,7 +226,7 @@ int sgnx_create(const sgnx_desc* d, sgnx_solver** out) {
     CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device));
     const Geometry* const one = &g;
     g.rows = sweep_rows(&one, 1, cus);
-    g.vrows = vjp_rows(&one, 1, cus);
+    for (int k = 0; k < 2; ++k) g.vrows[k] = vjp_rows(&one, 1, cus, k == 1);
   }
   const size_t Nd = (size_t)g.Nd, nst = (size_t)NV * Nd;
   const size_t nfx = (size_t)(d->Nx + 1) * d->Ny * NP, nfy = (size_t)d->Nx * (d->Ny + 1) * NP;

@@ -621,10 +621,12 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
     }
     return SGNX_OK;
   }
-  // one tile height for all members' products, unless set from outside
+  // the products' tile heights for all members, unless set from outside
   std::vector<const Geometry*> gs;
   for (int i = 0; i < n; ++i) gs.push_back(&b->m[i]->g);
-  const int vrows = std::getenv("SGNX_SWEEP_ROWS") ? 0 : vjp_rows(gs.data(), n, b->cus);
+  int vrows[2] = {0, 0};
+  if (!std::getenv("SGNX_SWEEP_ROWS"))
+    for (int k = 0; k < 2; ++k) vrows[k] = vjp_rows(gs.data(), n, b->cus, k == 1);
   std::vector<AdjTape*> tp(n, nullptr);
   std::vector<const double*> gb(n, nullptr);
   long Nmax = 0;
@@ -648,7 +650,8 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
   const size_t oV3 = up(oRT + (nn + 1) * sizeof(long long));
   const size_t oV2 = up(oV3 + nn * sizeof(VjpMember)), oV1 = up(oV2 + nn * sizeof(VjpMember));
   const size_t oVT = up(oV1 + nn * sizeof(VjpMember));
-  const size_t total = up(oVT + (nn + 1) * sizeof(long long));
+  const size_t oWT = up(oVT + (nn + 1) * sizeof(long long));   // the third product's offsets
+  const size_t total = up(oWT + (nn + 1) * sizeof(long long));
   if (b->adjCap < total) {
     if (b->h_adj) (void)hipHostFree(b->h_adj);
     if (b->d_adj) (void)hipFree(b->d_adj);
@@ -667,13 +670,14 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
   auto* hV2 = reinterpret_cast<VjpMember*>(b->h_adj + oV2);
   auto* hV1 = reinterpret_cast<VjpMember*>(b->h_adj + oV1);
   auto* hVT = reinterpret_cast<long long*>(b->h_adj + oVT);
+  auto* hWT = reinterpret_cast<long long*>(b->h_adj + oWT);
   auto dptr = [&](size_t off) { return b->d_adj + off; };
   std::vector<int> all(n);
   for (int i = 0; i < n; ++i) all[i] = i;
   const std::vector<int> times = row_multiples(b, all);
   for (long k = 0; k < Nmax; ++k) {
     int A = 0, Rn = 0;   // members in this step; of those, the ones that recompute stages
-    long long rAcc = 0, vAcc = 0;
+    long long rAcc = 0, vAcc = 0, wAcc = 0;
     for (int i = 0; i < n; ++i) {
       AdjTape* T = tp[i];
       const long m = (long)T->t.size() - 1 - k;
@@ -715,22 +719,24 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
       VjpArgs p[3];
       step_products(T, u, y2, y3, dt, T->thb, p);
       Geometry vg = s->g;
-      if (vrows) vg.vrows = vrows;
+      if (vrows[0]) std::memcpy(vg.vrows, vrows, sizeof vrows);
       hV3[A] = vjp_member(vg, s->ph, p[0], ghost_time(s, t + 0.75 * dt));
       hV2[A] = vjp_member(vg, s->ph, p[1], ghost_time(s, t + 0.5 * dt));
       hV1[A] = vjp_member(vg, s->ph, p[2], ghost_time(s, t));
       std::swap(T->lam, T->lamNew);   // (the tables hold this step's; the next reads its result)
       hVT[A] = vAcc;
-      vAcc += packed_tiles(vjp_tiles(vg));
+      hWT[A] = wAcc;
+      vAcc += packed_tiles(hV3[A].nTiles);
+      wAcc += packed_tiles(hV1[A].nTiles);
       ++A;
     }
     hRT[Rn] = rAcc;
     hVT[A] = vAcc;
+    hWT[A] = wAcc;
     BCHK(b, hipMemcpyAsync(b->d_adj, b->h_adj, total, hipMemcpyHostToDevice, b->stream));
     const auto* dR1 = reinterpret_cast<const BatchMember*>(dptr(oR1));
     const auto* dR2 = reinterpret_cast<const BatchMember*>(dptr(oR2));
     const auto* dRT = reinterpret_cast<const long long*>(dptr(oRT));
-    const auto* dVT = reinterpret_cast<const long long*>(dptr(oVT));
     BCHK(b, launch_gauge_bar_batch(reinterpret_cast<const GaugeMember*>(dptr(oG)), A, b->stream));
     if (Rn > 0) {
       BCHK(b, launch_rhs_stage_batch(dR1, dRT, Rn, rAcc, kPlain, b->waves3 & 1, b->stream, false,
@@ -738,10 +744,12 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
       BCHK(b, launch_rhs_stage_batch(dR2, dRT, Rn, rAcc, kAxpy, (b->waves3 >> 1) & 1, b->stream,
                                      true, batch_hxr(b)));
     }
-    int nop = 0;
-    for (size_t o : {oV3, oV2, oV1})
-      BCHK(b, launch_rhs_vjp_batch(reinterpret_cast<const VjpMember*>(dptr(o)), dVT, A, vAcc,
-                                   ++nop, b->stream));
+    const size_t oV[3] = {oV3, oV2, oV1};
+    for (int k = 0; k < 3; ++k)
+      BCHK(b, launch_rhs_vjp_batch(
+                  reinterpret_cast<const VjpMember*>(dptr(oV[k])),
+                  reinterpret_cast<const long long*>(dptr(k < 2 ? oVT : oWT)), A,
+                  k < 2 ? vAcc : wAcc, k + 1, b->stream));
     // the arena is refilled for the next iteration
     BCHK(b, hipStreamSynchronize(b->stream));
   }

@@ -96,7 +96,8 @@ struct Geometry {
   ConstDiv dx, dy;           // division by Jx, Jy
   int variant;               // RHS kernel: 0 element-row tiles, 1 row sweep
   int rows;                  // row sweep: element rows per workgroup (in a batch a multiple)
-  int vrows;                 // the adjoint's product: element rows per workgroup
+  int vrows[2];              // the adjoint's products: element rows per workgroup, of the
+                             // first two of a step and of the third
   int waves3;                // row sweep: bit m set = stage mode m built for 3 waves/SIMD
   int hxr;                   // Hx, Hy equal (D Hnod) / J bit for bit: the row sweep forms
                              // them from Hnod instead of reading them
