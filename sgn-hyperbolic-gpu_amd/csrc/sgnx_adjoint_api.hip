@@ -96,7 +96,6 @@ int bs3_fixed(sgnx_solver* s, const double* u, double* uNew, double t, double dt
     b.kc = s->d_k1;
     b.dt = dt;
     b.uNew = uNew;
-    b.zOut = s->d_k3;
     HIPCHK(s, launch_rhs_stage(s->g, s->ph, kCand, b, nullptr, ghost_time(s, t + 0.75 * dt),
                                s->stream));
   } else {
@@ -142,7 +141,7 @@ int step_adjoint(sgnx_solver* s, AdjTape* tp, const double* u, double t, double 
     a.yOut = y2;
     a.y3Out = y3;
     a.a3 = 0.75 * dt;
-    HIPCHK(s, launch_rhs_stage(s->g, s->ph, kAxpy, a, s->d_k2, ghost_time(s, t + 0.5 * dt),
+    HIPCHK(s, launch_rhs_stage(s->g, s->ph, kAxpy, a, nullptr, ghost_time(s, t + 0.5 * dt),
                                s->stream));
   } else {
     HIPCHK(s, launch_comb1(y2, u, 0.5 * dt, s->d_k1, n, s->stream));

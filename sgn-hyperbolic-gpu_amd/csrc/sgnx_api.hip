@@ -391,6 +391,7 @@ static int fused_bs3(sgnx_solver* s, double t, double dt, double atol, double rt
                      bool withErr) {
   BS3Launch L[3];
   bs3_launches(s, t, dt, atol, rtol, L);
+  if (!withErr && !L[1].sa.yOut) L[1].sa.zOut = nullptr;
   int rc;
   for (int k = 0; k < (withErr ? 3 : 2); ++k)
     if ((rc = rhs_launch(s, L[k].mode, L[k].sa, L[k].dU, L[k].t))) return rc;

@@ -711,7 +711,7 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
         s2.yOut = s->d_tmp;
         s2.y3Out = s->d_k3;
         s2.a3 = 0.75 * dt;
-        hR2[Rn] = member_args(s, u, s->d_k2, s2, t + 0.5 * dt, times[i]);
+        hR2[Rn] = member_args(s, u, nullptr, s2, t + 0.5 * dt, times[i]);
         hRT[Rn] = rAcc;
         rAcc += packed_tiles(hR1[Rn].nTiles);
         ++Rn;

@@ -130,7 +130,8 @@ struct Stage {
   const double* kc;   // kCand: k1 of the step
   double dt;          // kCand, kErr
   double* uNew;       // kCand: candidate out
-  double* zOut;       // kCand: partial embedded sum out
+  double* zOut;       // kCand: partial embedded sum out (null, in a launch that keeps
+                      // no input: a step without the norm)
   const double* u0;   // kErr: u of the step
   const double* z;    // kErr: partial embedded sum
   double atol, rtol;  // kErr
@@ -166,7 +167,8 @@ hipError_t launch_rhs(const Geometry& g, const Phys& ph, const double* U, double
 // dU = R(stage input) with the row-sweep kernel (kCand writes sa.uNew and
 // sa.zOut instead of dU; kErr also writes sa.part, 3 doubles per workgroup,
 // folded by launch_finish). kAxpy and kCand with sa.yOut set also write the
-// stage input they form (the batched form: keep = some member's yOut is set).
+// stage input they form (the batched form: keep = some member's yOut is set);
+// such a kAxpy launch may leave dU out (null).
 hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const Stage& sa,
                             double* dU, GhostTime gt, hipStream_t st);
 // out[0] = sum, out[1] = max of nb (sum, carry, max) partial triples, fixed order

@@ -355,18 +355,23 @@ struct Sweep {
   static_assert(2 * (NXI + NYI) <= NT, "two lanes per interface node");
 };
 
+// kCand of a step that takes no error norm: without the embedded sum (a build of
+// its own: a test of zOut in kCand costs the adaptive step's launch 0.5 %)
+constexpr int kCandOnly = 4;
+constexpr bool is_cand(int mode) { return mode == kCand || mode == kCandOnly; }
+
 // Operands of the stage input at one node (5 variables each): u, and the
 // increment k of u + a*k in the modes that have one.
 template <int MODE>
 struct StageRaw {
-  static constexpr bool kHasK = MODE == kAxpy || MODE == kCand;
+  static constexpr bool kHasK = MODE == kAxpy || is_cand(MODE);
   double u[NV], k[kHasK ? NV : 1];
 };
 // Per-node operands beyond the stage input: kCand: x0 = kc; kErr: x0 = u0,
 // x1 = z. Faces and halos never need them.
 template <int MODE>
 struct NodeExtra {
-  double x0[(MODE == kCand || MODE == kErr) ? NV : 1], x1[MODE == kErr ? NV : 1];
+  double x0[(is_cand(MODE) || MODE == kErr) ? NV : 1], x1[MODE == kErr ? NV : 1];
 };
 
 // The launch's arguments: its kernel's own, or one entry of a batch's table.
@@ -382,7 +387,7 @@ __device__ __forceinline__ void stage_load(SweepArgs A, size_t first, size_t pla
 template <int MODE>
 __device__ __forceinline__ void extra_load(SweepArgs A, size_t first, size_t plane, unsigned off,
                                            NodeExtra<MODE>& E) {
-  if (MODE == kCand || MODE == kErr) load_vars(MODE == kCand ? A->sa.kc : A->sa.u0, first, plane, off, E.x0);
+  if (is_cand(MODE) || MODE == kErr) load_vars(is_cand(MODE) ? A->sa.kc : A->sa.u0, first, plane, off, E.x0);
   if (MODE == kErr) load_vars(A->sa.z, first, plane, off, E.x1);
 }
 
@@ -808,12 +813,12 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
       const SweepArgs R = opaque(A);
       auto finish = [&](int v, double k4, size_t pl) {
         auto put = [&](double* base, double x) { store_at(global_at(base, pl), t8, x); };
-        if (MODE == kCand) {
+        if (is_cand(MODE)) {
           // rk.cpp:106-108 and the first three terms of :119-120 (k4 is k3 here)
           const double k1 = ext.x0[v], k2 = own.k[v];
           put(R->sa.uNew, own.u[v] + stDt * (2.0 / 9.0 * k1 + 1.0 / 3.0 * k2 + 4.0 / 9.0 * k4));
-          put(R->sa.zOut, 7.0 / 24.0 * k1 + 0.25 * k2 + 1.0 / 3.0 * k4);
-        } else {
+          if (MODE == kCand) put(R->sa.zOut, 7.0 / 24.0 * k1 + 0.25 * k2 + 1.0 / 3.0 * k4);
+        } else if (!(MODE == kAxpy && KEEP) || R->dU) {
           put(R->dU, k4);
         }
         if (MODE == kAxpy && KEEP && R->sa.y3Out) {
@@ -1313,12 +1318,14 @@ hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const S
   const BatchMember args = sweep_member(g, ph, sa.u, dU, gt, sa);
 #define SGNX_SWEEP(M, W, K) sweep_launch<M, W, K>(hxr, grid, block, st, args)
   const bool keep = sa.yOut != nullptr;
+  if (mode == kCand && keep && !sa.zOut) return hipErrorInvalidValue;
   if (mode == kPlain) { if (w3) SGNX_SWEEP(kPlain, 3, false); else SGNX_SWEEP(kPlain, 2, false); }
   else if (mode == kAxpy) {
     if (keep) { if (w3) SGNX_SWEEP(kAxpy, 3, true); else SGNX_SWEEP(kAxpy, 2, true); }
     else { if (w3) SGNX_SWEEP(kAxpy, 3, false); else SGNX_SWEEP(kAxpy, 2, false); }
   } else if (mode == kCand) {
     if (keep) { if (w3) SGNX_SWEEP(kCand, 3, true); else SGNX_SWEEP(kCand, 2, true); }
+    else if (!sa.zOut) { if (w3) SGNX_SWEEP(kCandOnly, 3, false); else SGNX_SWEEP(kCandOnly, 2, false); }
     else { if (w3) SGNX_SWEEP(kCand, 3, false); else SGNX_SWEEP(kCand, 2, false); }
   } else { if (w3) SGNX_SWEEP(kErr, 3, false); else SGNX_SWEEP(kErr, 2, false); }
 #undef SGNX_SWEEP
