@@ -465,7 +465,14 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
   const int nStrips = A->nStrips, rows = A->rows, Nx = A->g.Nx, Ny = A->g.Ny;
   __shared__ L lds;
 
-  if (threadIdx.x < NP) {
+  // The lane's rows of D and weights are kept in registers by the plain launch,
+  // which LDS reads bound (2000x1000 1302 -> 1256 us, 1024x512 350 -> 343); the
+  // stage launches wait for memory and gain nothing from that, but from fetching
+  // their first rows before anything else: the latency is then behind the rest of
+  // the preparation (387x191 stage 3 103.9 -> 102.5 us, 1024x512 635 -> 631). The
+  // plain launch, which waits for its tables, loses by it (8x6 6.14 -> 6.25 us).
+  constexpr bool kTabRegs = MODE == kPlain;
+  if (kTabRegs && threadIdx.x < NP) {
     const OpTables* const T = A->g.ops;
     double* const to = lds.tab[threadIdx.x];
 #pragma unroll
@@ -496,6 +503,55 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
   const int b = loc / NP, a = loc - NP * b;
   unsigned t8 = (unsigned)tn * 8u;                       // the node
   unsigned f8 = (unsigned)(j * NPP + a) * 8u;            // the bottom face of its column
+  const bool wallTop = bcT != 0;
+  // The nodes' operands, two rows ahead: while row r is worked on, row r + 1
+  // has landed (its bottom faces are the upper side of the y line between the
+  // two, so no lane loads a face a second time) and row r + 2 is in flight.
+  // Above the chunk only the bottom faces are needed (from the first row
+  // across a periodic top side), so every lane takes its column's; with
+  // nothing to load, row r's first nodes stand in.
+  struct Node {
+    StageRaw<MODE> s;
+    double H, Hx, Hy;
+    __device__ __forceinline__ void take(const Node& o) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        move_to(s.u[v], o.s.u[v]);
+        if (StageRaw<MODE>::kHasK) move_to(s.k[v], o.s.k[v]);
+      }
+      move_to(H, o.H);
+      if (!HXR) {
+        move_to(Hx, o.Hx);
+        move_to(Hy, o.Hy);
+      }
+    }
+  };
+  Node cur, nxt;
+  const unsigned row0 = (unsigned)ex0 * (NPP * 8u);
+  unsigned rowOff = row0 + (unsigned)ey0 * rowBytes;     // row r's first node (bytes)
+  auto node_load = [&](SweepArgs R, int r, int ahead, size_t plane, Node& n) {
+    int to = r + ahead;
+    const bool full = to < ey1;
+    to = to > ey1 ? r : to;
+    to = to == Ny ? (wallTop ? r : 0) : to;
+    const unsigned first =
+        __builtin_amdgcn_readfirstlane((int)(row0 + (unsigned)to * rowBytes));
+    const unsigned off = full ? t8 : f8;
+    stage_load<MODE>(R, first, plane, off, n.s);
+    n.H = load_at(global_at(R->g.Hnod, first), off);
+    if (!HXR) {
+      n.Hx = load_at(global_at(R->g.Hx, first), off);
+      n.Hy = load_at(global_at(R->g.Hy, first), off);
+    }
+  };
+  static_assert(offsetof(OpTables, gLp) == NPP * 8 && offsetof(OpTables, gRp) == (NPP + NP) * 8, "");
+  const int te = threadIdx.x < NPP + 2 * NP ? threadIdx.x : 0;   // a table entry per lane
+  double tabEntry = 0.0;
+  if (!kTabRegs) {
+    node_load(A, ey0, 0, plane0, cur);
+    node_load(A, ey0, 1, plane0, nxt);
+    tabEntry = ((const GlobalDouble*)A->g.ops)[te];
+  }
   // Interface half-items: two lanes per interface node, lane 2k + side
   // taking one side (0 = left / lower, 1 = right / upper) of interface k.
   // Items 0 .. nX - 1 are the x-interface nodes of the row (k = i NP + bb:
@@ -518,7 +574,6 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
   const bool gX = outer && (side == 0 ? ex0 > 0 || bcL == 0 : ex0 + nW < Nx || bcR == 0);
   const bool gY = isY && side == 1;
   const bool inflow = outer && side == 0 && ex0 == 0 && bcL == 2;
-  const bool wallTop = bcT != 0;
   int src;
   if (isX) {
     const int col = outer ? (side == 0 ? 0 : nW - 1) : (side == 0 ? xi - 1 : xi);
@@ -593,49 +648,14 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
     fH = *pHf;
   };
 
-  // The nodes' operands, two rows ahead: while row r is worked on, row r + 1
-  // has landed (its bottom faces are the upper side of the y line between the
-  // two, so no lane loads a face a second time) and row r + 2 is in flight.
-  // Above the chunk only the bottom faces are needed (from the first row
-  // across a periodic top side), so every lane takes its column's; with
-  // nothing to load, row r's first nodes stand in.
-  struct Node {
-    StageRaw<MODE> s;
-    double H, Hx, Hy;
-    __device__ __forceinline__ void take(const Node& o) {
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        move_to(s.u[v], o.s.u[v]);
-        if (StageRaw<MODE>::kHasK) move_to(s.k[v], o.s.k[v]);
-      }
-      move_to(H, o.H);
-      if (!HXR) {
-        move_to(Hx, o.Hx);
-        move_to(Hy, o.Hy);
-      }
-    }
-  };
-  Node cur, nxt;
-  const unsigned row0 = (unsigned)ex0 * (NPP * 8u);
-  unsigned rowOff = row0 + (unsigned)ey0 * rowBytes;     // row r's first node (bytes)
-  auto node_load = [&](SweepArgs R, int r, int ahead, size_t plane, Node& n) {
-    int to = r + ahead;
-    const bool full = to < ey1;
-    to = to > ey1 ? r : to;
-    to = to == Ny ? (wallTop ? r : 0) : to;
-    const unsigned first =
-        __builtin_amdgcn_readfirstlane((int)(row0 + (unsigned)to * rowBytes));
-    const unsigned off = full ? t8 : f8;
-    stage_load<MODE>(R, first, plane, off, n.s);
-    n.H = load_at(global_at(R->g.Hnod, first), off);
-    if (!HXR) {
-      n.Hx = load_at(global_at(R->g.Hx, first), off);
-      n.Hy = load_at(global_at(R->g.Hy, first), off);
-    }
-  };
-  node_load(A, ey0, 0, plane0, cur);
-  node_load(A, ey0, 1, plane0, nxt);
+  if (kTabRegs) {
+    node_load(A, ey0, 0, plane0, cur);
+    node_load(A, ey0, 1, plane0, nxt);
+  }
   face_load(A, plane0);
+  if (!kTabRegs)
+    (&lds.tab[0][0])[te < NPP ? te / NP * (NP + 2) + te % NP
+                              : (te - NPP) % NP * (NP + 2) + NP + (te - NPP) / NP] = tabEntry;
   // the y line at the bottom of the chunk, both sides from global memory (the
   // bottom wall's ghost mirrors the upper side)
   if (isY) {
@@ -666,10 +686,7 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
   LdsDouble* sTa = (LdsDouble*)lds.tab[a];
   LdsDouble* sTb = (LdsDouble*)lds.tab[b];
 
-  // The lane's rows of D and weights: kept in registers by the plain launch,
-  // which LDS reads bound (2000x1000 1302 -> 1256 us, 1024x512 350 -> 343); the
-  // stage launches wait for memory and gain nothing.
-  constexpr bool kTabRegs = MODE == kPlain;
+  // the lane's rows of D and weights
   double Da[NP], Db[NP], gLa, gRa, gLb, gRb;
   auto load_tab = [&](auto* ta, auto* tb) {
 #pragma unroll
