@@ -120,7 +120,7 @@ def profile_rhs(args):
 
 
 def profile_vjp(args):
-    """RHS vector-Jacobian products (k_vjp_coef + k_vjp_elem) on device-resident
+    """RHS vector-Jacobian products (k_vjp_sweep) on device-resident
     buffers of the shoal state, with the theta cotangent, then one reverse sweep
     of --profile-steps taped steps."""
     import numpy as np

@@ -143,10 +143,11 @@ int sgnx_bathymetry(const sgnx_solver* s, double* Hx, double* Hy);
 
 /* RHS kernel choice (tuning, no counterpart in the reference): variant 0 =
  * one workgroup per 5-element row tile, 1 = row sweep over a strip of 5
- * element columns and `rows` element rows per workgroup (default 1, rows 16,
- * or fewer on grids too small to give every compute unit three workgroups;
- * the environment variables SGNX_RHS_VARIANT / SGNX_SWEEP_ROWS set the
- * defaults at creation). Both are bitwise equal to the reference rhs(). The
+ * element columns and `rows` element rows per workgroup (default 1, rows 1 to
+ * 24 by the grid's size and the number of compute units; in a batch small
+ * members take multiples of their default; the environment variables
+ * SGNX_RHS_VARIANT / SGNX_SWEEP_ROWS set the defaults at creation, the latter
+ * for the adjoint's products too). Both are bitwise equal to the reference rhs(). The
  * row sweep has no Manning friction term: a solver with nManning != 0 uses
  * variant 0 (variant 1 then gives SGNX_EUNSUPPORTED, and such a solver
  * cannot join a batch or be autotuned). */

@@ -2,12 +2,11 @@
 // sgnx_batch.hip -- many independent solvers of uneven sizes advanced together.
 //
 // Every RHS launch of an adaptive step covers all running members: the
-// row-sweep workgroups of every member are packed back to back (a per-member
-// tile offset table) into one launch per stage kind, followed by one launch
-// that folds each member's error partials. Each member keeps its own state
-// buffers, time, step size and controller (the same RkCtl as sgnx_integrate)
-// and its own tile decomposition, so its results are bit for bit those of
-// sgnx_integrate on it alone. The reference's counterpart is a parameter sweep
+// row-sweep workgroups of every member follow each other (a per-member offset
+// table) in one launch per stage kind, followed by one launch that folds each
+// member's error partials. Each member keeps its own state buffers, time, step
+// size and controller (the same RkCtl as sgnx_integrate) and its own error
+// partials, so its results are bit for bit those of sgnx_integrate on it alone. The reference's counterpart is a parameter sweep
 // run as separate jobs (scripts/shoal_sweep.sbatch).
 //
 // Members recording an adjoint tape (sgnx_tape_begin) record it here as in
@@ -15,10 +14,10 @@
 // accepted steps after it.
 //
 // A step is: member arguments (pinned host -> device), three stage launches,
-// the fold, the (sum, max) pairs (device -> pinned host), one synchronisation;
-// optionally captured once into a hipGraph and replayed while the set of
-// running members is unchanged (the copies read and write the same pinned
-// buffers, which the host refills before each replay).
+// the fold, which posts the (sum, max) pairs to mapped host memory; optionally
+// captured once into a hipGraph and replayed while the set of running members
+// is unchanged (the copy reads the same pinned buffer, which the host refills
+// before each replay).
 // =============================================================================
 
 #include <hip/hip_runtime.h>

@@ -29,8 +29,8 @@ struct OpTables {
 // Element columns per RHS tile / row-sweep strip. Five columns make a
 // 128-work-item workgroup (125 node items, two waves), so a compute unit holds
 // four workgroups of the stage-3 build (190 registers) and six of the others
-// (130 to 168). Ten columns (256 work-items) ran stage 3 2 to 4 % faster and
-// the plain launch 4 % slower; seven, 11 % slower.
+// (136 to 168). Ten columns (256 work-items) ran stage 3 1 % faster at 1024x512
+// and 2000x1000 and everything else 1 to 10 % slower; eight, 10 to 30 % slower.
 constexpr int kStripW = 5;
 
 // The waves mask of SGNX_SWEEP_WAVES3 (host): 0x-prefixed hexadecimal or

@@ -339,14 +339,16 @@ k_rhs(const double* __restrict__ U, double* __restrict__ dU, Geometry g, Phys ph
 // Every y-interface is evaluated once; the stage input is read once per chunk,
 // plus the faces of the rows below and above the chunk and the x-halo nodes.
 //
-// What bounds it: the stage launches, their traffic (stage 3 moves 3.1 to 3.2
-// GB at 1024x512, 4.9 TB/s, the rate of a large copy); the plain launch, the
-// instructions and latencies of the row (about 500 vector and 80 LDS
-// instructions per wave and row, three waves per SIMD). Hence no branch around
-// a global access, no face loaded twice, quotients without a branch each, and
-// no vector instruction spent on an address. On 1024x512, per launch, before
+// What bounds it: the stage launches, their traffic (at 1024x512 stage 2 moves
+// 2.3 GB, stage 3 3.3, k4 2.6, all at 5.1 to 5.25 TB/s; a large copy reaches
+// 4.8); the plain launch, vector and LDS instructions (each 70 % busy: 640 and 80
+// per wave and row, three waves per SIMD); small grids, a workgroup's pace (2.7
+// to 3.2 us a row alone on its compute unit, 6 us around them). Hence no branch
+// around a global access, no face loaded twice, quotients without a branch each,
+// and no vector instruction spent on an address. On 1024x512, per launch, before
 // and after these (one MI355X, both builds in turn): plain 0.409 -> 0.348 ms,
-// stage 2 0.549 -> 0.436, stage 3 0.725 -> 0.640, k4 0.628 -> 0.505.
+// stage 2 0.549 -> 0.436, stage 3 0.725 -> 0.640, k4 0.628 -> 0.505; with what
+// is noted further down 0.340, 0.435, 0.631 and 0.496.
 template <int TW>
 struct Sweep {
   static constexpr int NT = ((NPP * TW + 63) / 64) * 64;
