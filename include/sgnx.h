@@ -144,10 +144,11 @@ int sgnx_bathymetry(const sgnx_solver* s, double* Hx, double* Hy);
 /* RHS kernel choice (tuning, no counterpart in the reference): variant 0 =
  * one workgroup per 5-element row tile, 1 = row sweep over a strip of 5
  * element columns and `rows` element rows per workgroup (default 1, rows 1 to
- * 24 by the grid's size and the number of compute units; in a batch small
- * members take multiples of their default; the environment variables
- * SGNX_RHS_VARIANT / SGNX_SWEEP_ROWS set the defaults at creation, the latter
- * for the adjoint's products too). Both are bitwise equal to the reference rhs(). The
+ * 24 by the grid's size and the number of compute units; with the default
+ * height the first workgroups of a larger grid take three or four times as
+ * many, and in a batch small members multiples of theirs; the environment
+ * variables SGNX_RHS_VARIANT / SGNX_SWEEP_ROWS set the defaults at creation,
+ * the latter for the adjoint's products too). Both are bitwise equal to the reference rhs(). The
  * row sweep has no Manning friction term: a solver with nManning != 0 uses
  * variant 0 (variant 1 then gives SGNX_EUNSUPPORTED, and such a solver
  * cannot join a batch or be autotuned). */
@@ -241,7 +242,8 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
 
 /* Autotuning (no counterpart in the reference): times every launch kind of an
  * adaptive step on the resident state for each candidate tile height (element
- * rows per workgroup: 2, 4, 8, 12, 16, 24, 32, up to Ny) and each build
+ * rows per workgroup: 2, 4, 8, 12, 16, 24, 32, up to Ny, and a larger grid's
+ * default with its taller first workgroups) and each build
  * (two or three waves per SIMD), keeps the fastest, and sets it (row-sweep
  * kernel; reps = launches timed per candidate). Only scratch stage buffers are
  * written; U and k1 are untouched. The tile height fixes the summation order

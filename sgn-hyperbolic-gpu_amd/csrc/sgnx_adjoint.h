@@ -14,8 +14,8 @@ namespace sgnx {
 
 // W = ca*A (+ cb*B when B is given); out = (dR/dU (U))^T W, or, when acc is
 // given (with B), ((A + acc) + B) + that; thetaBar += (dR/dtheta)^T W (when not
-// null; set to 0 + that where `fresh`, which takes A only). 5*Nd arrays; out is none of the inputs (a workgroup reads its
-// neighbours' A and B).
+// null; set to 0 + that where `fresh`, which takes A only). 5*Nd arrays; out is
+// none of the inputs (a workgroup reads its neighbours' A and B).
 struct VjpArgs {
   const double* U;
   const double* A;

@@ -226,6 +226,9 @@ int sgnx_create(const sgnx_desc* d, sgnx_solver** out) {
     CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device));
     const Geometry* const one = &g;
     g.rows = sweep_rows(&one, 1, cus);
+    g.tall = sweep_tall(g, cus, &g.rows);
+    s->ownRows = g.rows;
+    s->ownTall = g.tall;
     for (int k = 0; k < 2; ++k) g.vrows[k] = vjp_rows(&one, 1, cus, k == 1);
   }
   const size_t Nd = (size_t)g.Nd, nst = (size_t)NV * Nd;
@@ -663,7 +666,7 @@ int sgnx_set_rhs_kernel(sgnx_solver* s, int variant, int rows) {
   if (variant == 1 && s->ph.nManning != 0.0)
     return fail(s, SGNX_EUNSUPPORTED, "the row sweep has no Manning friction term (variant 0 has)");
   s->g.variant = variant;
-  s->g.rows = rows;
+  take_rows(s, rows);
   s->rowsSet = true;
   return SGNX_OK;
 }

@@ -26,6 +26,7 @@
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
+#include <iterator>
 #include <string>
 #include <vector>
 
@@ -459,9 +460,11 @@ int sgnx_autotune(sgnx_solver* s, int reps, int* rows_out, int* waves3_out) {
   };
   double best = 1e300;
   int bestRows = keep.rows, bestMask = keep.waves3;
-  for (int rows : kTuneRows) {
+  std::vector<int> heights(std::begin(kTuneRows), std::end(kTuneRows));
+  if (s->ownTall > 1) heights.push_back(s->ownRows);
+  for (int rows : heights) {
     if (rows > s->g.Ny && rows != kTuneRows[0]) continue;
-    s->g.rows = rows;
+    take_rows(s, rows);
     bs3_launches(s, 0.0, kProbeDt, 1.0, 0.0, L);
     double tot = 0.0;
     int mask = 0;
@@ -481,7 +484,7 @@ int sgnx_autotune(sgnx_solver* s, int reps, int* rows_out, int* waves3_out) {
       bestMask = mask;
     }
   }
-  s->g.rows = bestRows;
+  take_rows(s, bestRows);
   s->rowsSet = true;
   float p2 = 0.0f, p3 = 0.0f;
   if (timed(0, false, &p2) != hipSuccess || timed(0, true, &p3) != hipSuccess) {
@@ -565,7 +568,7 @@ int sgnx_batch_autotune(sgnx_batch* b, int reps, int* rows_out, int* waves3_out)
     }
   }
   for (sgnx_solver* s : b->m) {
-    s->g.rows = bestRows;
+    take_rows(s, bestRows);
     s->rowsSet = true;
   }
   const long long total = fill();

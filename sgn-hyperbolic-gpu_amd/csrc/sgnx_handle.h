@@ -22,6 +22,7 @@ struct sgnx_solver {
   double Lx = 0.0, Ly = 0.0, hx = 0.0, hy = 0.0;
   Geometry g{};
   bool rowsSet = false;      // g.rows set from outside or by an autotuner, not by the rule
+  int ownRows = 0, ownTall = 1;   // what the rule gives this grid
   Phys ph{};
   hipStream_t stream = nullptr;
   int device = 0;
@@ -98,6 +99,13 @@ inline GhostTime ghost_time(const sgnx_solver* s, double t) {
     gt.c = std::cos(s->inflowOmega * t);
   }
   return gt;
+}
+
+// A height for all tiles; the one that the rule gives the grid brings its tall
+// tiles too (the results are the same bits).
+inline void take_rows(sgnx_solver* s, int rows) {
+  s->g.rows = rows;
+  s->g.tall = rows == s->ownRows ? s->ownTall : 1;
 }
 
 // The three row-sweep launches of one BS3 attempt (rk.cpp:99-131) on a

@@ -96,6 +96,7 @@ struct Geometry {
   ConstDiv dx, dy;           // division by Jx, Jy
   int variant;               // RHS kernel: 0 element-row tiles, 1 row sweep
   int rows;                  // row sweep: element rows per workgroup (in a batch a multiple)
+  int tall;                  // its first tiles take tall * rows (launches by themselves; 0, 1: none)
   int vrows[2];              // the adjoint's products: element rows per workgroup, of the
                              // first two of a step and of the third
   int waves3;                // row sweep: bit m set = stage mode m built for 3 waves/SIMD
@@ -157,6 +158,7 @@ struct BatchMember {
   int nStrips;
   int nTiles;
   int parts;
+  int tall, tallTiles;   // element rows and number of the tall tiles, which come first
 };
 
 // ---- launchers (sgnx_kernels.hip); all asynchronous on `st` ----------------
@@ -193,6 +195,9 @@ long long sweep_tiles(const Geometry& g);
 // operands and decomposition of a launch whose workgroups take times * g.rows rows
 BatchMember sweep_member(const Geometry& g, const Phys& ph, const double* U, double* dU,
                          GhostTime gt, const Stage& sa, int times = 1);
+// tall and low tiles for a launch of g by itself: the multiple, and the low
+// height in *rows (1: one height, *rows as it was)
+int sweep_tall(const Geometry& g, int cus, int* rows);
 // element rows per workgroup for the grids of one launch
 int sweep_rows(const Geometry* const* g, int n, int cus);
 // Hx, Hy = (D . Hnod) / J per element line (sgn2d.cpp:54-71)

@@ -454,7 +454,7 @@ struct SweepLds {
 // One workgroup's strip x chunk `tile` of one grid (the body of the plain and
 // the batched launches).
 template <int TW, int MODE, int WAVES, bool KEEP = false, bool HXR = false>
-__device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
+__device__ __forceinline__ void sweep_tile(SweepArgs A, int tile, int rows, int base) {
   using L = SweepLds<TW, HXR>;
   constexpr int kRec = L::kRec, kJ = L::kJ, kJSide = L::kJSide, kJLine = L::kJLine;
   // the row sweep runs without the Manning friction term (the launchers
@@ -464,7 +464,7 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
   const ConstDiv divX{A->g.dx.b, A->g.dx.rh, A->g.dx.rl, 1}, divY{A->g.dy.b, A->g.dy.rh, A->g.dy.rl, 1};
   const double stA = A->sa.a, stDt = A->sa.dt, atol = A->sa.atol, rtol = A->sa.rtol;
   const int bcL = A->g.bc[0], bcR = A->g.bc[1], bcB = A->g.bc[2], bcT = A->g.bc[3];
-  const int nStrips = A->nStrips, rows = A->rows, Nx = A->g.Nx, Ny = A->g.Ny;
+  const int nStrips = A->nStrips, Nx = A->g.Nx, Ny = A->g.Ny;
   __shared__ L lds;
 
   // The lane's rows of D and weights are kept in registers by the plain launch,
@@ -486,7 +486,7 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
   const int chunk = __builtin_amdgcn_readfirstlane(tile / nStrips);
   const int strip = tile - chunk * nStrips, ex0 = strip * TW;
   const int nW = min(TW, Nx - ex0);
-  const int ey0 = chunk * rows;
+  const int ey0 = base + chunk * rows;
   const int ey1 = min(Ny, ey0 + rows);
   const int nNodes = NPP * nW;
   const int t = threadIdx.x;
@@ -943,9 +943,13 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile) {
 // The arguments are the kernel's only parameter, read where they lie.
 template <int TW, int MODE, int WAVES, bool KEEP = false, bool HXR = false>
 __global__ void __launch_bounds__(Sweep<TW>::NT, WAVES) k_rhs_sweep(BatchMember) {
+  const SweepArgs A = (SweepArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  const int b = blockIdx.x, tall = A->tallTiles, low = (tall + kXcd - 1) / kXcd * kXcd;
+  if (b >= tall && b < low) return;          // (filling up)
+  const bool isTall = b < tall;
   sweep_tile<TW, MODE, WAVES, KEEP, HXR>(
-      (SweepArgs)__builtin_amdgcn_kernarg_segment_ptr(),
-      xcd_tile(blockIdx.x, gridDim.x));
+      A, isTall ? xcd_tile(b, tall) : xcd_tile(b - low, A->nTiles - tall),
+      isTall ? A->tall : A->rows, isTall ? 0 : A->tall * (tall / A->nStrips));
 }
 
 // Many grids in one launch: the workgroups of every member's tiles, one member
@@ -965,7 +969,7 @@ k_rhs_sweep_batch(const BatchMember* __restrict__ mem, const long long* __restri
   const SweepArgs M = const_entry(mem, lo);
   const int own = __builtin_amdgcn_readfirstlane((int)(w - tileStart[lo]));
   if (own >= M->nTiles) return;               // (filling up)
-  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(M, xcd_tile(own, M->nTiles));
+  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(M, xcd_tile(own, M->nTiles), M->rows, 0);
 }
 
 // Hx, Hy at every node (sgn2d.cpp:54-71).
@@ -1324,17 +1328,50 @@ void sweep_launch_batch(bool hxr, dim3 grid, dim3 block, hipStream_t st, const B
 
 }  // namespace
 
+// A launch of a grid by itself takes its rows in tall tiles first and the last
+// kLowTiles or so in low ones (g.rows high): tall tiles start and load their
+// borders less often, low ones even out the end. Tall and low heights against
+// one height, us:
+//   387 x 191   9, 3 against 5    plain 59.6 -> 58.2   76.0 -> 72.6   100.8 -> 96.5   86.4 -> 80.4
+//   603 x 301  12, 4 against 8         135.0 -> 129.0 170.4 -> 166.6  228.7 -> 226.9 192.1 -> 193.4
+//  1024 x 512  12, 4 against 8         341.9 -> 330.0 440.0 -> 426.2  635.6 -> 628.6 498.7 -> 493.7
+//  2000 x 1000 16, 4 against 18         1239 -> 1221   1607 -> 1588    2396 -> 2376   1887 -> 1858
+// (1024 x 512 at 16, 4: 333, 427, 630, 502; 2000 x 1000 at 12, 4: 1234, 1620, 2391,
+// 1871.) A grid that has not 1.6 sets of four workgroups per compute unit at 6
+// rows takes one height (sweep_rows).
+constexpr int kLowTiles = 1280;
+int sweep_tall(const Geometry& g, int cus, int* rows) {
+  const long long strips = (g.Nx + kTileW - 1) / kTileW, unit = 4LL * std::max(cus, 1);
+  constexpr struct { int tall, rows; double sets; } kHeights[] = {
+      {16, 4, 12.0}, {12, 4, 1.6}, {9, 3, 1.6}, {6, 2, 1.6}};
+  for (const auto& h : kHeights) {
+    if (strips * ((g.Ny + h.tall - 1) / h.tall) < h.sets * unit) continue;
+    *rows = h.rows;
+    return h.tall / h.rows;
+  }
+  return 1;
+}
+
 hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const Stage& sa,
                             double* dU, GhostTime gt, hipStream_t st) {
-  const long long tiles = sweep_tiles(g);
-  if (tiles > 0x7fffffffLL || g.rows < 1) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)tiles), block(Sweep<kTileW>::NT);
+  if (sweep_tiles(g) > 0x7fffffffLL || g.rows < 1) return hipErrorInvalidValue;
+  BatchMember args = sweep_member(g, ph, sa.u, dU, gt, sa);
+  int low = 0;                               // workgroups of the tall tiles, filled up
+  if (g.tall > 1) {
+    const int strips = args.nStrips, lowChunks = (kLowTiles + strips - 1) / strips;
+    args.tall = g.tall * g.rows;
+    const int tallChunks = std::max(0, (g.Ny - lowChunks * g.rows) / args.tall);
+    const int left = g.Ny - tallChunks * args.tall;
+    args.tallTiles = tallChunks * strips;
+    args.nTiles = args.tallTiles + strips * ((left + g.rows - 1) / g.rows);
+    low = (int)packed_tiles(args.tallTiles);
+  }
+  const dim3 grid((unsigned)(low + args.nTiles - args.tallTiles)), block(Sweep<kTileW>::NT);
   // waves per SIMD the register allocation targets, per stage mode (bit m of
   // g.waves3 set: 3 waves, else 2)
   const bool w3 = (g.waves3 >> mode) & 1;
   if (mode < kPlain || mode > kErr || ph.nManning != 0.0) return hipErrorInvalidValue;
   const bool hxr = g.hxr != 0;   // Hx, Hy formed from Hnod
-  const BatchMember args = sweep_member(g, ph, sa.u, dU, gt, sa);
 #define SGNX_SWEEP(M, W, K) sweep_launch<M, W, K>(hxr, grid, block, st, args)
   const bool keep = sa.yOut != nullptr;
   if (mode == kCand && keep && !sa.zOut) return hipErrorInvalidValue;
@@ -1353,7 +1390,7 @@ hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const S
 
 BatchMember sweep_member(const Geometry& g, const Phys& ph, const double* U, double* dU,
                          GhostTime gt, const Stage& sa, int times) {
-  BatchMember m{U, dU, g, ph, gt, sa, times * g.rows, (g.Nx + kTileW - 1) / kTileW, 0, 0};
+  BatchMember m{U, dU, g, ph, gt, sa, times * g.rows, (g.Nx + kTileW - 1) / kTileW, 0, 0, 0, 0};
   m.nTiles = (int)(m.nStrips * (((long long)g.Ny + m.rows - 1) / m.rows));
   m.parts = (int)sweep_tiles(g);
   return m;
@@ -1367,7 +1404,7 @@ BatchMember sweep_member(const Geometry& g, const Phys& ph, const double* U, dou
 //   256 x 128  38 47 58 49  34 41 50 43  33 40 55 42  35 40 43 43  38 43 46 47  50 55 58 61  63 68 72 76
 //   387 x 191 73 104 145 109 63 87 118 92 60 77 105 88 66 82 108 89 72 86 100 96 65 78 109 88 71 85 100 96
 //   603 x 301 (all four) 1033  833  734  728  735  786  770;  1024 x 512  -  -  -  -  1932 1943 1951
-// It takes 2, 7, 5, 8 and 8 rows there.
+// It takes 2, 7, 5, 8 and 8 rows there (launches by themselves: sweep_tall).
 int sweep_rows(const Geometry* const* g, int n, int cus) {
   constexpr SweepPace six{6, 2.5, 0.5, 0.5, 1.8}, four{4, 2.6, 0.65, 0.5, 1.6};
   cus = std::max(cus, 1);
