@@ -158,7 +158,9 @@ struct BatchMember {
   int nStrips;
   int nTiles;
   int parts;
-  int tall, tallTiles;   // element rows and number of the tall tiles, which come first
+  // the tall tiles, which come first: their element rows and number, the
+  // workgroups they take up, and the low ones' number and first row
+  int tall, tallTiles, tallBlocks, lowTiles, lowFrom;
 };
 
 // ---- launchers (sgnx_kernels.hip); all asynchronous on `st` ----------------

@@ -944,12 +944,15 @@ __device__ __forceinline__ void sweep_tile(SweepArgs A, int tile, int rows, int 
 template <int TW, int MODE, int WAVES, bool KEEP = false, bool HXR = false>
 __global__ void __launch_bounds__(Sweep<TW>::NT, WAVES) k_rhs_sweep(BatchMember) {
   const SweepArgs A = (SweepArgs)__builtin_amdgcn_kernarg_segment_ptr();
-  const int b = blockIdx.x, tall = A->tallTiles, low = (tall + kXcd - 1) / kXcd * kXcd;
-  if (b >= tall && b < low) return;          // (filling up)
-  const bool isTall = b < tall;
-  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(
-      A, isTall ? xcd_tile(b, tall) : xcd_tile(b - low, A->nTiles - tall),
-      isTall ? A->tall : A->rows, isTall ? 0 : A->tall * (tall / A->nStrips));
+  const int b = blockIdx.x, low = b - A->tallBlocks;
+  int tile = xcd_tile(low, A->lowTiles), rows = A->rows, base = A->lowFrom;
+  if (low < 0) {
+    if (b >= A->tallTiles) return;           // (filling up)
+    tile = xcd_tile(b, A->tallTiles);
+    rows = A->tall;
+    base = 0;
+  }
+  sweep_tile<TW, MODE, WAVES, KEEP, HXR>(A, tile, rows, base);
 }
 
 // Many grids in one launch: the workgroups of every member's tiles, one member
@@ -1356,17 +1359,18 @@ hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const S
                             double* dU, GhostTime gt, hipStream_t st) {
   if (sweep_tiles(g) > 0x7fffffffLL || g.rows < 1) return hipErrorInvalidValue;
   BatchMember args = sweep_member(g, ph, sa.u, dU, gt, sa);
-  int low = 0;                               // workgroups of the tall tiles, filled up
+  args.lowTiles = args.nTiles;
   if (g.tall > 1) {
     const int strips = args.nStrips, lowChunks = (kLowTiles + strips - 1) / strips;
     args.tall = g.tall * g.rows;
     const int tallChunks = std::max(0, (g.Ny - lowChunks * g.rows) / args.tall);
-    const int left = g.Ny - tallChunks * args.tall;
+    args.lowFrom = tallChunks * args.tall;
     args.tallTiles = tallChunks * strips;
-    args.nTiles = args.tallTiles + strips * ((left + g.rows - 1) / g.rows);
-    low = (int)packed_tiles(args.tallTiles);
+    args.tallBlocks = (int)packed_tiles(args.tallTiles);
+    args.lowTiles = strips * ((g.Ny - args.lowFrom + g.rows - 1) / g.rows);
+    args.nTiles = args.tallTiles + args.lowTiles;
   }
-  const dim3 grid((unsigned)(low + args.nTiles - args.tallTiles)), block(Sweep<kTileW>::NT);
+  const dim3 grid((unsigned)(args.tallBlocks + args.lowTiles)), block(Sweep<kTileW>::NT);
   // waves per SIMD the register allocation targets, per stage mode (bit m of
   // g.waves3 set: 3 waves, else 2)
   const bool w3 = (g.waves3 >> mode) & 1;
@@ -1390,7 +1394,7 @@ hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const S
 
 BatchMember sweep_member(const Geometry& g, const Phys& ph, const double* U, double* dU,
                          GhostTime gt, const Stage& sa, int times) {
-  BatchMember m{U, dU, g, ph, gt, sa, times * g.rows, (g.Nx + kTileW - 1) / kTileW, 0, 0, 0, 0};
+  BatchMember m{U, dU, g, ph, gt, sa, times * g.rows, (g.Nx + kTileW - 1) / kTileW, 0, 0, 0, 0, 0, 0, 0};
   m.nTiles = (int)(m.nStrips * (((long long)g.Ny + m.rows - 1) / m.rows));
   m.parts = (int)sweep_tiles(g);
   return m;
