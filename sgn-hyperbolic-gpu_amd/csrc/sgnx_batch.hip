@@ -6,8 +6,9 @@
 // table) in one launch per stage kind, followed by one launch that folds each
 // member's error partials. Each member keeps its own state buffers, time, step
 // size and controller (the same RkCtl as sgnx_integrate) and its own error
-// partials, so its results are bit for bit those of sgnx_integrate on it alone. The reference's counterpart is a parameter sweep
-// run as separate jobs (scripts/shoal_sweep.sbatch).
+// partials, so its results are bit for bit those of sgnx_integrate on it
+// alone. The reference's counterpart is a parameter sweep run as separate jobs
+// (scripts/shoal_sweep.sbatch).
 //
 // Members recording an adjoint tape (sgnx_tape_begin) record it here as in
 // sgnx_integrate: snapshot copies on the batch stream ahead of a step, the
