@@ -1304,7 +1304,7 @@ constexpr int kTileW = kStripW;   // elements per RHS tile / sweep strip
 
 long long sweep_tiles(const Geometry& g) {
   const long long strips = (g.Nx + kTileW - 1) / kTileW;
-  const long long chunks = (g.Ny + g.rows - 1) / g.rows;
+  const long long chunks = ((long long)g.Ny + g.rows - 1) / g.rows;   // (rows up to 2^31 - 1)
   return strips * chunks;
 }
 
