@@ -1341,14 +1341,28 @@ void sweep_launch_batch(bool hxr, dim3 grid, dim3 block, hipStream_t st, const B
 //  2000 x 1000 16, 4 against 18         1239 -> 1221   1607 -> 1588    2396 -> 2376   1887 -> 1858
 // (1024 x 512 at 16, 4: 333, 427, 630, 502; 2000 x 1000 at 12, 4: 1234, 1620, 2391,
 // 1871.) A grid that has not 1.6 sets of four workgroups per compute unit at 6
-// rows takes one height (sweep_rows).
+// rows takes one height (sweep_rows), and so does a flat one: the rows that a
+// strip has left beside its tall tiles all go into low ones, which costs more than
+// their even end gives where there is no tall tile, or, with two sets of strips or
+// more, not four of them. The plain launch and a step's three, one height against
+// tall and low:
+//    8201 x 16   104  435, 12, 4: 105  434      14800 x 13   147  600,  9, 3: 160  662
+//   20000 x 11   164  673,  6, 2: 188  774      61440 x 11   488 1987,  6, 2: 548 2424
 constexpr int kLowTiles = 1280;
+
+// chunks of `tall` rows above which the rest of the rows makes the low tiles
+int tall_chunks(const Geometry& g, int strips, int tall, int rows) {
+  const int lowChunks = (kLowTiles + strips - 1) / strips;
+  return std::max(0, (g.Ny - lowChunks * rows) / tall);
+}
+
 int sweep_tall(const Geometry& g, int cus, int* rows) {
   const long long strips = (g.Nx + kTileW - 1) / kTileW, unit = 4LL * std::max(cus, 1);
   constexpr struct { int tall, rows; double sets; } kHeights[] = {
       {16, 4, 12.0}, {12, 4, 1.6}, {9, 3, 1.6}, {6, 2, 1.6}};
   for (const auto& h : kHeights) {
     if (strips * ((g.Ny + h.tall - 1) / h.tall) < h.sets * unit) continue;
+    if (tall_chunks(g, (int)strips, h.tall, h.rows) < (strips < 2 * unit ? 1 : 4)) break;
     *rows = h.rows;
     return h.tall / h.rows;
   }
@@ -1361,9 +1375,9 @@ hipError_t launch_rhs_stage(const Geometry& g, const Phys& ph, int mode, const S
   BatchMember args = sweep_member(g, ph, sa.u, dU, gt, sa);
   args.lowTiles = args.nTiles;
   if (g.tall > 1) {
-    const int strips = args.nStrips, lowChunks = (kLowTiles + strips - 1) / strips;
+    const int strips = args.nStrips;
     args.tall = g.tall * g.rows;
-    const int tallChunks = std::max(0, (g.Ny - lowChunks * g.rows) / args.tall);
+    const int tallChunks = tall_chunks(g, strips, args.tall, g.rows);
     args.lowFrom = tallChunks * args.tall;
     args.tallTiles = tallChunks * strips;
     args.tallBlocks = (int)packed_tiles(args.tallTiles);
