@@ -232,8 +232,9 @@ int sgnx_batch_integrate(sgnx_batch* b, const double* t0, const double* tEnd, co
 
 /* sgnx_adjoint for every member, their reverse sweeps in lockstep with one
  * launch per kind over all members (aligned at each member's last step), or,
- * when every member alone fills the GPU, the members' own sweeps back to
- * back; each member's cotangents are bit for bit its own sgnx_adjoint's.
+ * for one member, and for two large ones that fill the GPU about as well
+ * alone, the members' own sweeps back to back; each member's cotangents are
+ * bit for bit its own sgnx_adjoint's.
  * Arrays of n pointers (Ubar_final, gauge_bar, theta_bar may be NULL, or hold
  * NULLs); every member's tape must hold every step's snapshot. */
 int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,

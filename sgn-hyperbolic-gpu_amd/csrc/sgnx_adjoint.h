@@ -50,6 +50,9 @@ struct GaugeMember {
 long long vjp_row_tiles(const Geometry& g);   // strips times element rows
 // element rows per workgroup for the grids of one launch (Geometry::vrows[third])
 int vjp_rows(const Geometry* const* g, int n, int cus, bool third);
+// about what a reversed step's three products of these grids take, packed, at the
+// heights rows[0] (the first two) and rows[1], in us
+double vjp_step_cost(const Geometry* const* g, int n, int cus, const int* rows);
 // nop: 1 = A only, 2 = A and B, 3 = with acc too, for all members
 hipError_t launch_rhs_vjp_batch(const VjpMember* mem, const long long* tileStart, int nMem,
                                 long long totalTiles, int nop, hipStream_t st);

@@ -706,10 +706,21 @@ int vjp_nop(const VjpArgs& va) { return va.acc ? 3 : va.B ? 2 : 1; }
 
 long long vjp_row_tiles(const Geometry& g) { return (long long)vjp_strips(g) * g.Ny; }
 
-// The lowest time by sweep_cost: per row a lone workgroup on a unit takes 2.8 us,
-// two, three and four together 3.6, 4.4 and 5.2 (a unit holds four), of the third
-// product 3.2, 4.1 and 5.0 (three); the rows staged beside a chunk cost as much
-// as its own.
+// Per row a lone workgroup on a unit takes 2.8 us, two, three and four together
+// 3.6, 4.4 and 5.2 (a unit holds four), of the third product 3.2, 4.1 and 5.0
+// (three); the rows staged beside a chunk cost as much as its own.
+namespace {
+constexpr SweepPace kPace[2] = {{4, 2.0, 0.8, 2.0, 2.0}, {3, 2.3, 0.9, 2.0, 2.0}};
+
+double vjp_cost(const Geometry* const* g, int n, int cus, bool third, int rows) {
+  long long tiles = 0;
+  for (int i = 0; i < n; ++i)
+    tiles += (long long)vjp_strips(*g[i]) * (((long long)g[i]->Ny + rows - 1) / rows);
+  return sweep_cost(tiles, rows, cus, kPace[third]);
+}
+}  // namespace
+
+// The lowest time by sweep_cost:
 //   first two products, us     rows: 2    3    4    7   10   16   32
 //    128 x   64                     44   46   46   65   73
 //    256 x  128                    126  115  112   99  107  130  199
@@ -719,13 +730,13 @@ long long vjp_row_tiles(const Geometry& g) { return (long long)vjp_strips(g) * g
 //    256 x  128                     81   71   70   68   62   74  111
 //   1024 x  512                   1269 1121 1038  948  906  854  829
 int vjp_rows(const Geometry* const* g, int n, int cus, bool third) {
-  constexpr SweepPace two{4, 2.0, 0.8, 2.0, 2.0}, last{3, 2.3, 0.9, 2.0, 2.0};
   cus = std::max(cus, 1);
-  return choose_rows(32, [&](int r) {
-    long long tiles = 0;
-    for (int i = 0; i < n; ++i) tiles += (long long)vjp_strips(*g[i]) * ((g[i]->Ny + r - 1) / r);
-    return sweep_cost(tiles, r, cus, third ? last : two);
-  });
+  return choose_rows(32, [&](int r) { return vjp_cost(g, n, cus, third, r); });
+}
+
+double vjp_step_cost(const Geometry* const* g, int n, int cus, const int* rows) {
+  cus = std::max(cus, 1);
+  return 2.0 * vjp_cost(g, n, cus, false, rows[0]) + vjp_cost(g, n, cus, true, rows[1]);
 }
 
 VjpMember vjp_member(const Geometry& g, const Phys& ph, const VjpArgs& va, GhostTime gt) {

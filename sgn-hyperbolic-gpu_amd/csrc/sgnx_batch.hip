@@ -595,11 +595,19 @@ int sgnx_batch_autotune(sgnx_batch* b, int reps, int* rows_out, int* waves3_out)
 // stage-2 launch that writes y2 and forms y3; the three products), each
 // member on its own buffers. The arithmetic is that of sgnx_adjoint on each
 // member alone, so the cotangents are bit for bit the same. Every member's
-// tape must hold every step's snapshot. When every member alone gives each
-// compute unit a full round of product workgroups (6 of 128 work-items), the
-// members' own sweeps run back to back instead: the products are bound by
-// their traffic, so the lockstep's launches gain nothing there, and its
-// per-step argument tables and member lookups made it slower (same bits).
+// tape must hold every step's snapshot. One member, and two large ones whose
+// products would hardly end sooner in one launch each, are swept by their own
+// calls back to back (same bits). A reversed step with kept stages and with
+// recomputed ones, us, back to back -> in lockstep:
+//   16 x 128x64   1143 ->  628  1604 ->  896     2 x 128x64   143 -> 120   199 -> 167
+//    8 x 128x64    572 ->  354   802 ->  503     2 x 220x110  254 -> 245   359 -> 354
+//    8 x 256x128  1301 -> 1140  1882 -> 1627     2 x 200x100  222 -> 218   314 -> 325
+//    3 x 450x225  1255 -> 1200  1906 -> 1750     2 x 300x150  407 -> 404   591 -> 616
+//    3 x 1024x512 6226 -> 5987  8991 -> 8810     2 x 450x225  857 -> 877  1304 -> 1283
+// By vjp_step_cost the pairs take 1.37, 1.15, 1.11, 1.07 and 1.00 times the
+// lockstep's time back to back; the line lies at 1.12. A pair with a small member
+// (less than six one-row tiles per compute unit) hides that one's launches in the
+// other's: 92x63 and 334x197 374 -> 355 and 541 -> 504. One of 64x32: 43 -> 60.
 int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
                        const double* const* gauge_bar, double* const* U0bar,
                        double* const* theta_bar, int mem) {
@@ -608,9 +616,19 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
     return bfail(b, SGNX_EINVAL, "batch adjoint: bad memory kind");
   const int n = b->n;
   BCHK(b, hipSetDevice(b->device));
-  bool each_fills = n > 0;
-  for (int i = 0; i < n; ++i) each_fills = each_fills && vjp_row_tiles(b->m[i]->g) >= 6LL * b->cus;
-  if (each_fills) {
+  // the products' tile heights for all members, unless set from outside
+  std::vector<const Geometry*> gs;
+  for (int i = 0; i < n; ++i) gs.push_back(&b->m[i]->g);
+  int vrows[2] = {0, 0};
+  if (!std::getenv("SGNX_SWEEP_ROWS"))
+    for (int k = 0; k < 2; ++k) vrows[k] = vjp_rows(gs.data(), n, b->cus, k == 1);
+  bool own = n == 1;
+  if (n == 2 && std::min(vjp_row_tiles(*gs[0]), vjp_row_tiles(*gs[1])) >= 6LL * b->cus) {
+    double alone = 0.0;
+    for (const Geometry*& g : gs) alone += vjp_step_cost(&g, 1, b->cus, g->vrows);
+    own = alone < 1.12 * vjp_step_cost(gs.data(), n, b->cus, vrows[0] ? vrows : gs[0]->vrows);
+  }
+  if (own) {
     for (int i = 0; i < n; ++i) {
       sgnx_solver* s = b->m[i];
       if (!U0bar[i]) return bfail(b, SGNX_EINVAL, "batch adjoint: U0bar missing for a member");
@@ -624,12 +642,8 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
     }
     return SGNX_OK;
   }
-  // the products' tile heights for all members, unless set from outside
-  std::vector<const Geometry*> gs;
-  for (int i = 0; i < n; ++i) gs.push_back(&b->m[i]->g);
-  int vrows[2] = {0, 0};
-  if (!std::getenv("SGNX_SWEEP_ROWS"))
-    for (int k = 0; k < 2; ++k) vrows[k] = vjp_rows(gs.data(), n, b->cus, k == 1);
+  // (work on the null stream that a member's own stream would wait for)
+  if (mem == SGNX_MEM_DEVICE) BCHK(b, hipStreamSynchronize(nullptr));
   std::vector<AdjTape*> tp(n, nullptr);
   std::vector<const double*> gb(n, nullptr);
   long Nmax = 0;
@@ -642,6 +656,7 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
       rc = adjoint_inputs(s, tp[i], Ubar_final ? Ubar_final[i] : nullptr,
                           gauge_bar ? gauge_bar[i] : nullptr, mem, b->stream, &gb[i]);
     if (rc) return bfail(b, rc, "batch adjoint, member " + std::to_string(i) + ": " + s->err);
+    tp[i]->recomputed = tp[i]->peakSlots = 0;
     Nmax = std::max(Nmax, (long)tp[i]->t.size());
   }
   // argument arena: gauges, two RHS tables (R(u); the stage-2 launch keeping
