@@ -250,8 +250,10 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
  * written; U and k1 are untouched. The tile height fixes the summation order
  * of the error norm, so a run is reproducible bit for bit under the same
  * setting (a batch member and its solo run share it). rows_out / waves3_out
- * (optional) receive the choice. The batch form picks one tile height for
- * every member and the batch's waves. */
+ * (optional) receive the choice. The batch form picks one tile height for the
+ * batch's launches, its untuned heights among the candidates, and the waves: a
+ * member with its default height keeps it alone and takes the nearest multiple
+ * in the batch, one whose height was set takes the one picked. */
 int sgnx_autotune(sgnx_solver* s, int reps, int* rows_out, int* waves3_out);
 int sgnx_batch_autotune(sgnx_batch* b, int reps, int* rows_out, int* waves3_out);
 

@@ -39,6 +39,8 @@ struct sgnx_batch {
   int n = 0;
   int device = 0, cus = 1;
   int waves3 = 0x2;                    // bit k: launch kind k built for 3 waves/SIMD
+  int rows = 0;                        // the packed launches' height from the autotuner
+                                       // (0: by the rule for the running members)
   hipStream_t stream = nullptr;
   // argument tables, [4 launch kinds][n slots], then the tile offsets, then the
   // attempt's sequence number, in one block (one copy takes a step's part)
@@ -106,17 +108,20 @@ BatchMember member_args(const sgnx_solver* s, const double* U, double* dU, const
 // 34x17 to 126x63, heights 1 and 2, or 4 for all: stages 2, 3 and 4 103, 142 and
 // 106 us, or 96, 128 and 109; ten accepted steps 5.25 ms, or 5.03).
 // So the members in `set` take the multiple of their own that is nearest to the
-// height for all their tiles together; a height set from outside or by an
-// autotuner is taken as it is.
-std::vector<int> row_multiples(const sgnx_batch* b, const std::vector<int>& set) {
+// height for all their tiles together, by the rule or by the batch's autotuner;
+// a height set from outside or by an autotuner is taken as it is.
+int packed_rows(const sgnx_batch* b, const std::vector<int>& set) {
   std::vector<const Geometry*> gs;
   for (int i : set) gs.push_back(&b->m[i]->g);
-  const int rows = sweep_rows(gs.data(), (int)gs.size(), b->cus);
+  return sweep_rows(gs.data(), (int)gs.size(), b->cus);
+}
+int row_multiple(const sgnx_solver* s, int rows) {
+  return s->rowsSet ? 1 : std::max(1, (2 * rows + s->g.rows) / (2 * s->g.rows));
+}
+std::vector<int> row_multiples(const sgnx_batch* b, const std::vector<int>& set) {
+  const int rows = b->rows ? b->rows : packed_rows(b, set);
   std::vector<int> times;
-  for (int i : set) {
-    const sgnx_solver* s = b->m[i];
-    times.push_back(s->rowsSet ? 1 : std::max(1, (2 * rows + s->g.rows) / (2 * s->g.rows)));
-  }
+  for (int i : set) times.push_back(row_multiple(b->m[i], rows));
   return times;
 }
 
@@ -513,17 +518,25 @@ int sgnx_batch_autotune(sgnx_batch* b, int reps, int* rows_out, int* waves3_out)
   int maxNy = 1;
   for (sgnx_solver* s : b->m) maxNy = std::max(maxNy, s->g.Ny);
   const size_t nn = (size_t)n;
-  // fill the tables of every kind for the members' current tile height
-  auto fill = [&]() -> long long {
+  // Fill the tables of every kind for a candidate height (0: the rule's). A member
+  // with its default height takes the nearest multiple of it, as it will in the
+  // batch; one whose height was set, the candidate.
+  auto fill = [&](int rows) -> long long {
+    const int packed = rows ? rows : packed_rows(b, all);
     for (int i = 0; i < n; ++i) {
       sgnx_solver* s = b->m[i];
+      Geometry g = s->g;
+      if (s->rowsSet && rows) g.rows = rows;
+      const int times = row_multiple(s, packed);
+      const GhostTime gt = ghost_time(s, 0.0);
       BS3Launch L[3];
       bs3_launches(s, 0.0, kProbeDt, 1.0, 0.0, L);
       Stage sa{};
       sa.u = s->d_U;
-      b->h_mem[i] = member_args(s, s->d_U, s->d_k2, sa, 0.0);
+      b->h_mem[i] = sweep_member(g, s->ph, s->d_U, s->d_k2, gt, sa, times);
       for (int k = 0; k < 3; ++k)
-        b->h_mem[(size_t)(k + 1) * nn + i] = member_args(s, L[k].sa.u, L[k].dU, L[k].sa, L[k].t);
+        b->h_mem[(size_t)(k + 1) * nn + i] =
+            sweep_member(g, s->ph, L[k].sa.u, L[k].dU, ghost_time(s, L[k].t), L[k].sa, times);
     }
     return fill_offsets(b, all, b->h_mem);
   };
@@ -540,14 +553,17 @@ int sgnx_batch_autotune(sgnx_batch* b, int reps, int* rows_out, int* waves3_out)
     if ((e = hipEventSynchronize(ev.b)) != hipSuccess) return e;
     return hipEventElapsedTime(ms, ev.a, ev.b);
   };
-  std::vector<int> keepRows(n);
-  for (int i = 0; i < n; ++i) keepRows[i] = b->m[i]->g.rows;
+  // the rule's heights are a candidate where a member has its default one
+  bool rule = false;
+  for (const sgnx_solver* s : b->m) rule = rule || !s->rowsSet;
+  std::vector<int> heights;
+  if (rule) heights.push_back(0);
+  for (int rows : kTuneRows)
+    if (rows <= maxNy || rows == kTuneRows[0]) heights.push_back(rows);
   double best = 1e300;
-  int bestRows = keepRows[0], bestMask = b->waves3;
-  for (int rows : kTuneRows) {
-    if (rows > maxNy && rows != kTuneRows[0]) continue;
-    for (sgnx_solver* s : b->m) s->g.rows = rows;
-    const long long total = fill();
+  int bestRows = heights[0], bestMask = b->waves3;
+  for (int rows : heights) {
+    const long long total = fill(rows);
     BCHK(b, hipMemcpyAsync(b->d_mem, b->h_mem, 4 * nn * sizeof(BatchMember),
                            hipMemcpyHostToDevice, b->stream));
     BCHK(b, hipMemcpyAsync(b->d_ts, b->h_ts, (nn + 1) * sizeof(long long),
@@ -568,11 +584,7 @@ int sgnx_batch_autotune(sgnx_batch* b, int reps, int* rows_out, int* waves3_out)
       bestMask = mask;
     }
   }
-  for (sgnx_solver* s : b->m) {
-    take_rows(s, bestRows);
-    s->rowsSet = true;
-  }
-  const long long total = fill();
+  const long long total = fill(bestRows);
   BCHK(b, hipMemcpyAsync(b->d_mem, b->h_mem, 4 * nn * sizeof(BatchMember),
                          hipMemcpyHostToDevice, b->stream));
   BCHK(b, hipMemcpyAsync(b->d_ts, b->h_ts, (nn + 1) * sizeof(long long), hipMemcpyHostToDevice,
@@ -581,9 +593,15 @@ int sgnx_batch_autotune(sgnx_batch* b, int reps, int* rows_out, int* waves3_out)
   BCHK(b, timed(0, false, total, &p2));
   BCHK(b, timed(0, true, total, &p3));
   BCHK(b, hipStreamSynchronize(b->stream));
+  b->rows = bestRows;
   b->waves3 = bestMask | (p3 < p2 ? 1 : 0);
-  for (sgnx_solver* s : b->m) s->g.waves3 = b->waves3;
-  if (rows_out) *rows_out = bestRows;
+  for (sgnx_solver* s : b->m) {
+    // (a default height stays: alone, a member is faster with it, and its norm's
+    // partial sums follow it in the batch too)
+    if (s->rowsSet && bestRows) take_rows(s, bestRows);
+    s->g.waves3 = b->waves3;
+  }
+  if (rows_out) *rows_out = bestRows ? bestRows : packed_rows(b, all);
   if (waves3_out) *waves3_out = b->waves3;
   return SGNX_OK;
 }

@@ -53,8 +53,9 @@ class Batch:
         self._check(self.lib.sgnx_batch_set_waves(self.h, int(mask)))
 
     def autotune(self, reps=3):
-        """One tile height for every member and the batch's waves per SIMD, by
-        timing the batched launches; returns (rows, waves mask)."""
+        """The tile height of the batched launches and their waves per SIMD, by
+        timing them; returns (rows, waves mask). Members with their default
+        height keep it alone; members whose height was set take this one."""
         r, w = C.c_int(), C.c_int()
         self._check(self.lib.sgnx_batch_autotune(self.h, int(reps), C.byref(r), C.byref(w)))
         return r.value, w.value
@@ -92,9 +93,10 @@ class Batch:
         """Every member's SGN2D.adjoint (its tape recorded with a snapshot of
         every step), the reverse sweeps in lockstep with one launch per kind
         (or, for one member, and for two large ones that fill the GPU about as
-        well alone, their own sweeps back to back); each member's result is bit for bit its own adjoint's. Ubar_final,
-        gauge_bar: None or one array (or None) per member. Returns a list of
-        (U0bar, thetaBar) (or U0bar when theta is False)."""
+        well alone, their own sweeps back to back); each member's result is bit
+        for bit its own adjoint's. Ubar_final, gauge_bar: None or one array (or
+        None) per member. Returns a list of (U0bar, thetaBar) (or U0bar when
+        theta is False)."""
         n = len(self.members)
         keep = []
 
