@@ -146,9 +146,11 @@ int sgnx_bathymetry(const sgnx_solver* s, double* Hx, double* Hy);
  * element columns and `rows` element rows per workgroup (default 1, rows 1 to
  * 24 by the grid's size and the number of compute units; with the default
  * height the first workgroups of a larger grid take three or four times as
- * many, and in a batch small members multiples of theirs; the environment
- * variables SGNX_RHS_VARIANT / SGNX_SWEEP_ROWS set the defaults at creation,
- * the latter for the adjoint's products too). Both are bitwise equal to the reference rhs(). The
+ * many, and in a batch small members multiples of theirs: setting that height,
+ * which sgnx_get_rhs_kernel gives after creation, brings both back; the
+ * environment variables SGNX_RHS_VARIANT / SGNX_SWEEP_ROWS set the defaults at
+ * creation, the latter for the adjoint's products too). Both are bitwise equal
+ * to the reference rhs(). The
  * row sweep has no Manning friction term: a solver with nManning != 0 uses
  * variant 0 (variant 1 then gives SGNX_EUNSUPPORTED, and such a solver
  * cannot join a batch or be autotuned). */

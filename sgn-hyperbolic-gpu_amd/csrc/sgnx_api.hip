@@ -667,7 +667,6 @@ int sgnx_set_rhs_kernel(sgnx_solver* s, int variant, int rows) {
     return fail(s, SGNX_EUNSUPPORTED, "the row sweep has no Manning friction term (variant 0 has)");
   s->g.variant = variant;
   take_rows(s, rows);
-  s->rowsSet = true;
   return SGNX_OK;
 }
 

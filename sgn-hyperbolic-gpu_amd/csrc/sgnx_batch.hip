@@ -444,6 +444,13 @@ int sgnx_autotune(sgnx_solver* s, int reps, int* rows_out, int* waves3_out) {
   if (hipEventCreate(&ev.a) != hipSuccess || hipEventCreate(&ev.b) != hipSuccess)
     return SGNX_EDEVICE;
   const Geometry keep = s->g;
+  const bool keepSet = s->rowsSet;
+  auto failed = [&] {
+    s->g = keep;
+    s->rowsSet = keepSet;
+    s->err = "autotune: probe launch failed";
+    return SGNX_EDEVICE;
+  };
   s->g.variant = 1;
   BS3Launch L[3];
   // ms of `reps` launches of kind k (0: R(U) into k2's buffer; 1..3: a BS3
@@ -476,11 +483,7 @@ int sgnx_autotune(sgnx_solver* s, int reps, int* rows_out, int* waves3_out) {
     int mask = 0;
     for (int k = 1; k <= 3; ++k) {
       float t2 = 0.0f, t3 = 0.0f;
-      if (timed(k, false, &t2) != hipSuccess || timed(k, true, &t3) != hipSuccess) {
-        s->g = keep;
-        s->err = "autotune: probe launch failed";
-        return SGNX_EDEVICE;
-      }
+      if (timed(k, false, &t2) != hipSuccess || timed(k, true, &t3) != hipSuccess) return failed();
       tot += std::min(t2, t3);
       if (t3 < t2) mask |= 1 << k;
     }
@@ -491,13 +494,8 @@ int sgnx_autotune(sgnx_solver* s, int reps, int* rows_out, int* waves3_out) {
     }
   }
   take_rows(s, bestRows);
-  s->rowsSet = true;
   float p2 = 0.0f, p3 = 0.0f;
-  if (timed(0, false, &p2) != hipSuccess || timed(0, true, &p3) != hipSuccess) {
-    s->g = keep;
-    s->err = "autotune: probe launch failed";
-    return SGNX_EDEVICE;
-  }
+  if (timed(0, false, &p2) != hipSuccess || timed(0, true, &p3) != hipSuccess) return failed();
   s->g.waves3 = bestMask | (p3 < p2 ? 1 : 0);
   if (rows_out) *rows_out = s->g.rows;
   if (waves3_out) *waves3_out = s->g.waves3;

@@ -101,11 +101,13 @@ inline GhostTime ghost_time(const sgnx_solver* s, double t) {
   return gt;
 }
 
-// A height for all tiles; the one that the rule gives the grid brings its tall
-// tiles too (the results are the same bits).
+// A height for all tiles; the one that the rule gives the grid is the default
+// again, with its tall tiles and, in a batch, its multiples (the results are the
+// same bits).
 inline void take_rows(sgnx_solver* s, int rows) {
   s->g.rows = rows;
-  s->g.tall = rows == s->ownRows ? s->ownTall : 1;
+  s->rowsSet = rows != s->ownRows;
+  s->g.tall = s->rowsSet ? 1 : s->ownTall;
 }
 
 // The three row-sweep launches of one BS3 attempt (rk.cpp:99-131) on a

@@ -75,3 +75,26 @@ def test_a_height_set_after_tuning_is_taken():
         s.close()
     for x in d + [u]:
         x.free()
+
+
+def test_the_default_height_can_be_set_again():
+    """A member that went to the element-row tiles, or to another height, and back
+    to its default height is a default member again: the batch autotuner, which
+    gives members with a height of their own the one it picks, leaves it."""
+    import sgnx
+    from sgnx import cases
+    cs = [cases.gate(Nx=8, Ny=6), cases.gate(Nx=24, Ny=17), cases.gate(Nx=200, Ny=101)]
+    ss = [sgnx.SGN2D(**c.solver_kwargs()) for c in cs]
+    default = [s.rhs_kernel()[1] for s in ss]
+    assert 1 in default                       # (no height that a tuner tries)
+    for s, c, r in zip(ss, cs, default):
+        s.upload(c.U0)
+        s.set_rhs_kernel(0, r)
+        s.set_rhs_kernel(1, 16)
+        s.set_rhs_kernel(1, r)
+    b = sgnx.Batch(ss)
+    b.autotune(1)
+    assert [s.rhs_kernel()[1] for s in ss] == default
+    b.close()
+    for s in ss:
+        s.close()
