@@ -178,9 +178,9 @@ def batched_sweep(args, nx_min=128, nx_max=768, n_members=None, steps=None, sing
     --batch-steps accepted adaptive steps, first one at a time with the plain
     solver, then all together in one Batch (one launch per stage kind, a
     captured step graph); every member must end bit for bit where its solo run
-    did. The tile height is chosen once by the batch autotuner and used by
-    both runs. Before that, the members also run one at a time with their
-    own default tile heights: the plain solver's rate without the batch,
+    did. The batch autotuner chooses the packed tile height and the waves;
+    members keep their default heights alone. Before that, the members also
+    run one at a time as created: the plain solver's rate without the batch,
     against which `speedup` is taken (each member's best solo setting).
     `speedup_bound` is what batching could gain at most if every member ran
     at `single_rate` (the rate of one production-size grid): the members'
@@ -205,9 +205,8 @@ def batched_sweep(args, nx_min=128, nx_max=768, n_members=None, steps=None, sing
         f"{nodes / 1e6:.1f} M nodes, built in {time.perf_counter() - t:.1f}s")
     opts = sgnx.RkOpts(atol=1e-8, rtol=1e-6, max_accepted=steps)
     one = sgnx.RkOpts(atol=1e-8, rtol=1e-6, max_accepted=1)
-    # the members one at a time with their own default tile heights (the
-    # tallest that fills the chip, per grid): the sequential rate a user of
-    # the plain solver gets
+    # the members one at a time as created (default tile heights and waves):
+    # the sequential rate a user of the plain solver gets
     members[0].integrateAdaptive(0.0, 1e9, dt0s[0], one)
     own_wall, own_dof = 0.0, 0.0
     for s, U0, dt0 in zip(members, U0s, dt0s):
@@ -475,9 +474,9 @@ def batched_adjoint_leg(args):
     (plain run, taped run, reverse sweep) and as one batch (a batched taped
     run, one launch per kind over all members, then the batched reverse
     sweep); the tapes keep the stage inputs; the cotangents must agree bit
-    for bit. The batch autotuner picks one tile height, used by both. Each member's gradient is
-    checked in one smooth direction near its gauges against fourth-order
-    differences of its plain solver's replay."""
+    for bit. The batch autotuner picks the packed tile height and the waves.
+    Each member's gradient is checked in one smooth direction near its gauges
+    against fourth-order differences of its plain solver's replay."""
     import numpy as np
     import sgnx
     from sgnx import cases
@@ -499,8 +498,8 @@ def batched_adjoint_leg(args):
         members.append(s)
         data.append((c, theta, nodes, dt0))
     opts = sgnx.RkOpts(atol=1e-10, rtol=1e-8, max_accepted=steps)
-    # one tile height for every member, chosen by the batch autotuner and used
-    # by both the one-by-one and the batched runs (as in the batched sweep)
+    # the packed tile height and the waves from the batch autotuner (as in the
+    # batched sweep)
     b = sgnx.Batch(members)
     rows, waves = b.autotune()
 

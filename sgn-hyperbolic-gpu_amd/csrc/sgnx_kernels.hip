@@ -1340,7 +1340,19 @@ void sweep_launch_batch(bool hxr, dim3 grid, dim3 block, hipStream_t st, const B
 //  1024 x 512  12, 4 against 8         341.9 -> 330.0 440.0 -> 426.2  635.6 -> 628.6 498.7 -> 493.7
 //  2000 x 1000 16, 4 against 18         1239 -> 1221   1607 -> 1588    2396 -> 2376   1887 -> 1858
 // (1024 x 512 at 16, 4: 333, 427, 630, 502; 2000 x 1000 at 12, 4: 1234, 1620, 2391,
-// 1871.) A grid that has not 1.6 sets of four workgroups per compute unit at 6
+// 1871.) 16, 4 against 12, 4, by the sets of four workgroups per compute unit that
+// 16 rows make (the place of the arrays moves stage 3 by more than that):
+//   6.4  1024 x 512   plain 377, 369   443, 451   k4 504, 514
+//   8.8  1200 x 600         503, 513   600, 600      696, 689
+//  10.4  1300 x 650         588, 589   699, 709      810, 814
+//  13.0  1448 x 724         731, 737   868, 880     1004, 1002
+//  15.6  1600 x 800         886, 894  1051, 1059    1206, 1210
+// 6, 2 against one height, plain and the step's three together, at 1.6 to 2.4 sets
+// of 6 rows: 303 x 161 50.6 185 -> 43.9 172, 256 x 210 50.5 198 -> 47.5 189, 370 x 185
+// 60.7 247 -> 57.0 236, but 320 x 160 46.6 170 -> 44.3 176, 330 x 165 52.0 191 -> 51.7
+// 203, where the one height makes just one set, which stage 3 takes in one go; in the
+// mean of 16 sizes 1 % faster, the plain launch 5 %.
+// A grid that has not 1.6 sets of four workgroups per compute unit at 6
 // rows takes one height (sweep_rows), and so does a flat one: the rows that a
 // strip has left beside its tall tiles all go into low ones, which costs more than
 // their even end gives where there is no tall tile, or, with two sets of strips or
@@ -1350,8 +1362,8 @@ void sweep_launch_batch(bool hxr, dim3 grid, dim3 block, hipStream_t st, const B
 //   20000 x 11   164  673,  6, 2: 188  774      61440 x 11   488 1987,  6, 2: 548 2424
 constexpr int kLowTiles = 1280;
 
-// chunks of `tall` rows above which the rest of the rows makes the low tiles
-int tall_chunks(const Geometry& g, int strips, int tall, int rows) {
+// chunks of `tall` rows, which leave the rest of the rows to the low tiles
+static int tall_chunks(const Geometry& g, int strips, int tall, int rows) {
   const int lowChunks = (kLowTiles + strips - 1) / strips;
   return std::max(0, (g.Ny - lowChunks * rows) / tall);
 }
@@ -1414,9 +1426,12 @@ BatchMember sweep_member(const Geometry& g, const Phys& ph, const double* U, dou
   return m;
 }
 
-// The lowest time of a step by sweep_cost, in us: six workgroups of the plain
-// launch and of stage 2 fit on a compute unit, four of stage 3 and of the last
-// stage. Measured (plain, stage 2, stage 3, last):
+// The lowest time of a step by sweep_cost, in us: six workgroups fit on a compute
+// unit, four of stage 3 (kStripW). The last stage fits six times too, yet the rule
+// counts it with stage 3: counted with the others it picks 1 row for 103 x 77 (62.6
+// us a step, 57.6 at the 2 rows taken), 3 for 156 x 117 (94.1, 90.5 at 4), 4 for 197 x
+// 147 (127.6, 120.0 at 6), 3 for 333 x 133 (175.3, 165.5 at 9). Measured (plain, stage
+// 2, stage 3, last):
 //   rows            1            2            5            7            8           12           16
 //   128 x  64  16 20 22 20  15 18 19 19  24 28 28 30  31 34 36 37  29 31 33 34  40 43 46 47  51 54 58 60
 //   256 x 128  38 47 58 49  34 41 50 43  33 40 55 42  35 40 43 43  38 43 46 47  50 55 58 61  63 68 72 76
