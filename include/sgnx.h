@@ -149,8 +149,8 @@ int sgnx_bathymetry(const sgnx_solver* s, double* Hx, double* Hy);
  * many, and in a batch small members multiples of theirs: setting that height,
  * which sgnx_get_rhs_kernel gives after creation, brings both back; the
  * environment variables SGNX_RHS_VARIANT / SGNX_SWEEP_ROWS set the defaults at
- * creation, the latter for the adjoint's products too). Both are bitwise equal
- * to the reference rhs(). The
+ * creation, SGNX_VJP_ROWS the height of the adjoint's products, which changes no
+ * bit of them). Both are bitwise equal to the reference rhs(). The
  * row sweep has no Manning friction term: a solver with nManning != 0 uses
  * variant 0 (variant 1 then gives SGNX_EUNSUPPORTED, and such a solver
  * cannot join a batch or be autotuned). */

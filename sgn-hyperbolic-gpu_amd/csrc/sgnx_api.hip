@@ -217,20 +217,24 @@ int sgnx_create(const sgnx_desc* d, sgnx_solver** out) {
 
   CK(hipGetDevice(&s->device));
   CK(scratch_address(s->device, &s->scratch));
-  g.vrows[0] = g.vrows[1] = g.rows;
+  // The RHS and the products do not depend on the heights; the adaptive step's
+  // error norm is summed per g.rows rows, so its last bits can. A height given for
+  // the sweep is none for the products: 16 rows, which suit the sweep of a large
+  // grid, made the reverse sweep of 64x32 three times as long.
   s->rowsSet = std::getenv("SGNX_SWEEP_ROWS") != nullptr;
+  const char* const vjpRows = std::getenv("SGNX_VJP_ROWS");
+  s->vrowsSet = vjpRows != nullptr;
+  int cus = 0;
+  CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device));
+  const Geometry* const one = &g;
   if (!s->rowsSet) {
-    // The RHS and the products do not depend on the heights; the adaptive
-    // step's error norm is summed per g.rows rows, so its last bits can.
-    int cus = 0;
-    CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device));
-    const Geometry* const one = &g;
     g.rows = sweep_rows(&one, 1, cus);
     g.tall = sweep_tall(g, cus, &g.rows);
     s->ownRows = g.rows;
     s->ownTall = g.tall;
-    for (int k = 0; k < 2; ++k) g.vrows[k] = vjp_rows(&one, 1, cus, k == 1);
   }
+  for (int k = 0; k < 2; ++k)
+    g.vrows[k] = vjpRows ? std::max(1, std::atoi(vjpRows)) : vjp_rows(&one, 1, cus, k == 1);
   const size_t Nd = (size_t)g.Nd, nst = (size_t)NV * Nd;
   const size_t nfx = (size_t)(d->Nx + 1) * d->Ny * NP, nfy = (size_t)d->Nx * (d->Ny + 1) * NP;
   OpTables T;

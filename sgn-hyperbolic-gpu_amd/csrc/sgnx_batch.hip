@@ -636,9 +636,13 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
   BCHK(b, hipSetDevice(b->device));
   // the products' tile heights for all members, unless set from outside
   std::vector<const Geometry*> gs;
-  for (int i = 0; i < n; ++i) gs.push_back(&b->m[i]->g);
+  bool given = false;
+  for (const sgnx_solver* s : b->m) {
+    gs.push_back(&s->g);
+    given = given || s->vrowsSet;
+  }
   int vrows[2] = {0, 0};
-  if (!std::getenv("SGNX_SWEEP_ROWS"))
+  if (!given)
     for (int k = 0; k < 2; ++k) vrows[k] = vjp_rows(gs.data(), n, b->cus, k == 1);
   bool own = n == 1;
   if (n == 2 && std::min(vjp_row_tiles(*gs[0]), vjp_row_tiles(*gs[1])) >= 6LL * b->cus) {

@@ -22,6 +22,7 @@ struct sgnx_solver {
   double Lx = 0.0, Ly = 0.0, hx = 0.0, hy = 0.0;
   Geometry g{};
   bool rowsSet = false;      // g.rows set from outside or by an autotuner, not by the rule
+  bool vrowsSet = false;     // g.vrows set from outside
   int ownRows = 0, ownTall = 1;   // what the rule gives this grid
   Phys ph{};
   hipStream_t stream = nullptr;

@@ -50,7 +50,7 @@ def test_products_at_the_largest_height(monkeypatch):
     W = np.random.default_rng(2).normal(size=c.U0.size)
     got = []
     for rows in (6, 2 ** 31 - 1):
-        monkeypatch.setenv("SGNX_SWEEP_ROWS", str(rows))
+        monkeypatch.setenv("SGNX_VJP_ROWS", str(rows))
         s = sgnx.SGN2D(**c.solver_kwargs())
         s.setDepth(c.depth["Hnod"])
         got.append(s.rhs_vjp(c.U0, W, 0.3))
