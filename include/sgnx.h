@@ -245,8 +245,9 @@ int sgnx_batch_adjoint(sgnx_batch* b, const double* const* Ubar_final,
 
 /* Autotuning (no counterpart in the reference): times every launch kind of an
  * adaptive step on the resident state for each candidate tile height (element
- * rows per workgroup: 2, 4, 8, 12, 16, 24, 32, up to Ny, and a larger grid's
- * default with its taller first workgroups) and each build
+ * rows per workgroup: 2, 4, 8, 12, 16, 24, 32, up to Ny, and the solver's
+ * default unless another height was set; a larger grid's default, with its
+ * taller first workgroups, in any case) and each build
  * (two or three waves per SIMD), keeps the fastest, and sets it (row-sweep
  * kernel; reps = launches timed per candidate). Only scratch stage buffers are
  * written; U and k1 are untouched. The tile height fixes the summation order

@@ -474,8 +474,10 @@ int sgnx_autotune(sgnx_solver* s, int reps, int* rows_out, int* waves3_out) {
   double best = 1e300;
   int bestRows = keep.rows, bestMask = keep.waves3;
   std::vector<int> heights(std::begin(kTuneRows), std::end(kTuneRows));
-  // (a default of 2 or 4 rows with tall tiles is among them already)
-  if (s->ownTall > 1 && std::find(heights.begin(), heights.end(), s->ownRows) == heights.end())
+  // the default height too, unless it is among them or another one was set (that of
+  // a larger grid, with its tall tiles, in any case)
+  if ((s->ownTall > 1 || !s->rowsSet) &&
+      std::find(heights.begin(), heights.end(), s->ownRows) == heights.end())
     heights.push_back(s->ownRows);
   for (int rows : heights) {
     if (rows > s->g.Ny && rows != kTuneRows[0]) continue;

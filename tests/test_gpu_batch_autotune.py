@@ -98,3 +98,16 @@ def test_the_default_height_can_be_set_again():
     b.close()
     for s in ss:
         s.close()
+
+
+def test_the_default_height_is_a_candidate():
+    """A grid of a few workgroups is fastest at one row, its default, which is none
+    of the heights that the tuner tries anyway: tuning keeps it."""
+    import sgnx
+    from sgnx import cases
+    c = cases.gate(Nx=8, Ny=6)
+    s = sgnx.SGN2D(**c.solver_kwargs())
+    s.upload(c.U0)
+    assert s.rhs_kernel()[1] == 1
+    assert s.autotune(20)[0] == 1
+    s.close()
